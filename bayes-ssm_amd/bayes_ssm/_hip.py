@@ -50,6 +50,8 @@ _SIGNATURES = {
     "bssm_backward_chunked_bf16": [_I, _I, _I] + [_P] * 10 + [_P] * 3 + [_P] * 8 + [_L, _L, _L, _F, _P],
     "bssm_forward_chunked_fp8": [_I, _I, _I, _I] + [_P] * 8 + [_P] * 5 + [_L, _L, _L, _F, _P],
     "bssm_backward_chunked_fp8": [_I, _I, _I, _I] + [_P] * 10 + [_P] * 3 + [_P] * 8 + [_L, _L, _L, _F, _P],
+    "bssm_forward_chunked_narrow": [_I, _I, _I, _I] + [_P] * 8 + [_P] * 5 + [_L, _L, _L, _F, _P],
+    "bssm_backward_chunked_narrow": [_I, _I, _I, _I] + [_P] * 10 + [_P] * 3 + [_P] * 8 + [_L, _L, _L, _F, _P],
     "bssm_round_float8": [_I, _P, _P, _L],
     "bssm_value_stats_workspace": [_I, _P],
     "bssm_value_stats": [_I, _P, _P, _P, _P, _L, _P, _P],
@@ -73,7 +75,7 @@ _SIGNATURES = {
     "bssm_preferred_checkpoint": [_I],
     "bssm_abi_version": [],
 }
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 _lock = threading.Lock()
 _lib: Optional[ctypes.CDLL] = None

@@ -405,10 +405,13 @@ class _ChunkedBayesianFunction(torch.autograd.Function):
 
 # float8 encodings the D4M8 kernels read (C ABI format argument).
 _FP8_FORMATS = {torch.float8_e4m3fn: 0, torch.float8_e5m2: 1}
+_NARROW_FORMATS = {**_FP8_FORMATS, torch.bfloat16: 2}
 
 
 def _narrow_call(keys: Tensor, direction: str) -> tuple[str, tuple[int, ...]]:
     """C ABI entry point and leading format argument for narrow keys/values/queries."""
+    if keys.shape[1] % 4:  # rows that do not start on a 16-byte boundary
+        return f"bssm_{direction}_chunked_narrow", (_NARROW_FORMATS[keys.dtype],)
     if keys.dtype == torch.bfloat16:
         return f"bssm_{direction}_chunked_bf16", ()
     return f"bssm_{direction}_chunked_fp8", (_FP8_FORMATS[keys.dtype],)
@@ -482,11 +485,15 @@ class _ChunkedBayesianBF16Function(torch.autograd.Function):
                 gd if need[3] else None, gp if need[4] else None, gr if need[5] else None, gm0, gc0, None, None)
 
 
-def _bf16_kernels_apply(keys: Tensor, values: Tensor, queries: Tensor) -> bool:
-    """The D4M8 kernels read these bfloat16 / float8 streams directly (else: widen, float32 path)."""
+def _bf16_kernels_apply(keys: Tensor, values: Tensor, queries: Tensor, fixed: bool) -> bool:
+    """The D4M8 kernels read these bfloat16 / float8 streams directly (else: widen, float32 path).
+
+    With fixed dynamics and T not a multiple of 4 the backward kernels take
+    no final-state gradients; whether there will be any is not known here.
+    """
     n, t, d = keys.shape
-    return ((d, values.shape[-1]) == (4, 8) and t > 0 and t % 4 == 0 and _hip.preferred_checkpoint(d) > 0
-            and all(x.data_ptr() % 16 == 0 for x in (keys, values, queries)))
+    return ((d, values.shape[-1]) == (4, 8) and t > 0 and (t % 4 == 0 or not fixed)
+            and _hip.preferred_checkpoint(d) > 0 and all(x.data_ptr() % 16 == 0 for x in (keys, values, queries)))
 
 
 def fused_diagonal_bayesian(
@@ -549,7 +556,7 @@ def fused_diagonal_bayesian(
         x if x.is_contiguous() else x.contiguous()
         for x in (keys, values, queries, decay, process, observation, initial_mean, initial_covariance))
     if bf16:
-        if _bf16_kernels_apply(keys, values, queries):
+        if _bf16_kernels_apply(keys, values, queries, bool(fixed_dynamics)):
             return _ChunkedBayesianBF16Function.apply(
                 keys, values, queries, decay, process, observation, initial_mean, initial_covariance,
                 float(denominator_floor), bool(fixed_dynamics))

@@ -38,15 +38,29 @@ bool supported(int d, int m) { return (m == 8 && (d == 1 || d == 2 || d == 4 || 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 bool aligned8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; }
 
-// The D = 4 rotated-layout kernels address each 16-sequence block through
-// 32-bit buffer offsets, move every stream in 16-byte chunks and store the
-// belief in 8-byte pieces.
-bool rot4_ok(int d, int m, int64_t t, int64_t nb, bool streams16, std::initializer_list<const void*> belief) {
-  if (d != 4 || m != 8 || t <= 0 || t % 4 != 0 || !streams16) return false;
+// The D = 4 kernels address each 16-sequence block through 32-bit buffer
+// offsets, move every stream in 16-byte pieces and store the belief in 8-byte
+// pieces.  They take every T: a row that does not start on a 16-byte boundary
+// (T not a multiple of 4) is moved by the same 16-byte accesses, which the
+// buffer instructions allow at any 4-byte aligned address.
+bool rot4_ok(int d, int m, int64_t t, int64_t nb, std::initializer_list<const void*> streams,
+             std::initializer_list<const void*> belief) {
+  if (d != 4 || m != 8 || t <= 0) return false;
+  for (const void* p : streams)
+    if (p != nullptr && !aligned16(p)) return false;
   if ((nb + 1) * 128 * 16 >= ((int64_t)1 << 31)) return false;
   for (const void* p : belief)
     if (p != nullptr && !aligned8(p)) return false;
   return true;
+}
+
+// A T that is not a multiple of 4 ends inside a chunk: the backward fills it
+// up with tokens that leave belief and adjoints as they are, which fixed
+// dynamics (constant decay and process noise) allow only while the adjoints
+// are zero, i.e. without final-state gradients.  The 16-token interval keeps
+// to multiples of 4.
+bool rot4_tail_ok(bool fixed, int64_t t, int64_t chunk, const void* gmf, const void* gcf) {
+  return t % 4 == 0 || (chunk == bssm::kRot4Chunk && !(fixed && (gmf != nullptr || gcf != nullptr)));
 }
 
 // 16-byte staging is valid when every sequence row of the stream starts on a
@@ -98,7 +112,7 @@ int forward_impl(const char* fn, bool fixed, int d, int m, const float* keys, co
                  const float* queries, const float* decay, const float* process, const float* observation,
                  const float* mean0, const float* cov0, float* out, float* mean_final, float* cov_final,
                  float* bmean, float* bcov, int64_t n, int64_t t, int64_t chunk, float floor, void* stream,
-                 int fmt = bssm::kInF32) {
+                 int fmt = bssm::kInF32, bool whole = true) {
   if (int rc = check_common(fn, d, m, n, t, chunk, floor)) return rc;
   BSSM_REQUIRE_T(keys);
   BSSM_REQUIRE_T(values);
@@ -123,10 +137,12 @@ int forward_impl(const char* fn, bool fixed, int d, int m, const float* keys, co
   a.vec_kqd = vec_flag_fmt(keys, t, d, fmt) && vec_flag_fmt(queries, t, d, fmt) && (fixed || vec_flag(decay, t, d));
   a.vec_v = vec_flag_fmt(values, t, m, fmt) && vec_flag(out, t, m);
   a.vec_pr = fixed || (vec_flag(process, t, 1) && vec_flag(observation, t, 1));
-  a.rot4 = rot4_ok(d, m, t, a.nb, a.vec_kqd && a.vec_v && a.vec_pr, {mean0, cov0, mean_final, cov_final, bmean, bcov});
-  if (fmt != bssm::kInF32 && !a.rot4 && n > 0)
-    return fail(BSSM_ERR_UNSUPPORTED, "%s: %s inputs need D = 4, M = 8, T a positive multiple of 4 and "
-                "16-byte aligned streams", fn, fmt_name(fmt));
+  a.rot4 = rot4_ok(d, m, t, a.nb, {keys, values, queries, out, fixed ? nullptr : decay, fixed ? nullptr : process,
+                                   fixed ? nullptr : observation},
+                   {mean0, cov0, mean_final, cov_final, bmean, bcov});
+  if (fmt != bssm::kInF32 && (!a.rot4 || (whole && t % 4 != 0)) && n > 0)
+    return fail(BSSM_ERR_UNSUPPORTED, "%s: %s inputs need D = 4, M = 8, T a positive %s and 16-byte aligned streams",
+                fn, fmt_name(fmt), whole ? "multiple of 4" : "number");
   if (n == 0) return ok();
   return launched(fn, bssm::launch_forward(d, fixed, a, static_cast<hipStream_t>(stream)));
 }
@@ -142,7 +158,7 @@ int backward_impl(const char* fn, bool fixed, bool dyn, int d, int m, const floa
                   const float* queries, const float* decay, const float* process, const float* observation,
                   const float* mean0, const float* cov0, const float* bmean, const float* bcov, const float* gy,
                   const float* gmf, const float* gcf, BwdOut o, int64_t n, int64_t t, int64_t chunk, float floor,
-                  void* stream, int fmt = bssm::kInF32) {
+                  void* stream, int fmt = bssm::kInF32, bool whole = true) {
   if (int rc = check_common(fn, d, m, n, t, chunk, floor)) return rc;
   BSSM_REQUIRE_T(keys);
   BSSM_REQUIRE_T(values);
@@ -170,11 +186,14 @@ int backward_impl(const char* fn, bool fixed, bool dyn, int d, int m, const floa
   a.vec_pr = (fixed || (vec_flag(process, t, 1) && vec_flag(observation, t, 1))) && vec_flag(o.gp, t, 1) &&
              vec_flag(o.gr, t, 1);
   a.rot4 = (chunk == bssm::kRot4Chunk || chunk == 2 * bssm::kRot4Chunk) &&
-           rot4_ok(d, m, t, a.nb, a.vec_kqd && a.vec_v && a.vec_pr, {bmean, bcov, gmf, gcf, o.gm0, o.gc0});
-  if (fmt != bssm::kInF32 && !a.rot4 && n > 0)
-    return fail(BSSM_ERR_UNSUPPORTED, "%s: %s inputs need D = 4, M = 8, T a positive multiple of 4, "
-                "checkpoint chunk %d or %d and 16-byte aligned streams", fn, fmt_name(fmt), bssm::kRot4Chunk,
-                2 * bssm::kRot4Chunk);
+           rot4_ok(d, m, t, a.nb, {keys, values, queries, fixed ? nullptr : decay, fixed ? nullptr : process,
+                                   fixed ? nullptr : observation, gy, o.gk, o.gv, o.gq, o.gd, o.gp, o.gr},
+                   {bmean, bcov, gmf, gcf, o.gm0, o.gc0}) &&
+           rot4_tail_ok(fixed, t, chunk, gmf, gcf);
+  if (fmt != bssm::kInF32 && (!a.rot4 || (whole && t % 4 != 0)) && n > 0)
+    return fail(BSSM_ERR_UNSUPPORTED, "%s: %s inputs need D = 4, M = 8, T a positive %s, checkpoint chunk %d%s and "
+                "16-byte aligned streams", fn, fmt_name(fmt), whole ? "multiple of 4" : "number", bssm::kRot4Chunk,
+                whole ? " or 16" : ", no final-state gradients with fixed dynamics");
   if (n == 0) return ok();
   return launched(fn, bssm::launch_backward(d, fixed, dyn, a, static_cast<hipStream_t>(stream)));
 }
@@ -249,7 +268,7 @@ extern "C" {
 
 const char* bssm_last_error(void) { return g_error; }
 
-int bssm_abi_version(void) { return 9; }
+int bssm_abi_version(void) { return 10; }
 
 int bssm_supported(int key_dim, int value_dim) { return supported(key_dim, value_dim) ? 1 : 0; }
 
@@ -516,6 +535,46 @@ int bssm_backward_chunked_fp8(int key_dim, int value_dim, int fixed, int format,
                        BwdOut{static_cast<float*>(gk), static_cast<float*>(gv), static_cast<float*>(gq), gd, gp, gr,
                               gm0, gc0},
                        n, t, chunk, denominator_floor, stream, format == 0 ? bssm::kInE4M3 : bssm::kInE5M2);
+}
+
+// InFmt of the narrow entry points' format argument (the float8 ones' 0 and 1,
+// 2: bfloat16), or -1.
+static int narrow_format(int format) {
+  return format == 0 ? bssm::kInE4M3 : format == 1 ? bssm::kInE5M2 : format == 2 ? bssm::kInBf16 : -1;
+}
+
+int bssm_forward_chunked_narrow(int key_dim, int value_dim, int fixed, int format, const void* keys,
+                                const void* values, const void* queries, const float* decay, const float* process,
+                                const float* observation, const float* mean0, const float* cov0, float* out,
+                                float* mean_final, float* cov_final, float* bmean, float* bcov, int64_t n, int64_t t,
+                                int64_t chunk, float denominator_floor, void* stream) {
+  const char* fn = "bssm_forward_chunked_narrow";
+  const int fmt = narrow_format(format);
+  if (fmt < 0) return fail(BSSM_ERR_ARGUMENT, "%s: format must be 0, 1 or 2, got %d", fn, format);
+  return forward_impl(fn, fixed != 0, key_dim, value_dim, static_cast<const float*>(keys),
+                      static_cast<const float*>(values), static_cast<const float*>(queries), decay, process,
+                      observation, mean0, cov0, out, mean_final, cov_final, bmean, bcov, n, t, chunk,
+                      denominator_floor, stream, fmt, false);
+}
+
+int bssm_backward_chunked_narrow(int key_dim, int value_dim, int fixed, int format, const void* keys,
+                                 const void* values, const void* queries, const float* decay, const float* process,
+                                 const float* observation, const float* mean0, const float* cov0, const float* bmean,
+                                 const float* bcov, const float* gy, const float* gmf, const float* gcf, void* gk,
+                                 void* gv, void* gq, float* gd, float* gp, float* gr, float* gm0, float* gc0,
+                                 int64_t n, int64_t t, int64_t chunk, float denominator_floor, void* stream) {
+  const char* fn = "bssm_backward_chunked_narrow";
+  const int fmt = narrow_format(format);
+  if (fmt < 0) return fail(BSSM_ERR_ARGUMENT, "%s: format must be 0, 1 or 2, got %d", fn, format);
+  const bool dyn = gd != nullptr;
+  if ((gd == nullptr) != (gp == nullptr) || (gd == nullptr) != (gr == nullptr))
+    return fail(BSSM_ERR_ARGUMENT, "%s: gd, gp and gr must be given together or all be null", fn);
+  return backward_impl(fn, fixed != 0, dyn && !fixed, key_dim, value_dim, static_cast<const float*>(keys),
+                       static_cast<const float*>(values), static_cast<const float*>(queries), decay, process,
+                       observation, mean0, cov0, bmean, bcov, gy, gmf, gcf,
+                       BwdOut{static_cast<float*>(gk), static_cast<float*>(gv), static_cast<float*>(gq), gd, gp, gr,
+                              gm0, gc0},
+                       n, t, chunk, denominator_floor, stream, fmt, false);
 }
 
 int64_t bssm_value_stats_workspace(int count, const int64_t* numels) {

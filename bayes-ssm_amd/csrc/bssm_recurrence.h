@@ -80,10 +80,12 @@ hipError_t launch_backward_saved(int key_dim, bool dynamics_grads, const BwdArgs
                                  hipStream_t stream);
 // D = 4, M = 8 kernels with the rotated per-lane layout (bssm_rot4.hip).
 // Preconditions (checked by the C ABI, recorded in rot4): 16-byte aligned
-// streams, T a positive multiple of 4, 8-byte aligned belief tensors, and for
-// the backward a checkpoint chunk of kRot4Chunk tokens (a record per chunk)
-// or 2 * kRot4Chunk (a record per 16-token tile; the tile's second chunk
-// starts from the belief advanced on chip over its first 8 tokens).
+// stream bases, T > 0, 8-byte aligned belief tensors, and for the backward a
+// checkpoint chunk of kRot4Chunk tokens (a record per chunk) or, with T a
+// multiple of 4, 2 * kRot4Chunk (a record per 16-token tile; the tile's
+// second chunk starts from the belief advanced on chip over its first 8
+// tokens).  With T not a multiple of 4 and fixed dynamics the backward takes
+// no final-state gradients.
 constexpr int kRot4Chunk = 8;
 hipError_t launch_forward_r4(bool fixed, const FwdArgs& a, hipStream_t stream);
 hipError_t launch_backward_r4(bool fixed, bool dyn, const BwdArgs& a, hipStream_t stream);
@@ -92,7 +94,8 @@ hipError_t launch_backward_r4(bool fixed, bool dyn, const BwdArgs& a, hipStream_
 // most small_batch_limit(0) (forward) or small_batch_limit(1) (backward);
 // as two / three waves per 4 sequences up to small_batch_limit(2) / (3).
 hipError_t launch_forward_small(bool fixed, const FwdArgs& a, hipStream_t stream);
-// The backward needs T a multiple of 16 and the kRot4Chunk checkpoint chunk.
+// The backward needs the kRot4Chunk checkpoint chunk and, with fixed dynamics
+// and final-state gradients, T a multiple of 16.
 hipError_t launch_backward_small(bool fixed, bool dyn, const BwdArgs& a, hipStream_t stream);
 int64_t small_batch_limit(int direction);
 int64_t set_small_batch_limit(int direction, int64_t limit);

@@ -138,6 +138,12 @@ __device__ __forceinline__ void st32(Rsrc r, float x, uint32_t voff, uint32_t so
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), r, static_cast<int>(voff),
                                         static_cast<int>(soff), 0);
 }
+// The first `words` 32-bit words of a 16-byte piece (the piece across the end
+// of a row whose bytes are not a multiple of 16: the rest is the next row's).
+__device__ __forceinline__ void store_words(Rsrc r, v4f x, uint32_t voff, int words, uint32_t soff = 0) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) st32(r, x[e], e < words ? voff + 4u * e : kOob, soff);
+}
 __device__ __forceinline__ v2f ld64(Rsrc r, uint32_t voff, uint32_t soff) {
   return __builtin_bit_cast(v2f, __builtin_amdgcn_raw_buffer_load_b64(r, static_cast<int>(voff),
                                                                       static_cast<int>(soff), 0));
@@ -963,6 +969,24 @@ struct BwdCore {
       StepOut o;
       forward_step(b, x[tt], floor, o);
       __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  // Tokens len .. 15 of a tile of two slots made neutral: k = q = v = gy = 0,
+  // d = 1, p = 0, r = 1.  Their step leaves the belief and their reverse the
+  // carried adjoints as they are, bit for bit, so a chunk that T ends in runs
+  // whole.  (With FIXED the constant d and p are not neutral: only for zero
+  // adjoints, that is without final-state gradients.)
+  __device__ __forceinline__ void neutral_tail(float* tile, int len) const {
+    for (int t = len; t < 2 * SUB; ++t) {
+      float* tl = tile + (t >> 3) * BwdTile::SIZE;
+      const int tt = t & 7, w = ix.i4(tt, g);
+      (tl + BwdTile::K)[w] = (tl + BwdTile::Q)[w] = 0.f;
+      (tl + BwdTile::D)[w] = 1.f;
+      const v2f zero = {0.f, 0.f};
+      *reinterpret_cast<v2f*>(&(tl + BwdTile::V)[ix.i8(tt)]) = zero;
+      *reinterpret_cast<v2f*>(&(tl + BwdTile::GY)[ix.i8(tt)]) = zero;
+      (tl + BwdTile::P)[ix.i1(tt)] = 0.f;
+      (tl + BwdTile::R)[ix.i1(tt)] = 1.f;
     }
   }
   // A chunk of `len` tokens (SUB, or 4 for the last one of T = 8n + 4).

@@ -235,7 +235,13 @@ struct BwdOutQ {
 // F: format of keys, values, queries and their gradients (InFmt).  IV:
 // checkpoint interval, 8 (a record per chunk slot) or 16 (a record per tile:
 // the tile's second chunk starts from the belief advanced over its first).
-template <bool FIXED, bool DYN, int F, int IV>
+// RAG: T is not a multiple of 4.  The last tile's tokens at and past T are
+// made neutral in LDS and its chunks run whole; pieces of several tokens that
+// straddle T are stored word by word; p and r carry their whole offset in the
+// range-checked operand, since a piece may reach past the last row.  A
+// template parameter, so that the register-bound loop of the other case
+// stays as it is.
+template <bool FIXED, bool DYN, int F, int IV, bool RAG>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1, 1))) void backward_tile_kernel(
     BwdArgs a) {
   static_assert(IV == SUB || IV == 2 * SUB, "checkpoint interval of one or two chunk slots");
@@ -320,8 +326,13 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1, 1))) v
     for (int I = 0; I < 8; ++I) x.gy[I] = ld128<kNtLoad>(rgy, in8 ? tm.o8[I] : kOob, s8);
     if constexpr (!FIXED) {
       const uint32_t s1 = static_cast<uint32_t>(t0) * 4u;
-      x.p = ld128<false>(rp, in1 ? tm.o1 : kOob, s1);
-      x.r = ld128<false>(rr, in1 ? tm.o1 : kOob, s1);
+      if constexpr (RAG) {
+        x.p = ld128<false>(rp, in1 ? tm.o1 + s1 : kOob);
+        x.r = ld128<false>(rr, in1 ? tm.o1 + s1 : kOob);
+      } else {
+        x.p = ld128<false>(rp, in1 ? tm.o1 : kOob, s1);
+        x.r = ld128<false>(rr, in1 ? tm.o1 : kOob, s1);
+      }
     }
   };
   auto put = [&](const Stage& x) __attribute__((always_inline)) {
@@ -429,6 +440,41 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1, 1))) v
     const uint32_t sk = static_cast<uint32_t>(t0 * e4), sv = static_cast<uint32_t>(t0 * e8);
     const uint32_t s4 = static_cast<uint32_t>(t0) * 16u, s8 = static_cast<uint32_t>(t0) * 32u;
     const bool in4 = t0 + tm.t4 < T, in8 = t0 + tm.t8 < T;
+    if (RAG && t0 + 2 * SUB > T) {
+      // The last tile: pieces of 2 (bf16) or 4 and 2 (float8) tokens, and of 4
+      // scalars, may straddle T.
+      const int len = static_cast<int>(T - t0);
+      if constexpr (W) {
+#pragma unroll
+        for (int I = 0; I < 4; ++I) {
+          st128<kNtStore>(rgk, o.k[I], in4 ? tm.o4[I] : kOob, s4);
+          st128<kNtStore>(rgq, o.q[I], in4 ? tm.o4[I] : kOob, s4);
+        }
+#pragma unroll
+        for (int I = 0; I < 8; ++I) st128<kNtStore>(rgv, o.v[I], in8 ? tm.o8[I] : kOob, s8);
+      } else if constexpr (Q8) {
+        store_words(rgk, o.k, qm.k_off, len - qm.k_tok, sk);
+        store_words(rgq, o.q, qm.k_off, len - qm.k_tok, sk);
+#pragma unroll
+        for (int I = 0; I < 2; ++I) store_words(rgv, o.v[I], qm.v_off[I], 2 * (len - qm.v_tok), sv);
+      } else {
+#pragma unroll
+        for (int I = 0; I < 2; ++I) {
+          store_words(rgk, o.k[I], hm.k_off[I], 2 * (len - hm.k_tok), sk);
+          store_words(rgq, o.q[I], hm.k_off[I], 2 * (len - hm.k_tok), sk);
+        }
+#pragma unroll
+        for (int I = 0; I < 4; ++I) st128<kNtStore>(rgv, o.v[I], hm.v_tok < len ? hm.v_off[I] : kOob, sv);
+      }
+      if (a.gd) {
+#pragma unroll
+        for (int I = 0; I < 4; ++I) st128<kNtStore>(rgd, o.d[I], in4 ? tm.o4[I] : kOob, s4);
+      }
+      const uint32_t s1 = static_cast<uint32_t>(t0) * 4u;
+      if (a.gp) store_words(rgp, o.p, tm.o1, len - tm.t1, s1);
+      if (a.gr) store_words(rgr, o.r, tm.o1, len - tm.t1, s1);
+      return;
+    }
     if constexpr (W) {
 #pragma unroll
       for (int I = 0; I < 4; ++I) {
@@ -470,7 +516,8 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1, 1))) v
     Bel b;
     bel_from_lds(b, tl + BwdTile::CK, s, g);
     if (c >= 2) issue_ck(tl, c - 2);
-    core.run(tl, b, chunk_len(c));
+    if constexpr (RAG) core.template process<SUB>(tl, b);
+    else core.run(tl, b, chunk_len(c));
   };
   // Tile J with one record (interval 16, in slot 0's checkpoint region): the
   // second chunk starts from the record advanced over the first chunk's 8
@@ -509,6 +556,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1, 1))) v
     if (J + 1 < ntiles) take(go);
     __builtin_amdgcn_sched_barrier(0);
     put(st);
+    if (RAG && J + 1 == ntiles) core.neutral_tail(tile, static_cast<int>(T - J * 2 * SUB));
     __builtin_amdgcn_sched_barrier(0);
     if (J + 1 < ntiles) store_grads(go, J + 1);
     if (J > 0) load(st, J - 1);
@@ -555,30 +603,22 @@ hipError_t launch_forward_r4(bool fixed, const FwdArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <int IV>
+template <int F, int IV, bool RAG>
+void launch_backward_r4_fmt(bool fixed, bool dyn, const BwdArgs& a, dim3 grid, hipStream_t stream) {
+  const dim3 block(kWave);
+  if (fixed) hipLaunchKernelGGL((r4::backward_tile_kernel<true, false, F, IV, RAG>), grid, block, 0, stream, a);
+  else if (dyn) hipLaunchKernelGGL((r4::backward_tile_kernel<false, true, F, IV, RAG>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((r4::backward_tile_kernel<false, false, F, IV, RAG>), grid, block, 0, stream, a);
+}
+template <int IV, bool RAG>
 hipError_t launch_backward_r4_iv(bool fixed, bool dyn, const BwdArgs& a, hipStream_t stream) {
   const int64_t blocks = (a.n + r4::SPW - 1) / r4::SPW;
-  const dim3 grid(static_cast<unsigned>(blocks)), block(kWave);
+  const dim3 grid(static_cast<unsigned>(blocks));
   switch (a.in_fmt) {
-    case kInBf16:
-      if (fixed) hipLaunchKernelGGL((r4::backward_tile_kernel<true, false, kInBf16, IV>), grid, block, 0, stream, a);
-      else if (dyn) hipLaunchKernelGGL((r4::backward_tile_kernel<false, true, kInBf16, IV>), grid, block, 0, stream, a);
-      else hipLaunchKernelGGL((r4::backward_tile_kernel<false, false, kInBf16, IV>), grid, block, 0, stream, a);
-      break;
-    case kInE4M3:
-      if (fixed) hipLaunchKernelGGL((r4::backward_tile_kernel<true, false, kInE4M3, IV>), grid, block, 0, stream, a);
-      else if (dyn) hipLaunchKernelGGL((r4::backward_tile_kernel<false, true, kInE4M3, IV>), grid, block, 0, stream, a);
-      else hipLaunchKernelGGL((r4::backward_tile_kernel<false, false, kInE4M3, IV>), grid, block, 0, stream, a);
-      break;
-    case kInE5M2:
-      if (fixed) hipLaunchKernelGGL((r4::backward_tile_kernel<true, false, kInE5M2, IV>), grid, block, 0, stream, a);
-      else if (dyn) hipLaunchKernelGGL((r4::backward_tile_kernel<false, true, kInE5M2, IV>), grid, block, 0, stream, a);
-      else hipLaunchKernelGGL((r4::backward_tile_kernel<false, false, kInE5M2, IV>), grid, block, 0, stream, a);
-      break;
-    default:
-      if (fixed) hipLaunchKernelGGL((r4::backward_tile_kernel<true, false, kInF32, IV>), grid, block, 0, stream, a);
-      else if (dyn) hipLaunchKernelGGL((r4::backward_tile_kernel<false, true, kInF32, IV>), grid, block, 0, stream, a);
-      else hipLaunchKernelGGL((r4::backward_tile_kernel<false, false, kInF32, IV>), grid, block, 0, stream, a);
+    case kInBf16: launch_backward_r4_fmt<kInBf16, IV, RAG>(fixed, dyn, a, grid, stream); break;
+    case kInE4M3: launch_backward_r4_fmt<kInE4M3, IV, RAG>(fixed, dyn, a, grid, stream); break;
+    case kInE5M2: launch_backward_r4_fmt<kInE5M2, IV, RAG>(fixed, dyn, a, grid, stream); break;
+    default: launch_backward_r4_fmt<kInF32, IV, RAG>(fixed, dyn, a, grid, stream);
   }
   return hipGetLastError();
 }
@@ -587,9 +627,13 @@ hipError_t launch_backward_r4_iv(bool fixed, bool dyn, const BwdArgs& a, hipStre
 hipError_t launch_backward_r4(bool fixed, bool dyn, const BwdArgs& a, hipStream_t stream) {
   const int64_t blocks = (a.n + r4::SPW - 1) / r4::SPW;
   if (blocks == 0) return hipSuccess;
-  if (a.chunk == 2 * kRot4Chunk) return launch_backward_r4_iv<2 * kRot4Chunk>(fixed, dyn, a, stream);
+  if (a.chunk == 2 * kRot4Chunk) {
+    if (a.t % 4 != 0) return hipErrorInvalidValue;
+    return launch_backward_r4_iv<2 * kRot4Chunk, false>(fixed, dyn, a, stream);
+  }
   if (a.chunk != kRot4Chunk) return hipErrorInvalidValue;
-  return launch_backward_r4_iv<kRot4Chunk>(fixed, dyn, a, stream);
+  if (a.t % 4 != 0) return launch_backward_r4_iv<kRot4Chunk, true>(fixed, dyn, a, stream);
+  return launch_backward_r4_iv<kRot4Chunk, false>(fixed, dyn, a, stream);
 }
 
 }  // namespace bssm

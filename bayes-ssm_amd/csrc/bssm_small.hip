@@ -59,6 +59,7 @@ constexpr int kQuadRev = quad_perm(3, 2, 1, 0);
 using r4::Rsrc;
 using r4::make_rsrc;
 using r4::kOob;
+using r4::store_words;
 using r4::v4u;
 typedef float v2f __attribute__((ext_vector_type(2)));
 
@@ -158,8 +159,11 @@ __device__ __forceinline__ void put_v(float* dst, v4f v0, v4f v1, int c) {
 // The reverse: gradients in a region of TOK x 4 / TOK x 8 floats leave as
 // 16-byte pieces of format F (bfloat16: round to nearest even; float8:
 // narrow_f8, torch's rounding), at the loaders' offsets.
+// With len < TOK only the first len tokens' values are stored (a row that
+// ends inside the block: the piece across its end leaves word by word).
 template <int F, int TOK>
-__device__ __forceinline__ void store_kq(Rsrc r, uint32_t row, int s, int c, uint32_t t0, const float* src) {
+__device__ __forceinline__ void store_kq(Rsrc r, uint32_t row, int s, int c, uint32_t t0, int len,
+                                         const float* src) {
   const uint32_t off = static_cast<uint32_t>(s) * row + t0 * kq_bytes<F>() + static_cast<uint32_t>(c) * 16u;
   const uint32_t o = c < kq_lanes<F, TOK>() ? off : kOob;
   const int cc = c & (kq_lanes<F, TOK>() - 1);
@@ -174,10 +178,12 @@ __device__ __forceinline__ void store_kq(Rsrc r, uint32_t row, int s, int c, uin
     for (int u = 0; u < 4; ++u) w[u] = narrow_f8<F>(*reinterpret_cast<const v4f*>(src + 16 * cc + 4 * u));
     x = __builtin_bit_cast(v4f, w);
   }
-  r4::st128<r4::kNtStore>(r, x, o, 0);
+  if (len == TOK) r4::st128<r4::kNtStore>(r, x, o, 0);
+  else store_words(r, x, off, c < kq_lanes<F, TOK>() ? len * static_cast<int>(kq_bytes<F>() / 4) - 4 * c : 0);
 }
 template <int F, int TOK>
-__device__ __forceinline__ void store_v(Rsrc r, uint32_t row, int s, int c, uint32_t t0, const float* src) {
+__device__ __forceinline__ void store_v(Rsrc r, uint32_t row, int s, int c, uint32_t t0, int len,
+                                        const float* src) {
   static_assert(TOK * 2 * kq_bytes<F>() <= 256u, "one piece per lane");
   const uint32_t off = static_cast<uint32_t>(s) * row + t0 * 2u * kq_bytes<F>() + static_cast<uint32_t>(c) * 16u;
   const int lanes = 2 * kq_lanes<F, TOK>();
@@ -194,7 +200,8 @@ __device__ __forceinline__ void store_v(Rsrc r, uint32_t row, int s, int c, uint
     for (int u = 0; u < 4; ++u) w[u] = narrow_f8<F>(*reinterpret_cast<const v4f*>(src + 16 * cc + 4 * u));
     x = __builtin_bit_cast(v4f, w);
   }
-  r4::st128<r4::kNtStore>(r, x, o, 0);
+  if (len == TOK) r4::st128<r4::kNtStore>(r, x, o, 0);
+  else store_words(r, x, off, c < lanes ? len * static_cast<int>(kq_bytes<F>() / 2) - 4 * c : 0);
 }
 
 struct Streams {
@@ -1026,9 +1033,9 @@ __global__ __launch_bounds__(kWave) void rotation_forward_kernel(RotArgs a) {
 }
 
 // ----------------------------------------------------------------- backward
-// A 16-token tile holds two checkpoint chunks of 8 tokens (T a multiple of
-// 16); tiles are visited last to first, and in each the chunk 2J + 1 before
-// the chunk 2J.  A chunk is replayed from its checkpoint, keeping each
+// A 16-token tile holds two checkpoint chunks of 8 tokens; tiles are visited
+// last to first, and in each the chunk 2J + 1 before the chunk 2J.  The last
+// tile's tokens at and past T are filled with neutral ones (neutral_tail).  A chunk is replayed from its checkpoint, keeping each
 // token's belief and step intermediates in registers, and then reversed.
 // Gradients overwrite their inputs in the tile (gk over k, gq over q, gd over
 // d, gv over v, gp over p, gr over r) and leave with the next tile's loads.
@@ -1039,6 +1046,28 @@ __global__ __launch_bounds__(kWave) void rotation_forward_kernel(RotArgs a) {
 struct BTile {
   static constexpr int K = 0, D = 64, Q = 128, V = 192, GY = 320, P = 448, R = 464, SEQ = 488, SIZE = SPW * SEQ;
 };
+
+// Tokens len .. CAP - 1 of a sequence's LDS region (layout L) made neutral:
+// k = q = v = gy = 0, d = 1, p = 0, r = 1.  Their step leaves the belief as it
+// is (u = 0, e = 0) and their reverse leaves the carried adjoints as they are
+// (a = w = 0), bit for bit, so the unrolled chunks need no length test.  With
+// fixed dynamics d and p are constants and this does not hold for nonzero
+// carried adjoints: such calls (final-state gradients) take other kernels
+// when T ends inside a chunk.  Lane c of the sequence's 16.
+template <typename L, int CAP>
+__device__ __forceinline__ void neutral_tail(float* b, int len, int c) {
+  for (int t = len; t < CAP; ++t) {
+    if (c < 8) b[L::V + 8 * t + c] = b[L::GY + 8 * t + c] = 0.f;
+    if (c < 4) {
+      b[L::K + 4 * t + c] = b[L::Q + 4 * t + c] = 0.f;
+      b[L::D + 4 * t + c] = 1.f;
+    }
+    if (c == 0) {
+      b[L::P + t] = 0.f;
+      b[L::R + t] = 1.f;
+    }
+  }
+}
 
 struct BStage {
   v4f k, d, q, v0, v1, g0, g1, p, r;
@@ -1109,18 +1138,26 @@ __device__ __forceinline__ void get_grads(GStage& g, const float* tl, int s, int
 template <bool DYN>
 __device__ __forceinline__ void store_grads(const GStage& g, const BStreams& st, const BwdArgs& a, int s, int c,
                                             uint32_t t0) {
-  const uint32_t o4 = static_cast<uint32_t>(s) * st.row4 + (t0 + c) * 16u;
+  // Tokens of the tile below T; a partial (last) tile drops the others' pieces.
+  const int len = static_cast<int>(a.t - t0) < TT ? static_cast<int>(a.t - t0) : TT;
+  const uint32_t o4 = c < len ? static_cast<uint32_t>(s) * st.row4 + (t0 + c) * 16u : kOob;
   r4::st128<r4::kNtStore>(st.gk, g.k, o4, 0);
   r4::st128<r4::kNtStore>(st.gq, g.q, o4, 0);
   const uint32_t o8 = static_cast<uint32_t>(s) * st.row8 + t0 * 32u + c * 16u;
-  r4::st128<r4::kNtStore>(st.gv, g.v0, o8, 0);
-  r4::st128<r4::kNtStore>(st.gv, g.v1, o8 + 256u, 0);
+  r4::st128<r4::kNtStore>(st.gv, g.v0, (c >> 1) < len ? o8 : kOob, 0);
+  r4::st128<r4::kNtStore>(st.gv, g.v1, ((c + 16) >> 1) < len ? o8 + 256u : kOob, 0);
   // Without dynamics gradients, requested gd / gp / gr outputs are zero.
   const v4f zero = v4f{0.f, 0.f, 0.f, 0.f};
   if (a.gd) r4::st128<r4::kNtStore>(st.gd, DYN ? g.d : zero, o4, 0);
   const uint32_t o1 = c < 4 ? static_cast<uint32_t>(s) * st.row1 + t0 * 4u + c * 16u : kOob;
-  if (a.gp) r4::st128(st.gp, DYN ? g.p : zero, o1, 0);
-  if (a.gr) r4::st128(st.gr, DYN ? g.r : zero, o1, 0);
+  if (len == TT) {
+    if (a.gp) r4::st128(st.gp, DYN ? g.p : zero, o1, 0);
+    if (a.gr) r4::st128(st.gr, DYN ? g.r : zero, o1, 0);
+  } else {
+    const int words = c < 4 ? len - 4 * c : 0;
+    if (a.gp) store_words(st.gp, DYN ? g.p : zero, o1, words);
+    if (a.gr) store_words(st.gr, DYN ? g.r : zero, o1, words);
+  }
 }
 
 // Replay record of one token: the belief before it and the step's
@@ -1346,11 +1383,13 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
     }
   };
 
-  const int64_t ntiles = T / TT;
+  const int64_t ntiles = (T + TT - 1) / TT;
   BStage x;
   Bel nk0, nk1;
   if (ntiles > 0) {
     load_btile<FIXED>(x, st, s, c, static_cast<uint32_t>((ntiles - 1) * TT));
+    // A last tile of at most 8 tokens has no second chunk: its neutral tokens
+    // start from the final belief (record nb).
     load_ckpt(nk0, 2 * (ntiles - 1));
     load_ckpt(nk1, 2 * (ntiles - 1) + 1);
   }
@@ -1362,6 +1401,7 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
     r4::vm_wait<0>();
     const Bel k0 = nk0, k1 = nk1;
     put_btile<FIXED>(x, tile, s, c);
+    if (t0 + TT > T) neutral_tail<BTile, TT>(mine, static_cast<int>(T - t0), c);
     if (ti + 1 < ntiles) store_grads<DYN>(go, st, a, s, c, t0 + TT);
     if (ti > 0) {
       load_btile<FIXED>(x, st, s, c, t0 - TT);
@@ -1519,7 +1559,10 @@ __global__ __launch_bounds__(3 * G * kWave) void backward_split_kernel(BwdArgs a
   const uint32_t row4 = static_cast<uint32_t>(T) * 16u, row8 = static_cast<uint32_t>(T) * 32u,
                  row1 = static_cast<uint32_t>(T) * 4u;
   const uint32_t nbp = static_cast<uint32_t>(a.nb + 1);
-  const int64_t nb = T / CH;  // chunks; position x is chunk nb - 1 - x
+  const int64_t nb = (T + CH - 1) / CH;  // chunks; position x is chunk nb - 1 - x
+  // Tokens of chunk position x (position 0 holds the row's end).
+  const int len0 = static_cast<int>(T - (nb - 1) * CH);
+  auto clen = [&](int64_t x) __attribute__((always_inline)) { return x == 0 ? len0 : CH; };
   // Ring slots of step position x (T / 8 positions: 32-bit arithmetic).
   auto slot = [&](int64_t x) __attribute__((always_inline)) {
     return lds + SBTile::IN + static_cast<int>(static_cast<uint32_t>(x) % SBTile::NSLOT) * SBTile::SLOT +
@@ -1588,6 +1631,7 @@ __global__ __launch_bounds__(3 * G * kWave) void backward_split_kernel(BwdArgs a
       put_v<F, CH>(b + SBTile::V, sv, sv1, c);
       *reinterpret_cast<v4f*>(b + SBTile::GY + 4 * c) = sg;
       *reinterpret_cast<v2f*>(b + SBTile::MC + 2 * c) = sm;
+      if (x == 0 && len0 < CH) neutral_tail<SBTile, CH>(b, len0, c);
     };
     auto ckpt = [&](int64_t x) __attribute__((always_inline)) {
       return r4::ld32(rbc, cco + static_cast<uint32_t>(nb - 1 - x) * 64u, 0);
@@ -1604,19 +1648,29 @@ __global__ __launch_bounds__(3 * G * kWave) void backward_split_kernel(BwdArgs a
     auto store_mean = [&](int64_t x) __attribute__((always_inline)) {
       const float* b = slot(x);
       const uint32_t t0 = tok0(x);
-      store_kq<F, CH>(rgq, row4n, s, c, t0, b + SBTile::Q);
-      store_v<F, CH>(rgv, row8n, s, c, t0, b + SBTile::V);
+      const int len = clen(x);
+      store_kq<F, CH>(rgq, row4n, s, c, t0, len, b + SBTile::Q);
+      store_v<F, CH>(rgv, row8n, s, c, t0, len, b + SBTile::V);
     };
     auto store_cov = [&](int64_t x) __attribute__((always_inline)) {
       const float* b = slot(x);
       const uint32_t t0 = tok0(x);
-      const uint32_t q4 = c < CH ? o4 + t0 * 16u : kOob, q1 = c < CH / 4 ? o1 + t0 * 4u : kOob;
+      const int len = clen(x);
+      const uint32_t q4 = c < len ? o4 + t0 * 16u : kOob, q1 = c < CH / 4 ? o1 + t0 * 4u : kOob;
       const v4f zero = v4f{0.f, 0.f, 0.f, 0.f};
       const int c8 = c & (CH - 1), c2 = c & (CH / 4 - 1);
-      store_kq<F, CH>(rgk, row4n, s, c, t0, b + SBTile::K);
+      store_kq<F, CH>(rgk, row4n, s, c, t0, len, b + SBTile::K);
       if (a.gd) r4::st128<r4::kNtStore>(rgd, DYN ? *reinterpret_cast<const v4f*>(b + SBTile::D + 4 * c8) : zero, q4, 0);
-      if (a.gp) r4::st128(rgp, DYN ? *reinterpret_cast<const v4f*>(b + SBTile::P + 4 * c2) : zero, q1, 0);
-      if (a.gr) r4::st128(rgr, DYN ? *reinterpret_cast<const v4f*>(b + SBTile::R + 4 * c2) : zero, q1, 0);
+      const v4f xp = DYN ? *reinterpret_cast<const v4f*>(b + SBTile::P + 4 * c2) : zero;
+      const v4f xr = DYN ? *reinterpret_cast<const v4f*>(b + SBTile::R + 4 * c2) : zero;
+      if (len == CH) {
+        if (a.gp) r4::st128(rgp, xp, q1, 0);
+        if (a.gr) r4::st128(rgr, xr, q1, 0);
+      } else {
+        const int words = c < CH / 4 ? len - 4 * c : 0;
+        if (a.gp) store_words(rgp, xp, q1, words);
+        if (a.gr) store_words(rgr, xr, q1, words);
+      }
     };
     float Pload = 0.f;
     if (nb > 0) {
@@ -1903,7 +1957,7 @@ void launch_backward_split(bool fixed, bool dyn, const BwdArgs& a, dim3, hipStre
 // bf16 / float8 streams run the three-wave kernel only (the dispatch keeps
 // them within its limit).
 hipError_t launch_backward_small(bool fixed, bool dyn, const BwdArgs& a, hipStream_t stream) {
-  if (a.t % sn::TT != 0 || a.chunk != kRot4Chunk) return hipErrorInvalidValue;
+  if (a.chunk != kRot4Chunk) return hipErrorInvalidValue;
   const int64_t blocks = (a.n + sn::SPW - 1) / sn::SPW;
   if (blocks == 0) return hipSuccess;
   const dim3 grid(static_cast<unsigned>(blocks));

@@ -293,6 +293,26 @@ int bssm_backward_chunked_fp8(int key_dim, int value_dim, int fixed, int format,
                               float* gm0, float* gc0,
                               int64_t n, int64_t t, int64_t chunk, float denominator_floor, void* stream);
 
+/* The same two directions for every narrow format (0, 1: as above; 2:
+ * bfloat16) and every T > 0: rows that do not start on a 16-byte boundary are
+ * read and written in place.  With T not a multiple of 4 the backward needs
+ * checkpoint chunk bssm_preferred_checkpoint(4), and fixed dynamics together
+ * with final-state gradients (gmf, gcf) return BSSM_ERR_UNSUPPORTED. */
+int bssm_forward_chunked_narrow(int key_dim, int value_dim, int fixed, int format,
+                                const void* keys, const void* values, const void* queries,
+                                const float* decay, const float* process, const float* observation,
+                                const float* mean0, const float* cov0,
+                                float* out, float* mean_final, float* cov_final, float* bmean, float* bcov,
+                                int64_t n, int64_t t, int64_t chunk, float denominator_floor, void* stream);
+int bssm_backward_chunked_narrow(int key_dim, int value_dim, int fixed, int format,
+                                 const void* keys, const void* values, const void* queries,
+                                 const float* decay, const float* process, const float* observation,
+                                 const float* mean0, const float* cov0, const float* bmean, const float* bcov,
+                                 const float* gy, const float* gmf, const float* gcf,
+                                 void* gk, void* gv, void* gq, float* gd, float* gp, float* gr,
+                                 float* gm0, float* gc0,
+                                 int64_t n, int64_t t, int64_t chunk, float denominator_floor, void* stream);
+
 /* Host-side float32 -> float8 rounding of the float8 gradients (format as
  * above): round to nearest even; e4m3fn gives the NaN code 0x7f (with the
  * sign) for magnitudes that round past 448, for infinities and NaN; e5m2

@@ -43,11 +43,8 @@ bool aligned8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0
 // pieces.  They take every T: a row that does not start on a 16-byte boundary
 // (T not a multiple of 4) is moved by the same 16-byte accesses, which the
 // buffer instructions allow at any 4-byte aligned address.
-bool rot4_ok(int d, int m, int64_t t, int64_t nb, std::initializer_list<const void*> streams,
-             std::initializer_list<const void*> belief) {
-  if (d != 4 || m != 8 || t <= 0) return false;
-  for (const void* p : streams)
-    if (p != nullptr && !aligned16(p)) return false;
+bool rot4_ok(int d, int m, int64_t t, int64_t nb, bool base16, std::initializer_list<const void*> belief) {
+  if (d != 4 || m != 8 || t <= 0 || !base16) return false;
   if ((nb + 1) * 128 * 16 >= ((int64_t)1 << 31)) return false;
   for (const void* p : belief)
     if (p != nullptr && !aligned8(p)) return false;
@@ -63,15 +60,11 @@ bool rot4_tail_ok(bool fixed, int64_t t, int64_t chunk, const void* gmf, const v
   return t % 4 == 0 || (chunk == bssm::kRot4Chunk && !(fixed && (gmf != nullptr || gcf != nullptr)));
 }
 
-// 16-byte staging is valid when every sequence row of the stream starts on a
-// 16-byte boundary: base aligned and (T * width) a multiple of 4 floats.
-int vec_flag(const float* p, int64_t t, int64_t width) {
-  return (p == nullptr || aligned16(p)) && ((t * width) % 4 == 0);
-}
-// The same for a stream of the input format fmt (InFmt: 4, 8 or 16 elements per 16 bytes).
-int vec_flag_fmt(const void* p, int64_t t, int64_t width, int fmt) {
-  const int64_t per16 = fmt == bssm::kInF32 ? 4 : fmt == bssm::kInBf16 ? 8 : 16;
-  return (p == nullptr || aligned16(p)) && ((t * width) % per16 == 0);
+// Every given pointer on a 16-byte boundary.
+bool all_aligned16(std::initializer_list<const void*> ptrs) {
+  for (const void* p : ptrs)
+    if (p != nullptr && !aligned16(p)) return false;
+  return true;
 }
 const char* fmt_name(int fmt) {
   return fmt == bssm::kInBf16 ? "bfloat16" : fmt == bssm::kInE4M3 ? "float8_e4m3fn" : "float8_e5m2";
@@ -134,12 +127,9 @@ int forward_impl(const char* fn, bool fixed, int d, int m, const float* keys, co
   a.m0 = mean0; a.c0 = cov0; a.y = out; a.mT = mean_final; a.cT = cov_final; a.bm = bmean; a.bc = bcov;
   a.n = n; a.t = t; a.chunk = chunk; a.nb = (t + chunk - 1) / chunk; a.floor = floor;
   a.in_fmt = fmt;
-  a.vec_kqd = vec_flag_fmt(keys, t, d, fmt) && vec_flag_fmt(queries, t, d, fmt) && (fixed || vec_flag(decay, t, d));
-  a.vec_v = vec_flag_fmt(values, t, m, fmt) && vec_flag(out, t, m);
-  a.vec_pr = fixed || (vec_flag(process, t, 1) && vec_flag(observation, t, 1));
-  a.rot4 = rot4_ok(d, m, t, a.nb, {keys, values, queries, out, fixed ? nullptr : decay, fixed ? nullptr : process,
-                                   fixed ? nullptr : observation},
-                   {mean0, cov0, mean_final, cov_final, bmean, bcov});
+  a.base16 = all_aligned16({keys, values, queries, out, fixed ? nullptr : decay, fixed ? nullptr : process,
+                            fixed ? nullptr : observation});
+  a.rot4 = rot4_ok(d, m, t, a.nb, a.base16, {mean0, cov0, mean_final, cov_final, bmean, bcov});
   if (fmt != bssm::kInF32 && (!a.rot4 || (whole && t % 4 != 0)) && n > 0)
     return fail(BSSM_ERR_UNSUPPORTED, "%s: %s inputs need D = 4, M = 8, T a positive %s and 16-byte aligned streams",
                 fn, fmt_name(fmt), whole ? "multiple of 4" : "number");
@@ -180,15 +170,10 @@ int backward_impl(const char* fn, bool fixed, bool dyn, int d, int m, const floa
   a.gk = o.gk; a.gv = o.gv; a.gq = o.gq; a.gd = o.gd; a.gp = o.gp; a.gr = o.gr; a.gm0 = o.gm0; a.gc0 = o.gc0;
   a.n = n; a.t = t; a.chunk = chunk; a.nb = (t + chunk - 1) / chunk; a.floor = floor;
   a.in_fmt = fmt;
-  a.vec_kqd = vec_flag_fmt(keys, t, d, fmt) && vec_flag_fmt(queries, t, d, fmt) && (fixed || vec_flag(decay, t, d)) &&
-              vec_flag_fmt(o.gk, t, d, fmt) && vec_flag_fmt(o.gq, t, d, fmt) && vec_flag(o.gd, t, d);
-  a.vec_v = vec_flag_fmt(values, t, m, fmt) && vec_flag(gy, t, m) && vec_flag_fmt(o.gv, t, m, fmt);
-  a.vec_pr = (fixed || (vec_flag(process, t, 1) && vec_flag(observation, t, 1))) && vec_flag(o.gp, t, 1) &&
-             vec_flag(o.gr, t, 1);
+  a.base16 = all_aligned16({keys, values, queries, fixed ? nullptr : decay, fixed ? nullptr : process,
+                            fixed ? nullptr : observation, gy, o.gk, o.gv, o.gq, o.gd, o.gp, o.gr});
   a.rot4 = (chunk == bssm::kRot4Chunk || chunk == 2 * bssm::kRot4Chunk) &&
-           rot4_ok(d, m, t, a.nb, {keys, values, queries, fixed ? nullptr : decay, fixed ? nullptr : process,
-                                   fixed ? nullptr : observation, gy, o.gk, o.gv, o.gq, o.gd, o.gp, o.gr},
-                   {bmean, bcov, gmf, gcf, o.gm0, o.gc0}) &&
+           rot4_ok(d, m, t, a.nb, a.base16, {bmean, bcov, gmf, gcf, o.gm0, o.gc0}) &&
            rot4_tail_ok(fixed, t, chunk, gmf, gcf);
   if (fmt != bssm::kInF32 && (!a.rot4 || (whole && t % 4 != 0)) && n > 0)
     return fail(BSSM_ERR_UNSUPPORTED, "%s: %s inputs need D = 4, M = 8, T a positive %s, checkpoint chunk %d%s and "
@@ -957,11 +942,6 @@ int rotation_common(const char* fn, int d, int m, int64_t n, int64_t t, int64_t 
     return fail(BSSM_ERR_ARGUMENT, "%s: n or t too large", fn);
   return BSSM_OK;
 }
-int rotation_vec(std::initializer_list<const void*> streams, int64_t t, int d) {
-  for (const void* p : streams)
-    if (p != nullptr && !aligned16(p)) return 0;
-  return (t * (d / 2)) % 4 == 0 && t % 4 == 0;
-}
 }  // namespace
 
 int bssm_forward_chunked_rotation(int key_dim, int value_dim, const float* keys, const float* values,
@@ -990,7 +970,7 @@ int bssm_forward_chunked_rotation(int key_dim, int value_dim, const float* keys,
   a.k = keys; a.v = values; a.q = queries; a.rad = radii; a.ang = angles; a.p = process; a.r = observation;
   a.m0 = mean0; a.c0 = cov0; a.y = out; a.mT = mean_final; a.cT = cov_final; a.bm = bmean; a.bc = bcov;
   a.n = n; a.t = t; a.chunk = chunk; a.nb = (t + chunk - 1) / chunk; a.floor = denominator_floor;
-  a.vec = rotation_vec({keys, values, queries, radii, angles, process, observation, out}, t, key_dim);
+  a.base16 = all_aligned16({keys, values, queries, radii, angles, process, observation, out});
   if (n == 0) return ok();
   return launched(fn, bssm::launch_rotation_forward(key_dim, a, static_cast<hipStream_t>(stream)));
 }
@@ -1029,8 +1009,8 @@ int bssm_backward_chunked_rotation(int key_dim, int value_dim, const float* keys
   a.gk = gk; a.gv = gv; a.gq = gq; a.grad = g_radii; a.gang = g_angles; a.gp = g_process; a.gr = g_observation;
   a.gm0 = gm0; a.gc0 = gc0;
   a.n = n; a.t = t; a.chunk = chunk; a.nb = (t + chunk - 1) / chunk; a.floor = denominator_floor;
-  a.vec = rotation_vec({keys, values, queries, radii, angles, process, observation, gy, gk, gv, gq, g_radii,
-                        g_angles, g_process, g_observation}, t, key_dim);
+  a.base16 = all_aligned16({keys, values, queries, radii, angles, process, observation, gy, gk, gv, gq, g_radii,
+                        g_angles, g_process, g_observation});
   if (n == 0) return ok();
   return launched(fn, bssm::launch_rotation_backward(key_dim, a, static_cast<hipStream_t>(stream)));
 }

@@ -31,15 +31,13 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 #ifndef BSSM_NT_STORE_MIN
 #define BSSM_NT_STORE_MIN 128
 #endif
-template <bool NT>
-__device__ __forceinline__ v4f load_stream(const float* p) {
-  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const v4f*>(p));
-  else return *reinterpret_cast<const v4f*>(p);
-}
+// Tile rows start at any 4-byte boundary (T * W need not be a multiple of
+// 4 floats), so 16-byte stores are declared with that alignment.
+typedef float v4f_a4 __attribute__((ext_vector_type(4), aligned(4)));
 template <bool NT>
 __device__ __forceinline__ void store_stream(float* p, v4f v) {
-  if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<v4f*>(p));
-  else *reinterpret_cast<v4f*>(p) = v;
+  if constexpr (NT) __builtin_nontemporal_store(static_cast<v4f_a4>(v), reinterpret_cast<v4f_a4*>(p));
+  else *reinterpret_cast<v4f_a4*>(p) = v;
 }
 
 // ---------------------------------------------------------------- DPP moves
@@ -219,36 +217,44 @@ struct Tile {
 // the global loads and the LDS commit.  Every load of a tile is issued before
 // any of them is consumed, so a tile costs one memory latency, and a tile can
 // be loaded while the previous one is being computed.  Element e (a multiple
-// of 4) of the tile belongs to lane (e / 4) % 64; rows past N and tokens past
-// len read as zero so idle lanes compute on finite data.  Requires every
-// 4-float group to be 16-byte aligned (checked by the caller).
+// of 4) of the tile belongs to lane (e / 4) % 64; rows past N read as zero, so
+// idle lanes compute on finite data.  The loads go through a buffer
+// descriptor that ends at the wave's last row: they need 4-byte alignment
+// only, and a piece that straddles the end of the last row reads zeros past
+// it (the range check is per 32-bit word).  Elsewhere the piece across a
+// tile's end holds the next tokens' (or the next row's) values, which nothing
+// reads.  Typed 16-byte loads needed aligned rows, and the dword-per-lane
+// staging that stood in for them made these kernels several times slower
+// (D = 2 at 8192 x 509, generic forward and backward: 1043 and 1697 us).
 template <int W, int TT, int SPW>
 struct TileRegs {
   using T_ = Tile<W, TT>;
   static constexpr int TOTAL = SPW * T_::PER;
   static constexpr int NV = (TOTAL + 4 * kWave - 1) / (4 * kWave);
   // One wave instruction covers 4 * 64 floats = SEQ_STEP whole sequence rows,
-  // so lane l always holds column o0 of rows s0 + it * SEQ_STEP: one lane
-  // offset, and a wave-uniform base that advances per instruction.
+  // so lane l always holds column o0 of rows s0 + it * SEQ_STEP.
   static constexpr int SEQ_STEP = 4 * kWave / T_::PER;
   static_assert(T_::PER % 4 == 0 && (4 * kWave) % T_::PER == 0, "tile rows must divide a wave instruction");
   v4f r[NV];
 
-  // Rows of one tile are `row` floats apart in global memory (row = T * W).
+  // Rows of one tile are `row` floats apart in global memory (row = T * W;
+  // SPW rows stay below 2^31 bytes, checked by the C ABI).
   __device__ __forceinline__ void load(const float* __restrict__ g, int64_t n0, int64_t n, int64_t t, int64_t t0,
                                        int len, int lane) {
+    constexpr uint32_t kOutside = 0x80000000u;
     const int s0 = (lane * 4) / T_::PER, o0 = (lane * 4) % T_::PER;
-    const int64_t row = t * W;
-    const float* base = g + n0 * row + t0 * W;
-    const uint32_t off = static_cast<uint32_t>(s0) * static_cast<uint32_t>(row) + static_cast<uint32_t>(o0);
+    const int64_t row = t * W, rows = (n - n0) < SPW ? (n - n0) : SPW;
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(g + n0 * row + t0 * W), 0,
+                                                      static_cast<int>((rows * row - t0 * W) * 4), 0x00020000);
+    const uint32_t row4 = static_cast<uint32_t>(row) * 4u;
+    const uint32_t off = static_cast<uint32_t>(s0) * row4 + static_cast<uint32_t>(o0) * 4u;
     const bool col_ok = o0 < len * W;
 #pragma unroll
     for (int it = 0; it < NV; ++it) {
-      const int s = s0 + it * SEQ_STEP;
-      v4f val = {0.f, 0.f, 0.f, 0.f};
-      if (s < SPW && col_ok && n0 + s < n)
-        val = load_stream<(T_::PER * 4 >= BSSM_NT_LOAD_MIN)>(base + static_cast<int64_t>(it * SEQ_STEP) * row + off);
-      r[it] = val;
+      const bool ok = col_ok && s0 + it * SEQ_STEP < SPW;
+      r[it] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
+                                          rs, static_cast<int>(ok ? off + it * SEQ_STEP * row4 : kOutside), 0,
+                                          T_::PER * 4 >= BSSM_NT_LOAD_MIN ? 2 : 0));
     }
   }
 
@@ -263,70 +269,40 @@ struct TileRegs {
   }
 };
 
-// Scalar global -> LDS copy of one tile, for streams whose rows are not
-// 16-byte aligned (T * W not a multiple of 4, or an unaligned base pointer).
-// A compact rolled loop: this is the rarely used fallback, kept small so it
-// does not inflate the register budget of the fast path.
-template <int W, int TT, int SPW>
-__device__ __forceinline__ void stage_in_scalar(float* __restrict__ lds, const float* __restrict__ g, int64_t n0,
-                                                int64_t n, int64_t t, int64_t t0, int len, int lane) {
-  using T_ = Tile<W, TT>;
-  constexpr int TOTAL = SPW * T_::PER;
-  const int valid = len * W;
-#pragma unroll 1
-  for (int e = lane; e < TOTAL; e += kWave) {
-    const int s = e / T_::PER, o = e - s * T_::PER;
-    lds[s * T_::STRIDE + o] = (n0 + s < n && o < valid) ? g[((n0 + s) * t + t0) * W + o] : 0.f;
-  }
-}
-
 // Register-staged copy of one tile (loads, then LDS commit).
 template <int W, int TT, int SPW>
 __device__ __forceinline__ void stage_in(float* __restrict__ lds, const float* __restrict__ g, int64_t n0,
-                                         int64_t n, int64_t t, int64_t t0, int len, bool vec, int lane) {
-  if (vec) {
-    TileRegs<W, TT, SPW> regs;
-    regs.load(g, n0, n, t, t0, len, lane);
-    regs.commit(lds, lane);
-  } else {
-    stage_in_scalar<W, TT, SPW>(lds, g, n0, n, t, t0, len, lane);
-  }
+                                         int64_t n, int64_t t, int64_t t0, int len, int lane) {
+  TileRegs<W, TT, SPW> regs;
+  regs.load(g, n0, n, t, t0, len, lane);
+  regs.commit(lds, lane);
 }
 
 // LDS -> global copy of the first len tokens of a tile.
 template <int W, int TT, int SPW>
 __device__ __forceinline__ void stage_out(const float* __restrict__ lds, float* __restrict__ g, int64_t n0,
-                                          int64_t n, int64_t t, int64_t t0, int len, bool vec, int lane) {
+                                          int64_t n, int64_t t, int64_t t0, int len, int lane) {
   using T_ = Tile<W, TT>;
-  constexpr int TOTAL = SPW * T_::PER;
+  using R = TileRegs<W, TT, SPW>;
   const int valid = len * W;
-  if (vec) {
-    using R = TileRegs<W, TT, SPW>;
-    const int s0 = (lane * 4) / T_::PER, o0 = (lane * 4) % T_::PER;
-    const int64_t row = t * W;
-    float* base = g + n0 * row + t0 * W;
-    const uint32_t off = static_cast<uint32_t>(s0) * static_cast<uint32_t>(row) + static_cast<uint32_t>(o0);
-    const float* src = lds + s0 * T_::STRIDE + o0;
+  const int s0 = (lane * 4) / T_::PER, o0 = (lane * 4) % T_::PER;
+  const int64_t row = t * W;
+  float* base = g + n0 * row + t0 * W;
+  const uint32_t off = static_cast<uint32_t>(s0) * static_cast<uint32_t>(row) + static_cast<uint32_t>(o0);
+  const float* src = lds + s0 * T_::STRIDE + o0;
 #pragma unroll
-    for (int it = 0; it < R::NV; ++it) {
-      const int s = s0 + it * R::SEQ_STEP;
-      if (s < SPW && o0 < valid && n0 + s < n) {
-        float* dst = base + static_cast<int64_t>(it * R::SEQ_STEP) * row + off;
-        const float* lsrc = src + it * R::SEQ_STEP * T_::STRIDE;
-        if (o0 + 4 <= valid) {
-          store_stream<(T_::PER * 4 >= BSSM_NT_STORE_MIN)>(dst, *reinterpret_cast<const v4f*>(lsrc));
-        } else {
-          // The group straddles the end of the tile: the floats past `valid`
-          // belong to the next tile's tokens and must not be overwritten.
-          for (int e = 0; e < valid - o0; ++e) dst[e] = lsrc[e];
-        }
+  for (int it = 0; it < R::NV; ++it) {
+    const int s = s0 + it * R::SEQ_STEP;
+    if (s < SPW && o0 < valid && n0 + s < n) {
+      float* dst = base + static_cast<int64_t>(it * R::SEQ_STEP) * row + off;
+      const float* lsrc = src + it * R::SEQ_STEP * T_::STRIDE;
+      if (o0 + 4 <= valid) {
+        store_stream<(T_::PER * 4 >= BSSM_NT_STORE_MIN)>(dst, *reinterpret_cast<const v4f*>(lsrc));
+      } else {
+        // The group straddles the end of the tile: the floats past `valid`
+        // belong to the next tile's tokens and must not be overwritten.
+        for (int e = 0; e < valid - o0; ++e) dst[e] = lsrc[e];
       }
-    }
-  } else {
-#pragma unroll 1
-    for (int e = lane; e < TOTAL; e += kWave) {
-      const int s = e / T_::PER, o = e - s * T_::PER;
-      if (n0 + s < n && o < valid) g[((n0 + s) * t + t0) * W + o] = lds[s * T_::STRIDE + o];
     }
   }
 }

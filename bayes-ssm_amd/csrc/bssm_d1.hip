@@ -37,6 +37,7 @@ using r4::make_rsrc;
 using r4::Rsrc;
 using r4::st128;
 using r4::st32;
+using r4::store_words;
 using r4::vm_wait;
 
 constexpr int SPW = 8;     // sequences per wave
@@ -199,8 +200,10 @@ __global__ __launch_bounds__(kWave) void forward_kernel(FwdArgs a) {
     else if (b + 1 < nblk) vm_wait<kLoads>();
     else vm_wait<0>();
     const uint32_t t0 = b * FB;
-    const int npc = static_cast<int>(((T - t0) < FB ? (T - t0) : FB) / 4);
-    auto run_piece = [&](int pc, const Piece& x) __attribute__((always_inline)) {
+    const int len = static_cast<int>((T - t0) < FB ? (T - t0) : FB);
+    const int npc = (len + 3) / 4;
+    // The first cnt tokens of piece pc.
+    auto run_piece = [&](int pc, const Piece& x, int cnt) __attribute__((always_inline)) {
       if (t0 + 4u * pc == next_ckpt) {
         st32(rbm, M, bm_off, ckpt * 32u);
         st32(rbc, P, bc_off, ckpt * 4u);
@@ -209,12 +212,13 @@ __global__ __launch_bounds__(kWave) void forward_kernel(FwdArgs a) {
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
+        if (j >= cnt) break;
         Hist h;
         step(P, M, x.k[j], x.d[j], x.p[j], x.r[j], x.v[j], a.floor, h);
         sl[S::V + 64 * (4 * pc + j) + lane] = fmaf(M, x.q[j], 0.f);
       }
     };
-    if (npc == FB / 4) {
+    if (len == FB) {
       // Whole block: unrolled, each piece's LDS reads issued two pieces
       // ahead into a ring of registers.
       constexpr int A = 2;  // pieces read ahead
@@ -224,7 +228,7 @@ __global__ __launch_bounds__(kWave) void forward_kernel(FwdArgs a) {
 #pragma unroll
       for (int pc = 0; pc < FB / 4; ++pc) {
         if (pc + A < FB / 4) read_piece<FB, FIXED>(sl, pc + A, seq, lane, true, true, x[(pc + A) % (A + 1)]);
-        run_piece(pc, x[pc % (A + 1)]);
+        run_piece(pc, x[pc % (A + 1)], 4);
       }
     } else {
       Piece cur;
@@ -232,7 +236,7 @@ __global__ __launch_bounds__(kWave) void forward_kernel(FwdArgs a) {
       for (int pc = 0; pc < npc; ++pc) {
         Piece nxt;
         read_piece<FB, FIXED>(sl, pc + 1 < npc ? pc + 1 : pc, seq, lane, true, true, nxt);
-        run_piece(pc, cur);
+        run_piece(pc, cur, len - 4 * pc);
         cur = nxt;
       }
     }
@@ -360,14 +364,40 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
     const uint32_t t0 = b * BB;
     const uint32_t off = mp.sc(0, t0, T);
     const int e = 4 * lane;
-    st128<kNtSt>(rgk, lds4(sl + S::K + e), off, 0);
-    st128<kNtSt>(rgq, lds4(sl + S::Q + e), off, 0);
     const v4f zero = v4f{0.f, 0.f, 0.f, 0.f};
-    st128<kNtSt>(rgd, DYN ? lds4(sl + S::D + e) : zero, off, 0);
-    st128<kNtSt>(rgp, DYN ? lds4(sl + S::P + e) : zero, off, 0);
-    st128<kNtSt>(rgr, DYN ? lds4(sl + S::R + e) : zero, off, 0);
+    if (T - t0 >= static_cast<uint32_t>(BB)) {
+      st128<kNtSt>(rgk, lds4(sl + S::K + e), off, 0);
+      st128<kNtSt>(rgq, lds4(sl + S::Q + e), off, 0);
+      st128<kNtSt>(rgd, DYN ? lds4(sl + S::D + e) : zero, off, 0);
+      st128<kNtSt>(rgp, DYN ? lds4(sl + S::P + e) : zero, off, 0);
+      st128<kNtSt>(rgr, DYN ? lds4(sl + S::R + e) : zero, off, 0);
+    } else {
+      // The block T ends in: the piece across T leaves word by word.
+      const int words = static_cast<int>(T - t0) - 4 * static_cast<int>(mp.sc_piece);
+      store_words(rgk, lds4(sl + S::K + e), off, words);
+      store_words(rgq, lds4(sl + S::Q + e), off, words);
+      store_words(rgd, DYN ? lds4(sl + S::D + e) : zero, off, words);
+      store_words(rgp, DYN ? lds4(sl + S::P + e) : zero, off, words);
+      store_words(rgr, DYN ? lds4(sl + S::R + e) : zero, off, words);
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) st128<kNtSt>(rgv, lds4(sl + S::V + 256 * i + e), mp.v(i, t0, T), 0);
+  };
+
+  // Tokens len .. BB - 1 of the last block made neutral: k = q = v = gy = 0,
+  // d = 1, p = 0, r = 1.  Their step leaves the belief and their reverse the
+  // carried adjoints as they are, so the chunk T ends in runs whole.  (With
+  // FIXED only while the adjoints are zero; d1_backward_ok sees to it.)
+  auto neutral_tail = [&](float* sl, int len) {
+    for (int t = len; t < BB; ++t) {
+      sl[S::V + 64 * t + lane] = sl[S::GY + 64 * t + lane] = 0.f;
+      if (col == 0) {
+        const int o = 32 * (t >> 2) + 4 * seq + (t & 3);
+        sl[S::K + o] = sl[S::Q + o] = sl[S::P + o] = 0.f;
+        sl[S::D + o] = sl[S::R + o] = 1.f;
+      }
+    }
+    __syncthreads();
   };
 
   // Replay one 16-token chunk (pieces pc0 .. pc0 + 3 of the slot) from its
@@ -430,6 +460,7 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
     __syncthreads();
     if (b + 1 < nblk) store_grads(other, b + 1);
     if (b > 0) issue(other, b - 1);
+    if (i == 0) neutral_tail(cur, static_cast<int>(T - b * BB));
     if ((2u * b + 1u) * kChunk < T) run_chunk(cur, 4, cP1, cM1, false);
     run_chunk(cur, 0, cP0, cM0, b == 0);
   }
@@ -444,13 +475,14 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
 }  // namespace d1
 
 bool d1_forward_ok(const FwdArgs& a) {
-  return a.vec_kqd && a.vec_v && a.vec_pr && a.t % 4 == 0 && a.chunk % 4 == 0 && a.chunk < (int64_t(1) << 30) &&
-         a.t * 256 < (int64_t(1) << 31) && (a.nb + 1) * 256 < (int64_t(1) << 31);
+  return a.base16 && a.chunk % 4 == 0 && a.chunk < (int64_t(1) << 30) && a.t * 256 < (int64_t(1) << 31) &&
+         (a.nb + 1) * 256 < (int64_t(1) << 31);
 }
 
-bool d1_backward_ok(const BwdArgs& a) {
-  return a.vec_kqd && a.vec_v && a.vec_pr && a.t > 0 && a.t % d1::kChunk == 0 && a.chunk == d1::kChunk &&
-         a.t * 256 < (int64_t(1) << 31) && (a.nb + 1) * 256 < (int64_t(1) << 31);
+bool d1_backward_ok(const BwdArgs& a, bool fixed) {
+  const bool tail = a.t % d1::kChunk == 0 || !(fixed && (a.gmf != nullptr || a.gcf != nullptr));
+  return a.base16 && a.t > 0 && tail && a.chunk == d1::kChunk && a.t * 256 < (int64_t(1) << 31) &&
+         (a.nb + 1) * 256 < (int64_t(1) << 31);
 }
 
 hipError_t launch_forward_d1(bool fixed, const FwdArgs& a, hipStream_t stream) {

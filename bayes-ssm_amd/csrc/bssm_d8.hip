@@ -39,6 +39,7 @@ using r4::lds_wait;
 using r4::make_rsrc;
 using r4::Rsrc;
 using r4::st128;
+using r4::store_words;
 using r4::vm_wait;
 
 constexpr int SPW = 8;      // sequences per wave
@@ -206,7 +207,9 @@ __device__ __forceinline__ void reverse_step(const RevTok& in, const Hist& h, co
 }
 
 // ------------------------------------------------------------ backward
-template <bool FIXED, bool DYN>
+// RAG: T is not a multiple of 8 (a template parameter: the tail's tests in
+// the common case's loop cost 1 % of the step at 16384 x 512).
+template <bool FIXED, bool DYN, bool RAG>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1, 1))) void backward_kernel(BwdArgs a) {
   __shared__ float ta[Slot::SIZE], tb[Slot::SIZE];
   const int lane = threadIdx.x;
@@ -295,17 +298,45 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1, 1))) v
   };
   auto store_grads = [&](const float* tl, int64_t c) __attribute__((always_inline)) {
     const int64_t t0 = c * kChunk;
+    const int len = RAG && (T - t0) < kChunk ? static_cast<int>(T - t0) : kChunk;
     const uint32_t s8 = static_cast<uint32_t>(t0) * 32u, s1 = static_cast<uint32_t>(t0) * 4u;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int e = 256 * j + 4 * lane;
-      st128<kNtSt>(rgk, *reinterpret_cast<const v4f*>(&tl[Slot::K + e]), o8[j], s8);
-      st128<kNtSt>(rgq, *reinterpret_cast<const v4f*>(&tl[Slot::Q + e]), o8[j], s8);
-      if (a.gd) st128<kNtSt>(rgd, *reinterpret_cast<const v4f*>(&tl[Slot::D + e]), o8[j], s8);
-      st128<kNtSt>(rgv, *reinterpret_cast<const v4f*>(&tl[Slot::V + e]), o8[j], s8);
+      // Tokens of the chunk below T; the last chunk drops the others' pieces.
+      const uint32_t o = !RAG || 4 * j + (lane >> 4) < len ? o8[j] : kOob;
+      st128<kNtSt>(rgk, *reinterpret_cast<const v4f*>(&tl[Slot::K + e]), o, s8);
+      st128<kNtSt>(rgq, *reinterpret_cast<const v4f*>(&tl[Slot::Q + e]), o, s8);
+      if (a.gd) st128<kNtSt>(rgd, *reinterpret_cast<const v4f*>(&tl[Slot::D + e]), o, s8);
+      st128<kNtSt>(rgv, *reinterpret_cast<const v4f*>(&tl[Slot::V + e]), o, s8);
     }
-    if (a.gp) st128(rgp, *reinterpret_cast<const v4f*>(&tl[Slot::P + 4 * (lane & 15)]), o1, s1);
-    if (a.gr) st128(rgr, *reinterpret_cast<const v4f*>(&tl[Slot::R + 4 * (lane & 15)]), o1, s1);
+    const v4f xp = *reinterpret_cast<const v4f*>(&tl[Slot::P + 4 * (lane & 15)]);
+    const v4f xr = *reinterpret_cast<const v4f*>(&tl[Slot::R + 4 * (lane & 15)]);
+    if (len == kChunk) {
+      if (a.gp) st128(rgp, xp, o1, s1);
+      if (a.gr) st128(rgr, xr, o1, s1);
+    } else {
+      const int words = lane < 16 ? len - 4 * (lane & 1) : 0;
+      if (a.gp) store_words(rgp, xp, o1, words, s1);
+      if (a.gr) store_words(rgr, xr, o1, words, s1);
+    }
+  };
+
+  // Tokens len .. 7 of the last chunk made neutral: k = q = v = gy = 0, d = 1,
+  // p = 0, r = 1.  Their step leaves the belief and their reverse the carried
+  // adjoints as they are, so the chunk runs whole.  (With FIXED only while the
+  // adjoints are zero; d8_backward_ok sees to it.)
+  auto neutral_tail = [&](float* tl, int len) {
+    for (int t = len; t < kChunk; ++t) {
+      const int e = 64 * t + lane;
+      tl[Slot::K + e] = tl[Slot::Q + e] = tl[Slot::V + e] = tl[Slot::GY + e] = 0.f;
+      tl[Slot::D + e] = 1.f;
+      if (g == 0) {
+        tl[Slot::P + 8 * s + t] = 0.f;
+        tl[Slot::R + 8 * s + t] = 1.f;
+      }
+    }
+    lds_wait();
   };
 
   auto read_tok = [&](const float* tl, int tt, Tok& x) __attribute__((always_inline)) {
@@ -381,6 +412,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1, 1))) v
       lds_wait();
       issue(other, c - 1);
     }
+    if (RAG && c + 1 == nb) neutral_tail(cur, static_cast<int>(T - c * kChunk));
     process(cur, c);
   };
   if (nb > 0) issue(ta, nb - 1);
@@ -446,7 +478,7 @@ struct FwdStage {
   v4f k[4], d[4], q[4], v[4], p, r;
 };
 
-template <bool FIXED>
+template <bool FIXED, bool RAG>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void forward_kernel(FwdArgs a) {
   __shared__ float tile[FwdSlot::SIZE];
   const int lane = threadIdx.x;
@@ -552,9 +584,11 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void
       x.v[I] = r4::ld128<kNt>(rv, off, s8);
     }
     if constexpr (!FIXED) {
-      const uint32_t off = (in1 && o1 != kOob) ? o1 : kOob;
-      x.p = r4::ld128<false>(rp, off, s1);
-      x.r = r4::ld128<false>(rr, off, s1);
+      // RAG: the whole offset in the range-checked operand, since the last
+      // row's last piece may end past it.
+      const uint32_t off = (in1 && o1 != kOob) ? (RAG ? o1 + s1 : o1) : kOob;
+      x.p = r4::ld128<false>(rp, off, RAG ? 0u : s1);
+      x.r = r4::ld128<false>(rr, off, RAG ? 0u : s1);
     }
   };
   auto put = [&](const FwdStage& x) __attribute__((always_inline)) {
@@ -618,9 +652,9 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void
     }
     if (ti + 1 < ntiles) load(x, t0 + kFwdTile);
     lds_wait();
-    if (fast) {
-      // Records fall on 8-token boundaries (T is a multiple of 8); each is
-      // staged after the token before it, over the spent first half.
+    if (fast && (!RAG || len % 8 == 0)) {
+      // Records fall on 8-token boundaries; each is staged after the token
+      // before it, over the spent first half.
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) {
         if (hh * 8 >= len) break;
@@ -676,37 +710,48 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void
 
 }  // namespace d8
 
-// D = 8, M = 8 forward: T a positive multiple of 8, any checkpoint chunk,
-// 16-byte aligned streams (the records are stored entry by entry).
+// D = 8, M = 8 forward: T > 0, any checkpoint chunk, 16-byte aligned stream
+// bases.  A last tile that is not a multiple of 8 tokens runs token by token.
 bool d8_forward_ok(const FwdArgs& a) {
-  return a.vec_kqd && a.vec_v && a.vec_pr && a.in_fmt == kInF32 && a.t > 0 && a.t % 8 == 0 &&
-         a.t * 256 < (int64_t(1) << 31) && (a.nb + 1) * 2048 < (int64_t(1) << 31);
+  return a.base16 && a.in_fmt == kInF32 && a.t > 0 && a.t * 256 < (int64_t(1) << 31) &&
+         (a.nb + 1) * 2048 < (int64_t(1) << 31);
 }
 
 hipError_t launch_forward_d8(bool fixed, const FwdArgs& a, hipStream_t stream) {
   const int64_t blocks = (a.n + d8::SPW - 1) / d8::SPW;
   if (blocks == 0) return hipSuccess;
   const dim3 grid(static_cast<unsigned>(blocks)), block(kWave);
-  if (fixed) hipLaunchKernelGGL((d8::forward_kernel<true>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((d8::forward_kernel<false>), grid, block, 0, stream, a);
+  const bool rag = a.t % 8 != 0;
+  if (fixed && rag) hipLaunchKernelGGL((d8::forward_kernel<true, true>), grid, block, 0, stream, a);
+  else if (fixed) hipLaunchKernelGGL((d8::forward_kernel<true, false>), grid, block, 0, stream, a);
+  else if (rag) hipLaunchKernelGGL((d8::forward_kernel<false, true>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((d8::forward_kernel<false, false>), grid, block, 0, stream, a);
   return hipGetLastError();
 }
 
-// D = 8, M = 8 with T a positive multiple of 8, the preferred checkpoint
-// chunk (8), 16-byte aligned streams and 16-byte aligned checkpoint tensors.
-bool d8_backward_ok(const BwdArgs& a) {
+// D = 8, M = 8 with T > 0, the preferred checkpoint chunk (8), 16-byte aligned
+// stream bases and checkpoint tensors.
+bool d8_backward_ok(const BwdArgs& a, bool fixed) {
   const bool rec16 = (reinterpret_cast<uintptr_t>(a.bm) & 15u) == 0 && (reinterpret_cast<uintptr_t>(a.bc) & 15u) == 0;
-  return a.vec_kqd && a.vec_v && a.vec_pr && rec16 && a.t > 0 && a.t % d8::kChunk == 0 && a.chunk == d8::kChunk &&
-         a.t * 256 < (int64_t(1) << 31) && (a.nb + 1) * 2048 < (int64_t(1) << 31);
+  const bool tail = a.t % d8::kChunk == 0 || !(fixed && (a.gmf != nullptr || a.gcf != nullptr));
+  return a.base16 && rec16 && a.t > 0 && tail && a.chunk == d8::kChunk && a.t * 256 < (int64_t(1) << 31) &&
+         (a.nb + 1) * 2048 < (int64_t(1) << 31);
+}
+
+template <bool RAG>
+void launch_backward_d8_rag(bool fixed, bool dyn, const BwdArgs& a, dim3 grid, hipStream_t stream) {
+  const dim3 block(kWave);
+  if (fixed) hipLaunchKernelGGL((d8::backward_kernel<true, false, RAG>), grid, block, 0, stream, a);
+  else if (dyn) hipLaunchKernelGGL((d8::backward_kernel<false, true, RAG>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((d8::backward_kernel<false, false, RAG>), grid, block, 0, stream, a);
 }
 
 hipError_t launch_backward_d8(bool fixed, bool dyn, const BwdArgs& a, hipStream_t stream) {
   const int64_t blocks = (a.n + d8::SPW - 1) / d8::SPW;
   if (blocks == 0) return hipSuccess;
-  const dim3 grid(static_cast<unsigned>(blocks)), block(kWave);
-  if (fixed) hipLaunchKernelGGL((d8::backward_kernel<true, false>), grid, block, 0, stream, a);
-  else if (dyn) hipLaunchKernelGGL((d8::backward_kernel<false, true>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((d8::backward_kernel<false, false>), grid, block, 0, stream, a);
+  const dim3 grid(static_cast<unsigned>(blocks));
+  if (a.t % d8::kChunk != 0) launch_backward_d8_rag<true>(fixed, dyn, a, grid, stream);
+  else launch_backward_d8_rag<false>(fixed, dyn, a, grid, stream);
   return hipGetLastError();
 }
 

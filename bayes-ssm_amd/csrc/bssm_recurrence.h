@@ -27,7 +27,7 @@ struct FwdArgs {
   int64_t chunk;
   int64_t nb;
   float floor;
-  int vec_kqd, vec_v, vec_pr;  // 16-byte staging allowed per stream class
+  int base16;                  // every stream's base is 16-byte aligned
   int rot4;                    // D = 4 rotated-layout kernels allowed (see bssm_rot4.hip)
   int in_fmt;                  // InFmt of k, q, v (not float32: rotated-layout kernels only)
 };
@@ -59,7 +59,7 @@ struct BwdArgs {
   int64_t chunk;
   int64_t nb;
   float floor;
-  int vec_kqd, vec_v, vec_pr;
+  int base16;  // every stream's base is 16-byte aligned
   int rot4;  // D = 4 rotated-layout kernels allowed (see bssm_rot4.hip)
   int in_fmt;  // InFmt of k, q, v and gk, gq, gv (not float32: rotated-layout kernels only)
 };
@@ -100,33 +100,36 @@ hipError_t launch_backward_small(bool fixed, bool dyn, const BwdArgs& a, hipStre
 int64_t small_batch_limit(int direction);
 int64_t set_small_batch_limit(int direction, int64_t limit);
 
-// D = 1, M = 8 kernels with one lane per value column (bssm_d1.hip).  The
-// forward needs 16-byte aligned streams, T and the checkpoint chunk
-// multiples of 4; the backward also needs the checkpoint chunk to be 16 (the
-// library's preferred one for D = 1) and T a positive multiple of 16.
-// Other shapes take the generic kernels.
+// D = 1, M = 8 kernels with one lane per value column (bssm_d1.hip): 16-byte
+// aligned stream bases and every T; the forward needs a checkpoint chunk that
+// is a multiple of 4, the backward the chunk 16 (the library's preferred one
+// for D = 1) and T > 0.  Other shapes take the generic kernels, and so does
+// a backward with fixed dynamics and final-state gradients whose T is not a
+// multiple of the chunk (its last chunk is filled up with neutral tokens,
+// which fixed dynamics allow only while the carried adjoints are zero); the
+// D = 2 and D = 8 backwards below share that rule.
 bool d1_forward_ok(const FwdArgs& a);
-bool d1_backward_ok(const BwdArgs& a);
+bool d1_backward_ok(const BwdArgs& a, bool fixed);
 hipError_t launch_forward_d1(bool fixed, const FwdArgs& a, hipStream_t stream);
 hipError_t launch_backward_d1(bool fixed, bool dyn, const BwdArgs& a, hipStream_t stream);
 
-// D = 2, M = 8 kernels with two value columns per lane (bssm_d2.hip).  Both
-// need 16-byte aligned streams and T a multiple of 4 (the forward takes any
-// checkpoint chunk); the backward needs T > 0 and the checkpoint chunk 8
-// (the library's preferred one for D = 2).
+// D = 2, M = 8 kernels with two value columns per lane (bssm_d2.hip): 16-byte
+// aligned stream bases and every T (the forward takes any checkpoint chunk);
+// the backward needs T > 0 and the checkpoint chunk 8 (the library's
+// preferred one for D = 2).
 bool d2_forward_ok(const FwdArgs& a);
-bool d2_backward_ok(const BwdArgs& a);
+bool d2_backward_ok(const BwdArgs& a, bool fixed);
 hipError_t launch_forward_d2(bool fixed, const FwdArgs& a, hipStream_t stream);
 hipError_t launch_backward_d2(bool fixed, bool dyn, const BwdArgs& a, hipStream_t stream);
 
 // D = 8, M = 8 kernels with 8 lanes per sequence in XOR order (bssm_d8.hip).
-// The forward needs 16-byte aligned float32 streams and T a positive
-// multiple of 8 (any checkpoint chunk); the checkpoint-replay backward also
-// needs the checkpoint chunk 8 (the library's preferred one for D = 8) and
-// 16-byte aligned checkpoint tensors.  Other shapes take the generic kernels.
+// The forward needs 16-byte aligned float32 stream bases and T > 0 (any
+// checkpoint chunk); the checkpoint-replay backward also needs the checkpoint
+// chunk 8 (the library's preferred one for D = 8) and 16-byte aligned
+// checkpoint tensors.  Other shapes take the generic kernels.
 bool d8_forward_ok(const FwdArgs& a);
 hipError_t launch_forward_d8(bool fixed, const FwdArgs& a, hipStream_t stream);
-bool d8_backward_ok(const BwdArgs& a);
+bool d8_backward_ok(const BwdArgs& a, bool fixed);
 hipError_t launch_backward_d8(bool fixed, bool dyn, const BwdArgs& a, hipStream_t stream);
 
 // D = M = 64 kernels (bssm_d64.hip): one wave per sequence, lane = dimension.
@@ -195,8 +198,8 @@ hipError_t launch_mixer_backward(const MixArgs& a, hipStream_t stream);
 
 // Rotation dynamics (bssm_rotation.hip): keys/queries [N, T, D], values,
 // out, gy [N, T, 8], radii/angles/process (per pair) [N, T, D/2],
-// observation [N, T]; belief tensors as the diagonal ABI.  vec: every stream
-// 16-byte aligned with T a multiple of 4.
+// observation [N, T]; belief tensors as the diagonal ABI.  base16: every
+// stream's base is 16-byte aligned.
 struct RotArgs {
   const float *k, *v, *q, *rad, *ang, *p, *r;
   const float *m0, *c0;
@@ -205,13 +208,13 @@ struct RotArgs {
   float *gk, *gv, *gq, *grad, *gang, *gp, *gr, *gm0, *gc0;
   int64_t n, t, chunk, nb;
   float floor;
-  int vec;
+  int base16;
 };
 int rotation_checkpoint(int key_dim);
 hipError_t launch_rotation_forward(int key_dim, const RotArgs& a, hipStream_t stream);
 // Row-per-sequence rotation forward for D = 4, M = 8 (bssm_small.hip): used
-// with 16-byte aligned streams (vec), T a multiple of 4 and 8-byte aligned
-// mean tensors, for n up to small_batch_limit(4).
+// with 16-byte aligned stream bases and 8-byte aligned mean tensors, for n up
+// to small_batch_limit(4).
 hipError_t launch_rotation_forward_small(const RotArgs& a, hipStream_t stream);
 hipError_t launch_rotation_backward(int key_dim, const RotArgs& a, hipStream_t stream);
 

@@ -69,10 +69,7 @@ __global__ __launch_bounds__(kWave) void forward_kernel(FwdArgs a) {
   const float* qs = sq + s * SD;
   float* ys = sv + s * SM;
 
-  // All streams 16-byte aligned for every tile: register-staged loads with
-  // the next tile in flight while this one is computed.  Otherwise scalar
-  // staging per tile.
-  const bool vec = a.vec_kqd && a.vec_v && a.vec_pr;
+  // Register-staged loads with the next tile in flight while this one is computed.
   TileRegs<D, TT, SPW> rk, rq, rd;
   TileRegs<M, TT, SPW> rv;
   TileRegs<1, TT, SPW> rp, rr;
@@ -87,33 +84,22 @@ __global__ __launch_bounds__(kWave) void forward_kernel(FwdArgs a) {
       rr.load(a.r, n0, a.n, T, t0, len, lane);
     }
   };
-  if (vec && T > 0) issue(0);
+  if (T > 0) issue(0);
 
   int64_t next_ckpt = a.chunk;
   int64_t ckpt = 1;
   for (int64_t t0 = 0; t0 < T; t0 += TT) {
     const int len = tile_len(T, t0, TT);
-    if (vec) {
-      rk.commit(sk, lane);
-      rq.commit(sq, lane);
-      rv.commit(sv, lane);
-      if constexpr (!FIXED) {
-        rd.commit(sd, lane);
-        rp.commit(sp, lane);
-        rr.commit(sr, lane);
-      }
-    } else {
-      stage_in_scalar<D, TT, SPW>(sk, a.k, n0, a.n, T, t0, len, lane);
-      stage_in_scalar<D, TT, SPW>(sq, a.q, n0, a.n, T, t0, len, lane);
-      stage_in_scalar<M, TT, SPW>(sv, a.v, n0, a.n, T, t0, len, lane);
-      if constexpr (!FIXED) {
-        stage_in_scalar<D, TT, SPW>(sd, a.d, n0, a.n, T, t0, len, lane);
-        stage_in_scalar<1, TT, SPW>(sp, a.p, n0, a.n, T, t0, len, lane);
-        stage_in_scalar<1, TT, SPW>(sr, a.r, n0, a.n, T, t0, len, lane);
-      }
+    rk.commit(sk, lane);
+    rq.commit(sq, lane);
+    rv.commit(sv, lane);
+    if constexpr (!FIXED) {
+      rd.commit(sd, lane);
+      rp.commit(sp, lane);
+      rr.commit(sr, lane);
     }
     __syncthreads();
-    if (vec && t0 + TT < T) issue(t0 + TT);
+    if (t0 + TT < T) issue(t0 + TT);
     // Software pipeline: the LDS reads of token tt+1 are issued before the
     // update of token tt, so their latency hides behind the arithmetic.
     TokenIn<D, M, G> cur;
@@ -148,7 +134,7 @@ __global__ __launch_bounds__(kWave) void forward_kernel(FwdArgs a) {
       for (int j = 0; j < D; ++j) qc[j] = qn[j];
     }
     __syncthreads();
-    stage_out<M, TT, SPW>(sv, a.y, n0, a.n, T, t0, len, vec, lane);
+    stage_out<M, TT, SPW>(sv, a.y, n0, a.n, T, t0, len, lane);
     __syncthreads();
   }
   if (active) {
@@ -232,7 +218,6 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
   float* grs = sr + s * S1;
 
   const int64_t bm_seq = (a.nb + 1) * D * M, bc_seq = (a.nb + 1) * D * D;
-  const bool vec_all = a.vec_kqd && a.vec_v && a.vec_pr;
 
   // Replay tokens [ts, ts + len) of the staged piece from belief b, keeping
   // the replay history in registers, then run the reverse over them; the
@@ -317,16 +302,16 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
     }
   };
 
-  auto store_grads = [&](int64_t ts, int len, bool vec) {
-    stage_out<D, SUB, SPW>(sk, a.gk, n0, a.n, T, ts, len, vec, lane);
-    stage_out<D, SUB, SPW>(sq, a.gq, n0, a.n, T, ts, len, vec, lane);
-    stage_out<M, SUB, SPW>(sv, a.gv, n0, a.n, T, ts, len, vec, lane);
-    if (a.gd) stage_out<D, SUB, SPW>(sd, a.gd, n0, a.n, T, ts, len, vec, lane);
-    if (a.gp) stage_out<1, SUB, SPW>(sp, a.gp, n0, a.n, T, ts, len, vec, lane);
-    if (a.gr) stage_out<1, SUB, SPW>(sr, a.gr, n0, a.n, T, ts, len, vec, lane);
+  auto store_grads = [&](int64_t ts, int len) {
+    stage_out<D, SUB, SPW>(sk, a.gk, n0, a.n, T, ts, len, lane);
+    stage_out<D, SUB, SPW>(sq, a.gq, n0, a.n, T, ts, len, lane);
+    stage_out<M, SUB, SPW>(sv, a.gv, n0, a.n, T, ts, len, lane);
+    if (a.gd) stage_out<D, SUB, SPW>(sd, a.gd, n0, a.n, T, ts, len, lane);
+    if (a.gp) stage_out<1, SUB, SPW>(sp, a.gp, n0, a.n, T, ts, len, lane);
+    if (a.gr) stage_out<1, SUB, SPW>(sr, a.gr, n0, a.n, T, ts, len, lane);
   };
 
-  if (vec_all && a.chunk <= SUB && a.chunk % 4 == 0) {
+  if (a.chunk <= SUB) {
     // Hot path: one replay piece per checkpoint chunk.  The inputs and the
     // checkpoint belief of chunk c-1 are loaded into registers while chunk c
     // is replayed and reversed.
@@ -366,7 +351,7 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
       if (c > 0) issue(c - 1);
       run_piece(b, ts, len);
       __syncthreads();
-      store_grads(ts, len, true);
+      store_grads(ts, len);
       __syncthreads();
     }
   } else {
@@ -381,13 +366,12 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
         load_belief<D, M, G>(b, a.bm + na * bm_seq + c * D * M, a.bc + na * bc_seq + c * D * D, g, active);
         for (int j = 0; j < sc; ++j) {
           const int64_t ts = tc0 + static_cast<int64_t>(j) * SUB;
-          const bool vec = vec_all && (ts % 4 == 0);
-          stage_in<D, SUB, SPW>(sk, a.k, n0, a.n, T, ts, SUB, vec, lane);
-          stage_in<M, SUB, SPW>(sv, a.v, n0, a.n, T, ts, SUB, vec, lane);
+          stage_in<D, SUB, SPW>(sk, a.k, n0, a.n, T, ts, SUB, lane);
+          stage_in<M, SUB, SPW>(sv, a.v, n0, a.n, T, ts, SUB, lane);
           if constexpr (!FIXED) {
-            stage_in<D, SUB, SPW>(sd, a.d, n0, a.n, T, ts, SUB, vec, lane);
-            stage_in<1, SUB, SPW>(sp, a.p, n0, a.n, T, ts, SUB, vec, lane);
-            stage_in<1, SUB, SPW>(sr, a.r, n0, a.n, T, ts, SUB, vec, lane);
+            stage_in<D, SUB, SPW>(sd, a.d, n0, a.n, T, ts, SUB, lane);
+            stage_in<1, SUB, SPW>(sp, a.p, n0, a.n, T, ts, SUB, lane);
+            stage_in<1, SUB, SPW>(sr, a.r, n0, a.n, T, ts, SUB, lane);
           }
           __syncthreads();
 #pragma unroll 1
@@ -401,20 +385,19 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
         }
         const int64_t ts = tc0 + static_cast<int64_t>(sc) * SUB;
         const int len = static_cast<int>((lc - sc * SUB) < SUB ? (lc - sc * SUB) : SUB);
-        const bool vec = vec_all && (ts % 4 == 0);
-        stage_in<D, SUB, SPW>(sk, a.k, n0, a.n, T, ts, len, vec, lane);
-        stage_in<D, SUB, SPW>(sq, a.q, n0, a.n, T, ts, len, vec, lane);
-        stage_in<M, SUB, SPW>(sv, a.v, n0, a.n, T, ts, len, vec, lane);
-        stage_in<M, SUB, SPW>(sg, a.gy, n0, a.n, T, ts, len, vec, lane);
+        stage_in<D, SUB, SPW>(sk, a.k, n0, a.n, T, ts, len, lane);
+        stage_in<D, SUB, SPW>(sq, a.q, n0, a.n, T, ts, len, lane);
+        stage_in<M, SUB, SPW>(sv, a.v, n0, a.n, T, ts, len, lane);
+        stage_in<M, SUB, SPW>(sg, a.gy, n0, a.n, T, ts, len, lane);
         if constexpr (!FIXED) {
-          stage_in<D, SUB, SPW>(sd, a.d, n0, a.n, T, ts, len, vec, lane);
-          stage_in<1, SUB, SPW>(sp, a.p, n0, a.n, T, ts, len, vec, lane);
-          stage_in<1, SUB, SPW>(sr, a.r, n0, a.n, T, ts, len, vec, lane);
+          stage_in<D, SUB, SPW>(sd, a.d, n0, a.n, T, ts, len, lane);
+          stage_in<1, SUB, SPW>(sp, a.p, n0, a.n, T, ts, len, lane);
+          stage_in<1, SUB, SPW>(sr, a.r, n0, a.n, T, ts, len, lane);
         }
         __syncthreads();
         run_piece(b, ts, len);
         __syncthreads();
-        store_grads(ts, len, vec);
+        store_grads(ts, len);
         __syncthreads();
       }
     }
@@ -529,9 +512,9 @@ hipError_t launch_backward(int key_dim, bool fixed, bool dyn, const BwdArgs& a, 
   if (key_dim == 4 && a.rot4 && a.n <= row_limit && row_tail && a.chunk == kRot4Chunk)
     return launch_backward_small(fixed, dyn, a, stream);
   if (key_dim == 4 && a.rot4) return launch_backward_r4(fixed, dyn, a, stream);
-  if (key_dim == 1 && d1_backward_ok(a)) return launch_backward_d1(fixed, dyn, a, stream);
-  if (key_dim == 2 && d2_backward_ok(a)) return launch_backward_d2(fixed, dyn, a, stream);
-  if (key_dim == 8 && d8_backward_ok(a)) return launch_backward_d8(fixed, dyn, a, stream);
+  if (key_dim == 1 && d1_backward_ok(a, fixed)) return launch_backward_d1(fixed, dyn, a, stream);
+  if (key_dim == 2 && d2_backward_ok(a, fixed)) return launch_backward_d2(fixed, dyn, a, stream);
+  if (key_dim == 8 && d8_backward_ok(a, fixed)) return launch_backward_d8(fixed, dyn, a, stream);
   switch (key_dim) {
     case 1: return launch_backward_dd<1>(fixed, dyn, a, stream);
     case 2: return launch_backward_dd<2>(fixed, dyn, a, stream);

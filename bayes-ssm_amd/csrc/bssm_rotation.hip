@@ -505,9 +505,7 @@ __global__ __launch_bounds__(kWave) void forward_kernel(RotArgs a) {
              ssi + s * SJ};
   const float* qs = sq + s * SD;
   float* ys = sv + s * SM;
-  // With every stream 16-byte aligned the next tile is loaded into
-  // registers while this one is computed; otherwise tiles are staged
-  // synchronously.
+  // The next tile is loaded into registers while this one is computed.
   TileRegs<D, TT, SPW> rk, rq;
   TileRegs<M, TT, SPW> rv;
   TileRegs<J, TT, SPW> rrad, rang, rp;
@@ -522,7 +520,7 @@ __global__ __launch_bounds__(kWave) void forward_kernel(RotArgs a) {
     rp.load(a.p, n0, a.n, T, t0, len, lane);
     rr.load(a.r, n0, a.n, T, t0, len, lane);
   };
-  if (a.vec && T > 0) issue(0);
+  if (T > 0) issue(0);
   int64_t next_ckpt = a.chunk, ckpt = 1;
   // Eight tokens of a staged tile, unrolled: each token's LDS reads are
   // issued before the previous token is computed (the scheduling barriers
@@ -561,27 +559,17 @@ __global__ __launch_bounds__(kWave) void forward_kernel(RotArgs a) {
   };
   for (int64_t t0 = 0; t0 < T; t0 += TT) {
     const int len = tile_len(T, t0, TT);
-    if (a.vec) {
-      rk.commit(sk, lane);
-      rq.commit(sq, lane);
-      rv.commit(sv, lane);
-      rrad.commit(srad, lane);
-      rang.commit(sang, lane);
-      rp.commit(sp, lane);
-      rr.commit(sr, lane);
-    } else {
-      stage_in<D, TT, SPW>(sk, a.k, n0, a.n, T, t0, len, false, lane);
-      stage_in<D, TT, SPW>(sq, a.q, n0, a.n, T, t0, len, false, lane);
-      stage_in<M, TT, SPW>(sv, a.v, n0, a.n, T, t0, len, false, lane);
-      stage_in<J, TT, SPW>(srad, a.rad, n0, a.n, T, t0, len, false, lane);
-      stage_in<J, TT, SPW>(sang, a.ang, n0, a.n, T, t0, len, false, lane);
-      stage_in<J, TT, SPW>(sp, a.p, n0, a.n, T, t0, len, false, lane);
-      stage_in<1, TT, SPW>(sr, a.r, n0, a.n, T, t0, len, false, lane);
-    }
+    rk.commit(sk, lane);
+    rq.commit(sq, lane);
+    rv.commit(sv, lane);
+    rrad.commit(srad, lane);
+    rang.commit(sang, lane);
+    rp.commit(sp, lane);
+    rr.commit(sr, lane);
     __syncthreads();
     fill_trig<SPW, J, TT>(sang, ssi, lane);
     __syncthreads();
-    if (a.vec && t0 + TT < T) issue(t0 + TT);
+    if (t0 + TT < T) issue(t0 + TT);
     if (len == TT && TT % 8 == 0 && a.chunk % 8 == 0) {
       // Whole tile, checkpoints on 8-token boundaries only.
 #pragma unroll
@@ -608,7 +596,7 @@ __global__ __launch_bounds__(kWave) void forward_kernel(RotArgs a) {
       }
     }
     __syncthreads();
-    stage_out<M, TT, SPW>(sv, a.y, n0, a.n, T, t0, len, a.vec, lane);
+    stage_out<M, TT, SPW>(sv, a.y, n0, a.n, T, t0, len, lane);
     __syncthreads();
   }
   if (active) {
@@ -720,16 +708,15 @@ __global__ __launch_bounds__(kWave) void backward_kernel(RotArgs a) {
   const int64_t bm_seq = (a.nb + 1) * D * M, bc_seq = (a.nb + 1) * D * D;
 
   auto stage_piece = [&](int64_t ts, int len, bool with_grad) {
-    const bool vec = a.vec && (ts % 4 == 0);
-    stage_in<D, SUB, SPW>(sk, a.k, n0, a.n, T, ts, len, vec, lane);
-    stage_in<M, SUB, SPW>(sv, a.v, n0, a.n, T, ts, len, vec, lane);
-    stage_in<J, SUB, SPW>(srad, a.rad, n0, a.n, T, ts, len, vec, lane);
-    stage_in<J, SUB, SPW>(sang, a.ang, n0, a.n, T, ts, len, vec, lane);
-    stage_in<J, SUB, SPW>(sp, a.p, n0, a.n, T, ts, len, vec, lane);
-    stage_in<1, SUB, SPW>(sr, a.r, n0, a.n, T, ts, len, vec, lane);
+    stage_in<D, SUB, SPW>(sk, a.k, n0, a.n, T, ts, len, lane);
+    stage_in<M, SUB, SPW>(sv, a.v, n0, a.n, T, ts, len, lane);
+    stage_in<J, SUB, SPW>(srad, a.rad, n0, a.n, T, ts, len, lane);
+    stage_in<J, SUB, SPW>(sang, a.ang, n0, a.n, T, ts, len, lane);
+    stage_in<J, SUB, SPW>(sp, a.p, n0, a.n, T, ts, len, lane);
+    stage_in<1, SUB, SPW>(sr, a.r, n0, a.n, T, ts, len, lane);
     if (with_grad) {
-      stage_in<D, SUB, SPW>(sq, a.q, n0, a.n, T, ts, len, vec, lane);
-      stage_in<M, SUB, SPW>(sg, a.gy, n0, a.n, T, ts, len, vec, lane);
+      stage_in<D, SUB, SPW>(sq, a.q, n0, a.n, T, ts, len, lane);
+      stage_in<M, SUB, SPW>(sg, a.gy, n0, a.n, T, ts, len, lane);
     }
   };
 
@@ -838,23 +825,22 @@ __global__ __launch_bounds__(kWave) void backward_kernel(RotArgs a) {
     }
   };
   auto store_piece = [&](int64_t ts, int len) __attribute__((always_inline)) {
-    const bool vec = a.vec && (ts % 4 == 0);
-    stage_out<D, SUB, SPW>(sk, a.gk, n0, a.n, T, ts, len, vec, lane);
-    stage_out<D, SUB, SPW>(sq, a.gq, n0, a.n, T, ts, len, vec, lane);
-    stage_out<M, SUB, SPW>(sv, a.gv, n0, a.n, T, ts, len, vec, lane);
-    stage_out<J, SUB, SPW>(srad, a.grad, n0, a.n, T, ts, len, vec, lane);
-    stage_out<J, SUB, SPW>(sang, a.gang, n0, a.n, T, ts, len, vec, lane);
-    stage_out<J, SUB, SPW>(sp, a.gp, n0, a.n, T, ts, len, vec, lane);
-    stage_out<1, SUB, SPW>(sr, a.gr, n0, a.n, T, ts, len, vec, lane);
+    stage_out<D, SUB, SPW>(sk, a.gk, n0, a.n, T, ts, len, lane);
+    stage_out<D, SUB, SPW>(sq, a.gq, n0, a.n, T, ts, len, lane);
+    stage_out<M, SUB, SPW>(sv, a.gv, n0, a.n, T, ts, len, lane);
+    stage_out<J, SUB, SPW>(srad, a.grad, n0, a.n, T, ts, len, lane);
+    stage_out<J, SUB, SPW>(sang, a.gang, n0, a.n, T, ts, len, lane);
+    stage_out<J, SUB, SPW>(sp, a.gp, n0, a.n, T, ts, len, lane);
+    stage_out<1, SUB, SPW>(sr, a.gr, n0, a.n, T, ts, len, lane);
   };
 
-  // Hot path (aligned streams, one replay piece per checkpoint chunk): the
+  // Hot path (aligned stream bases, one replay piece per checkpoint chunk): the
   // next chunk (inputs and checkpoint records) lands in the staging area by
   // LDS-DMA while this one is computed; at a chunk's start the previous
   // chunk's gradients leave the tiles, then the staged rows are copied into
   // them.  Staging each chunk synchronously instead left the backward
   // waiting on memory for about a third of its time.
-  const bool dma = a.vec && a.chunk == SUB && a.nb > 0 && T * 4 * M * SPW < (int64_t(1) << 31) &&
+  const bool dma = a.base16 && a.chunk == SUB && a.nb > 0 && T * 4 * M * SPW < (int64_t(1) << 31) &&
                    (a.nb + 1) * 4 * D * M * SPW < (int64_t(1) << 31);
   if (dma) {
     const uint32_t Tu = static_cast<uint32_t>(T);
@@ -1020,7 +1006,7 @@ int rotation_checkpoint(int key_dim) {
 hipError_t launch_rotation_forward(int key_dim, const RotArgs& a, hipStream_t stream) {
   if (a.n == 0) return hipSuccess;
   auto al8 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; };
-  if (key_dim == 4 && a.vec && a.t % 4 == 0 && a.n <= small_batch_limit(4) && al8(a.m0) && al8(a.mT) && al8(a.bm))
+  if (key_dim == 4 && a.base16 && a.t > 0 && a.n <= small_batch_limit(4) && al8(a.m0) && al8(a.mT) && al8(a.bm))
     return launch_rotation_forward_small(a, stream);
   switch (key_dim) {
     case 2: return rot::fwd<2>(a, stream);

@@ -9,8 +9,6 @@ compared, so a store past a row's end shows in its neighbour.
 """
 from __future__ import annotations
 
-import contextlib
-
 import pytest
 import torch
 
@@ -23,7 +21,7 @@ pytestmark = pytest.mark.gpu
 
 # One token; around the 4-token pieces, the 8-token chunks and the 16-token tiles.
 TIMES = [1, 3, 6, 7, 9, 13, 15, 17, 23, 30, 33, 51]
-CHUNK = {4: 8}
+CHUNK = {1: 16, 2: 8, 4: 8, 8: 8}
 
 
 def _ext(d):
@@ -97,3 +95,53 @@ def test_d4_narrow_is_the_float32_kernel_on_the_widened_values(cuda_device, name
         assert torch.equal(a, b)
     for i, (a, b) in enumerate(zip(grads, egrads)):
         assert torch.equal(a.float(), b.to(a.dtype).float()), i
+
+
+@pytest.mark.parametrize("t", TIMES + [63, 65, 97])
+@pytest.mark.parametrize("final_grads", [False, True])
+@pytest.mark.parametrize("abi", ABIS, ids=[a[0] for a in ABIS])
+@pytest.mark.parametrize("d", [1, 2, 8])
+def test_other_dims_match_oracle(cuda_device, d, abi, final_grads, t):
+    """The dedicated kernels; fixed dynamics with final-state gradients take the generic backward."""
+    print(f"ragged D{d} {abi[0]} final_grads={final_grads} t={t}", flush=True)
+    cpu, dev = _case(21, t, d, seed=970 + t + d, device=cuda_device)
+    outs, grads = _run(d, dev, abi, final_grads)
+    _check(cpu, outs, grads, abi, CHUNK[d], final_grads)
+
+
+@pytest.mark.parametrize("t", [1, 7, 18, 33])
+@pytest.mark.parametrize("chunk", [1, 3, 5, 64])
+@pytest.mark.parametrize("d", [1, 2, 4, 8])
+def test_generic_kernels_match_oracle(cuda_device, monkeypatch, d, chunk, t):
+    """Checkpoint chunks the dedicated backwards do not take, on streams that start 4 bytes off a 16-byte boundary."""
+    print(f"ragged generic D{d} chunk={chunk} t={t}", flush=True)
+    cpu, dev = _case(21, t, d, seed=990 + t + d, device=cuda_device)
+    for x in ("k", "v", "q", "d", "p", "r", "gy"):
+        buf = torch.full((dev[x].numel() + 9,), float("nan"), device=cuda_device)
+        buf[1:1 + dev[x].numel()] = dev[x].flatten()
+        dev[x] = buf[1:1 + dev[x].numel()].view(dev[x].shape)
+    monkeypatch.setitem(CHUNK, d, chunk)
+    abi = ("backward_chunked", False, 8)
+    outs, grads = _run(d, dev, abi, True)
+    _check(cpu, outs, grads, abi, chunk, True)
+
+
+@pytest.mark.parametrize("t", [1, 3, 7, 9, 17, 30, 33])
+@pytest.mark.parametrize("d", [2, 4, 8])
+@pytest.mark.parametrize("name", ["row", "quad"])
+def test_rotation_matches_oracle(cuda_device, name, d, t):
+    from bayes_ssm import _hip
+    from tests.test_gpu_rotation import _case as rotation_case
+    from tests.test_gpu_rotation import _run as run_rotation
+
+    print(f"ragged rotation {name} D{d} t={t}", flush=True)
+    ins, gy, gmf, gcf = rotation_case(21, t, d, seed=40 * d + t)
+    with layout(name):
+        y, mT, cT, _, _, grads = run_rotation(ins, gy, gmf, gcf, _hip.load().bssm_rotation_checkpoint(d), cuda_device)
+    leaves = [x.double().requires_grad_(True) for x in ins]
+    ey, em, ec = O.run_rotation(*leaves, 1e-6)
+    loss = (ey * gy.double()).sum() + (em * gmf.double()).sum() + (ec * gcf.double()).sum()
+    for got, want, what in zip((y, mT, cT, *grads), (ey, em, ec, *torch.autograd.grad(loss, leaves)),
+                               ("y", "mean_T", "cov_T", "gk", "gv", "gq", "g_radii", "g_angles", "g_process",
+                                "g_observation", "gm0", "gc0")):
+        close(got, want, what)

@@ -53,6 +53,8 @@ _SIGNATURES = {
     "bssm_forward_chunked_narrow": [_I, _I, _I, _I] + [_P] * 8 + [_P] * 5 + [_L, _L, _L, _F, _P],
     "bssm_backward_chunked_narrow": [_I, _I, _I, _I] + [_P] * 10 + [_P] * 3 + [_P] * 8 + [_L, _L, _L, _F, _P],
     "bssm_round_float8": [_I, _P, _P, _L],
+    "bssm_bf16_large_blocks": [],
+    "bssm_bf16_large": [_I, _P, _P, _P, _P, _P, _P],
     "bssm_value_stats_workspace": [_I, _P],
     "bssm_value_stats": [_I, _P, _P, _P, _P, _L, _P, _P],
     "bssm_associative_static_scan": [_P] * 9 + [_L, _L, _I, _I, _P],
@@ -76,6 +78,7 @@ _SIGNATURES = {
     "bssm_abi_version": [],
 }
 ABI_VERSION = 10
+ANY_SHAPE = 1 << 32  # or-ed into the mixer entry points' chunk (BSSM_ANY_SHAPE)
 
 _lock = threading.Lock()
 _lib: Optional[ctypes.CDLL] = None

@@ -21,12 +21,21 @@ chip (C ABI ``bssm_mixer_forward`` / ``bssm_mixer_backward``).  Projection
 gradients come back as bfloat16, the float32 gradient rounded to nearest even,
 which is what autograd through the reference's ``.float()`` widening yields.
 
-Shapes the kernels do not take (heads not a multiple of 16, T not a multiple
-of 4, other dtypes or devices, strided rows the kernels cannot address) run the
-reference's op chain through ``bayesian_layer`` instead.
+Heads a multiple of 16 with T a multiple of 4 ("whole tiles") always run the
+kernels.  Heads a multiple of 4 with any T run them when the call is one that
+the op chain would take without complaint (see ``_any_shape_call``): the op
+chain validates the layer's inputs, so the projections are scanned on the
+device first, and a call with a non-finite (or enormous) value is left to the
+op chain, which raises or computes as it always has.  Other shapes (and other
+dtypes or devices, or strided rows the kernels cannot address) run the
+reference's op chain through ``bayesian_layer``.
 """
 from __future__ import annotations
 
+import ctypes
+import math
+import os
+from numbers import Real
 from typing import Optional
 
 import torch
@@ -34,7 +43,7 @@ import torch.nn.functional as F
 from torch import Tensor
 
 from . import _hip
-from .bayesian_layer import bayesian_layer
+from .bayesian_layer import _replay_enabled, _skip_host_checks, bayesian_layer
 
 KEY_DIM = 4
 VALUE_DIM = 8
@@ -63,12 +72,67 @@ def _row_stride(x: Tensor, t: int) -> Optional[int]:
     return ld
 
 
-def _fused_eligible(projections: tuple[Tensor, ...], heads: int) -> Optional[tuple[int, ...]]:
+def _whole_tiles(heads: int, t: int) -> bool:
+    return heads % 16 == 0 and t % 4 == 0
+
+
+def _chunk_arg(heads: int, t: int) -> int:
+    """The checkpoint interval as the C entry points take it (with BSSM_ANY_SHAPE off whole tiles)."""
+    interval = _hip.preferred_checkpoint(KEY_DIM)
+    return interval if _whole_tiles(heads, t) else interval | _hip.ANY_SHAPE
+
+
+def _any_shape_call(heads: int, t: int, initial_mean: Optional[Tensor], initial_covariance: Optional[Tensor],
+                    chunk_length: Optional[int], denominator_floor: float, optimized: bool) -> bool:
+    """Off whole tiles the kernels take calls that the op chain's own argument checks would pass (the values aside):
+    the default prior, a valid chunk length and floor, the optimized core, no switch that selects another core."""
+    return (heads > 0 and heads % 4 == 0 and t > 0 and optimized and initial_mean is None
+            and initial_covariance is None and isinstance(denominator_floor, Real) and math.isfinite(denominator_floor)
+            and (chunk_length is None or (isinstance(chunk_length, int) and not isinstance(chunk_length, bool)
+                                          and chunk_length > 0))
+            and os.environ.get("BAYES_SSM_DISABLE_FUSED_CUDA", "0") != "1"
+            and not (torch.is_grad_enabled() and _replay_enabled()))
+
+
+class _LargeScan:
+    """Device scan of bfloat16 row views [B, T, W] (rows ``stride(1)`` apart) for NaN, infinities and magnitudes of
+    2^63 or more (C ABI ``bssm_bf16_large``), started on construction and read back by ``clean``: the wait is for
+    the scan alone, so kernels queued in between run on.  Within the bound no transform of the mixer overflows."""
+
+    def __init__(self, views: tuple[Tensor, ...]) -> None:
+        self._event: Optional[torch.cuda.Event] = None
+        if _skip_host_checks(views[0]):
+            return
+        n = len(views)
+        as_ptr = lambda arr: ctypes.cast(arr, ctypes.c_void_p)  # noqa: E731
+        ptrs = (ctypes.c_void_p * n)(*[x.data_ptr() for x in views])
+        lds = (ctypes.c_int64 * n)(*[x.stride(1) for x in views])
+        cols = (ctypes.c_int64 * n)(*[x.shape[2] for x in views])
+        rows = (ctypes.c_int64 * n)(*[x.shape[0] * x.shape[1] for x in views])
+        dev = views[0].device
+        flags = torch.empty(_hip.function("bssm_bf16_large_blocks")(), device=dev, dtype=torch.int32)
+        self._flags = torch.empty(flags.shape, dtype=torch.int32, pin_memory=True)
+        with _hip.on_device(dev):
+            _hip.call("bssm_bf16_large", n, as_ptr(ptrs), as_ptr(lds), as_ptr(cols), as_ptr(rows), flags.data_ptr(),
+                      _hip.stream_of(dev))
+            self._flags.copy_(flags, non_blocking=True)
+            self._event = torch.cuda.Event()
+            self._event.record()
+
+    def clean(self) -> bool:
+        if self._event is None:
+            return True
+        self._event.synchronize()
+        return not self._flags.any()
+
+
+def _fused_eligible(projections: tuple[Tensor, ...], heads: int, whole: bool = True) -> Optional[tuple[int, ...]]:
+    """Row strides of projections the kernels can address (with ``whole``: in whole tiles), else None."""
     q = projections[0]
     if q.device.type != "cuda" or q.ndim != 3:
         return None
     b, t, _ = q.shape
-    if heads % 16 != 0 or t <= 0 or t % 4 != 0:
+    if t <= 0 or (not _whole_tiles(heads, t) if whole else heads % 4 != 0):
         return None
     lds = []
     for x, w in zip(projections, _WIDTHS):
@@ -101,12 +165,12 @@ class _MixerCoreFunction(torch.autograd.Function):
         with _hip.on_device(dev):
             _hip.call("bssm_mixer_forward", P(q_proj), lds[0], P(k_proj), lds[1], P(v_proj), lds[2],
                       P(decay_logits), lds[3], P(noise), lds[4], P(initial_mean), P(initial_covariance), P(read),
-                      P(mean_t), P(cov_t), P(bmean), P(bcov), b, t, heads, interval, float(denominator_floor),
+                      P(mean_t), P(cov_t), P(bmean), P(bcov), b, t, heads, _chunk_arg(heads, t),
+                      float(denominator_floor),
                       _hip.stream_of(dev))
         ctx.save_for_backward(q_proj, k_proj, v_proj, decay_logits, noise, initial_mean, initial_covariance,
                               bmean, bcov)
         ctx.heads = heads
-        ctx.interval = interval
         ctx.lds = lds
         ctx.denominator_floor = float(denominator_floor)
         ctx.set_materialize_grads(False)
@@ -140,7 +204,7 @@ class _MixerCoreFunction(torch.autograd.Function):
             _hip.call("bssm_mixer_backward", P(q_proj), lds[0], P(k_proj), lds[1], P(v_proj), lds[2],
                       P(decay_logits), lds[3], P(noise), lds[4], P(mean0), P(cov0), P(bmean), P(bcov),
                       P(grad_read), P(gm), P(gc), P(gq), P(gk), P(gv), P(gdl), P(gnz), P(gm0), P(gc0), b, t, heads,
-                      ctx.interval, ctx.denominator_floor, 0, _hip.stream_of(dev))
+                      _chunk_arg(heads, t), ctx.denominator_floor, 0, _hip.stream_of(dev))
         return (gq if need[0] else None, gk if need[1] else None, gv if need[2] else None,
                 gdl if need[3] else None, gnz if need[4] else None, gm0, gc0, None, None, None)
 
@@ -224,8 +288,8 @@ def bayes_mixer_core(
     (float32; the reference's permuted view, made contiguous) and the final
     mean [B*H, 4, 8] and covariance [B*H, 4, 4].
 
-    Eligible inputs (CUDA, bfloat16, H % 16 == 0, T % 4 == 0, rows
-    addressable as described in the module docstring) run the fused kernels;
+    Eligible inputs (CUDA, bfloat16, shapes and calls as described in the
+    module docstring, addressable rows) run the fused kernels;
     others run the reference op chain and ``bayesian_layer`` with
     ``chunk_length`` (which the fused kernels do not need: the recurrence is
     exact for every chunk length) and ``optimized``, the mixer's own switch
@@ -242,12 +306,17 @@ def bayes_mixer_core(
     for x, w, name in zip(projections, _WIDTHS, ("q_proj", "k_proj", "v_proj", "decay_logits", "noise")):
         if tuple(x.shape) != (b, t, w * heads):
             raise ValueError(f"{name} must have shape [B, T, H*{w}] = {(b, t, w * heads)}, got {tuple(x.shape)}")
-    lds = _fused_eligible(projections, heads)
-    if lds is not None:
+    lds = _fused_eligible(projections, heads, whole=False)
+    whole = _whole_tiles(heads, t)
+    if lds is not None and (whole or _any_shape_call(heads, t, initial_mean, initial_covariance, chunk_length,
+                                                     denominator_floor, optimized)):
         _hip.load()  # on a GPU the fused path never degrades silently
+        scan = None if whole else _LargeScan(projections)
         mean0, cov0 = _initial_state(initial_mean, initial_covariance, b * heads, q_proj.device)
-        return _MixerCoreFunction.apply(q_proj, k_proj, v_proj, decay_logits, noise, mean0, cov0, int(heads),
+        outs = _MixerCoreFunction.apply(q_proj, k_proj, v_proj, decay_logits, noise, mean0, cov0, int(heads),
                                         float(denominator_floor), lds)
+        if scan is None or scan.clean():
+            return outs
     k, v, q, decay, process, observation = mixer_layer_inputs(*projections, heads)
     read, mean_t, cov_t = bayesian_layer(
         k, v, q, transition_diagonals=decay, process_variances=process, observation_variances=observation,
@@ -280,11 +349,10 @@ class _MixerReadoutFunction(torch.autograd.Function):
             _hip.call("bssm_mixer_gated_forward", P(q_proj), lds[0], P(k_proj), lds[1], P(v_proj), lds[2],
                       P(decay_logits), lds[3], P(noise), lds[4], P(gate), lds[5], P(w32), float(norm_eps),
                       P(initial_mean), P(initial_covariance), P(out), P(read_bf16), P(mean_t), P(cov_t), P(bmean),
-                      P(bcov), b, t, heads, interval, float(denominator_floor), 0, _hip.stream_of(dev))
+                      P(bcov), b, t, heads, _chunk_arg(heads, t), float(denominator_floor), 0, _hip.stream_of(dev))
         ctx.save_for_backward(q_proj, k_proj, v_proj, decay_logits, noise, gate, w32, initial_mean,
                               initial_covariance, bmean, bcov, read_bf16)
         ctx.heads = heads
-        ctx.interval = interval
         ctx.lds = lds
         ctx.norm_eps = float(norm_eps)
         ctx.weight_dtype = norm_weight.dtype
@@ -315,7 +383,7 @@ class _MixerReadoutFunction(torch.autograd.Function):
         gdl = empty(decay_logits) if dyn else None
         gnz = empty(noise) if dyn else None
         ggate = empty(gate)
-        partials = torch.empty(b * heads // 16, VALUE_DIM, device=dev, dtype=torch.float32)
+        partials = torch.empty(b * (-(-heads // 16)), VALUE_DIM, device=dev, dtype=torch.float32)
         gm0 = torch.empty_like(mean0) if need[7] else None
         gc0 = torch.empty_like(cov0) if need[8] else None
         P = _hip.ptr
@@ -323,7 +391,7 @@ class _MixerReadoutFunction(torch.autograd.Function):
             _hip.call("bssm_mixer_gated_backward", P(q_proj), lds[0], P(k_proj), lds[1], P(v_proj), lds[2],
                       P(decay_logits), lds[3], P(noise), lds[4], P(gate), lds[5], P(w32), ctx.norm_eps, P(mean0),
                       P(cov0), P(bmean), P(bcov), P(read_bf16), P(grad_out), P(gm), P(gc), P(gq), P(gk), P(gv),
-                      P(gdl), P(gnz), P(ggate), P(partials), P(gm0), P(gc0), b, t, heads, ctx.interval,
+                      P(gdl), P(gnz), P(ggate), P(partials), P(gm0), P(gc0), b, t, heads, _chunk_arg(heads, t),
                       ctx.denominator_floor, 0, _hip.stream_of(dev))
         gw = partials.sum(0).to(ctx.weight_dtype) if need[6] else None
         return (gq if need[0] else None, gk if need[1] else None, gv if need[2] else None,
@@ -370,13 +438,20 @@ def bayes_mixer_readout(
         raise ValueError("norm_weight must have shape [8]")
     eps = torch.finfo(torch.float32).eps if norm_eps is None else float(norm_eps)
     projections = (q_proj, k_proj, v_proj, decay_logits, noise)
-    lds = _fused_eligible(projections, heads)
+    lds = _fused_eligible(projections, heads, whole=False)
     ldg = _row_stride(gate, t) if gate.dtype == torch.bfloat16 and gate.device == q_proj.device else None
-    if lds is not None and ldg is not None:
+    whole = _whole_tiles(heads, t)
+    if lds is not None and ldg is not None and (whole or (
+            _any_shape_call(heads, t, initial_mean, initial_covariance, chunk_length, denominator_floor, optimized)
+            and denominator_floor > 0 and eps >= 0 and norm_weight.dtype == torch.bfloat16
+            and norm_weight.device == q_proj.device)):
         _hip.load()
+        scan = None if whole else _LargeScan(projections)
         mean0, cov0 = _initial_state(initial_mean, initial_covariance, b * heads, q_proj.device)
-        return _MixerReadoutFunction.apply(q_proj, k_proj, v_proj, decay_logits, noise, gate, norm_weight, mean0,
+        outs = _MixerReadoutFunction.apply(q_proj, k_proj, v_proj, decay_logits, noise, gate, norm_weight, mean0,
                                            cov0, int(heads), eps, float(denominator_floor), (*lds, ldg))
+        if scan is None or scan.clean():
+            return outs
     read, mean_t, cov_t = bayes_mixer_core(*projections, heads=heads, initial_mean=initial_mean,
                                            initial_covariance=initial_covariance, chunk_length=chunk_length,
                                            denominator_floor=denominator_floor, optimized=optimized)
@@ -414,9 +489,9 @@ class _MixerBlockFunction(torch.autograd.Function):
         with _hip.on_device(dev):
             _hip.call("bssm_mixer_block_forward", P(projected), ld, P(cw32), P(bias), P(nw32), float(norm_eps),
                       P(mean0), P(cov0), P(convolved), P(out), P(read_bf16), P(mean_t), P(cov_t), P(bmean),
-                      P(bcov), b, t, heads, interval, float(denominator_floor), _hip.stream_of(dev))
+                      P(bcov), b, t, heads, _chunk_arg(heads, t), float(denominator_floor), _hip.stream_of(dev))
         ctx.save_for_backward(projected, cw32, bias, convolved, nw32, mean0, cov0, bmean, bcov, read_bf16)
-        ctx.heads, ctx.interval, ctx.ld = heads, interval, ld
+        ctx.heads, ctx.ld = heads, ld
         ctx.norm_eps, ctx.denominator_floor = float(norm_eps), float(denominator_floor)
         ctx.conv_shape, ctx.conv_dtype = tuple(conv_weight.shape), conv_weight.dtype
         ctx.norm_dtype = norm_weight.dtype
@@ -441,7 +516,7 @@ class _MixerBlockFunction(torch.autograd.Function):
         gproj = torch.empty(b, t, core + aux_w + heads * VALUE_DIM, device=dev, dtype=torch.bfloat16)
         gconv = torch.empty(b, t, core, device=dev, dtype=torch.bfloat16)
         cpart = torch.empty(b, core, 4, device=dev, dtype=torch.float32)
-        npart = torch.empty(b * heads // 16, VALUE_DIM, device=dev, dtype=torch.float32)
+        npart = torch.empty(b * (-(-heads // 16)), VALUE_DIM, device=dev, dtype=torch.float32)
         apart = torch.empty(b, aux_w, device=dev, dtype=torch.float32) if need[3] else None
         # The weight gradients are summed from their partials in the same call,
         # in the parameters' dtype when all of them are bf16 (else float32).
@@ -457,8 +532,8 @@ class _MixerBlockFunction(torch.autograd.Function):
             _hip.call("bssm_mixer_block_backward", P(projected), ctx.ld, P(cw32), P(bias), P(convolved),
                       P(nw32), ctx.norm_eps, P(mean0), P(cov0), P(bmean), P(bcov), P(read_bf16), P(grad_out), P(gm),
                       P(gc), P(gconv), P(gproj), gproj.shape[-1], P(cpart), P(npart), P(apart), P(g_conv),
-                      P(g_norm), P(g_bias), int(wdt == torch.bfloat16), P(gm0), P(gc0), b, t, heads, ctx.interval,
-                      ctx.denominator_floor, _hip.stream_of(dev))
+                      P(g_norm), P(g_bias), int(wdt == torch.bfloat16), P(gm0), P(gc0), b, t, heads,
+                      _chunk_arg(heads, t), ctx.denominator_floor, _hip.stream_of(dev))
         if g_conv is not None and g_conv.dtype != ctx.conv_dtype:
             g_conv = g_conv.to(ctx.conv_dtype)
         if g_norm is not None and g_norm.dtype != ctx.norm_dtype:
@@ -495,9 +570,9 @@ def bayes_mixer_block(
     (:599-601); the rest is ``bayes_mixer_readout``.  Returns the gated
     readout [B, T, H*8] and the final mean and covariance.
 
-    On the GPU (bf16 ``projected`` whose rows the kernels can address, heads a
-    multiple of 16, T a positive multiple of 4, an absent or bf16 [H*4 + H*2]
-    aux bias) the block is one C call per direction: the filter reads the
+    On the GPU (bf16 ``projected`` whose rows the kernels can address, shapes
+    and calls as described in the module docstring, an absent or bf16
+    [H*4 + H*2] aux bias) the block is one C call per direction: the filter reads the
     core columns in place and writes one contiguous [B, T, 2*H*4 + H*8]
     tensor, whose column views, with the aux and gate columns of
     ``projected``, feed the producer-fused readout kernels (which add the aux
@@ -523,7 +598,12 @@ def bayes_mixer_block(
         raise ValueError(f"conv_weight must have shape [{core}, 1, 4]")
     b, t = projected.shape[:2]
     ld = _row_stride(projected, t) if projected.is_cuda and projected.dtype == torch.bfloat16 else None
-    fused = (ld is not None and heads % 16 == 0 and t > 0 and t % 4 == 0
+    whole = _whole_tiles(heads, t)
+    fused = (ld is not None and t > 0
+             and (whole or (_any_shape_call(heads, t, initial_mean, initial_covariance, chunk_length,
+                                            denominator_floor, optimized)
+                            and conv_weight.dtype == norm_weight.dtype == torch.bfloat16
+                            and (norm_eps is None or norm_eps >= 0)))
              and conv_weight.device == projected.device and norm_weight.device == projected.device
              and tuple(norm_weight.shape) == (VALUE_DIM,)
              and (aux_bias is None or (aux_bias.device == projected.device and aux_bias.dtype == torch.bfloat16
@@ -531,9 +611,19 @@ def bayes_mixer_block(
     if fused:
         _hip.load()
         eps = torch.finfo(torch.float32).eps if norm_eps is None else float(norm_eps)
+        scan = None
+        if not whole:
+            # The layer's inputs come of the core and aux columns, the filter's taps and the bias (the taps as rows
+            # of 8: core is a multiple of 64).
+            views = [projected[..., :core + aux], _aligned(conv_weight.detach().reshape(1, -1, 8))]
+            if aux_bias is not None:
+                views.append(_aligned(aux_bias.detach()).view(1, 1, aux))
+            scan = _LargeScan(tuple(views))
         mean0, cov0 = _initial_state(initial_mean, initial_covariance, b * heads, projected.device)
-        return _MixerBlockFunction.apply(projected, conv_weight, norm_weight, aux_bias, mean0, cov0, int(heads), eps,
+        outs = _MixerBlockFunction.apply(projected, conv_weight, norm_weight, aux_bias, mean0, cov0, int(heads), eps,
                                          float(denominator_floor), ld)
+        if scan is None or scan.clean():
+            return outs
     from .conv import causal_depthwise4
 
     qkv = projected[..., :core]

@@ -186,18 +186,24 @@ int backward_impl(const char* fn, bool fixed, bool dyn, int d, int m, const floa
 // Shape and layout checks of the producer-fused mixer entry points.  The
 // kernels take 16 heads of one batch row per wave and address each batch
 // row of a stream through a 32-bit buffer range of T rows.
+// chunk: BSSM_ANY_SHAPE is taken out of it.
 int mixer_check(const char* fn, const void* const (&in)[5], const int64_t (&ld)[5], int64_t b, int64_t t, int64_t h,
-                int64_t chunk, float floor) {
+                int64_t& chunk, float floor) {
   static const int64_t kWidth[5] = {4, 4, 8, 4, 2};  // q, k, v, decay logits, noise (per head)
   static const char* kName[5] = {"q_proj", "k_proj", "v_proj", "decay_logits", "noise"};
   if (b < 0 || t < 0 || h < 0)
     return fail(BSSM_ERR_ARGUMENT, "%s: negative size b=%lld t=%lld h=%lld", fn, (long long)b, (long long)t,
                 (long long)h);
   if (!(floor > 0.f)) return fail(BSSM_ERR_ARGUMENT, "%s: denominator_floor must be positive", fn);
-  if (h % 16 != 0 || t <= 0 || t % 4 != 0 || chunk != bssm::kRot4Chunk)
+  const bool any_shape = chunk > 0 && (chunk & BSSM_ANY_SHAPE) != 0;
+  if (any_shape) chunk &= ~BSSM_ANY_SHAPE;
+  if (any_shape && (h <= 0 || h % 4 != 0 || t <= 0 || chunk != bssm::kRot4Chunk))
+    return fail(BSSM_ERR_UNSUPPORTED, "%s: needs heads a positive multiple of 4, T > 0 and chunk == %d (got h=%lld "
+                "t=%lld chunk=%lld)", fn, bssm::kRot4Chunk, (long long)h, (long long)t, (long long)chunk);
+  if (!any_shape && (h % 16 != 0 || t <= 0 || t % 4 != 0 || chunk != bssm::kRot4Chunk))
     return fail(BSSM_ERR_UNSUPPORTED, "%s: needs heads %% 16 == 0, T a positive multiple of 4 and chunk == %d (got h=%lld t=%lld "
                 "chunk=%lld)", fn, bssm::kRot4Chunk, (long long)h, (long long)t, (long long)chunk);
-  if (b * h / 16 > 0x7fffffff) return fail(BSSM_ERR_ARGUMENT, "%s: batch * heads too large", fn);
+  if (b * ((h + 15) / 16) > 0x7fffffff) return fail(BSSM_ERR_ARGUMENT, "%s: batch * heads too large", fn);
   const int64_t nb = (t + chunk - 1) / chunk;
   if ((nb + 1) * 128 * 16 >= ((int64_t)1 << 31) || t * h * 32 >= ((int64_t)1 << 31))
     return fail(BSSM_ERR_ARGUMENT, "%s: T * heads too large for 32-bit stream offsets", fn);
@@ -599,6 +605,31 @@ int bssm_value_stats(int count, const void* const* tensors, const int64_t* numel
   return launched(fn, bssm::launch_value_stats(a, workspace, out, static_cast<hipStream_t>(stream)));
 }
 
+int bssm_bf16_large_blocks(void) { return bssm::kLargeBlocks; }
+
+int bssm_bf16_large(int count, const void* const* tensors, const int64_t* ld, const int64_t* cols,
+                    const int64_t* rows, int32_t* flags, void* stream) {
+  const char* fn = "bssm_bf16_large";
+  if (count < 1 || count > bssm::kMaxLargeStreams)
+    return fail(BSSM_ERR_ARGUMENT, "%s: needs 1 to %d streams", fn, bssm::kMaxLargeStreams);
+  if (tensors == nullptr || ld == nullptr || cols == nullptr || rows == nullptr || flags == nullptr)
+    return fail(BSSM_ERR_ARGUMENT, "%s: null argument", fn);
+  bssm::LargeArgs a{};
+  a.count = count;
+  for (int i = 0; i < count; ++i) {
+    if (rows[i] < 0) return fail(BSSM_ERR_ARGUMENT, "%s: stream %d has a negative row count", fn, i);
+    if (rows[i] * cols[i] > 0 && (tensors[i] == nullptr || !aligned16(tensors[i])))
+      return fail(BSSM_ERR_ARGUMENT, "%s: stream %d must be non-null and 16-byte aligned", fn, i);
+    if (cols[i] < 0 || cols[i] % 8 != 0 || (rows[i] > 1 && (ld[i] < cols[i] || ld[i] % 8 != 0)))
+      return fail(BSSM_ERR_ARGUMENT, "%s: stream %d needs columns and a row stride that are multiples of 8", fn, i);
+    a.ptr[i] = tensors[i];
+    a.ld[i] = ld[i];
+    a.cols[i] = cols[i];
+    a.rows[i] = rows[i];
+  }
+  return launched(fn, bssm::launch_large_bf16(a, flags, static_cast<hipStream_t>(stream)));
+}
+
 int bssm_round_float8(int format, const float* x, uint8_t* out, int64_t count) {
   const char* fn = "bssm_round_float8";
   if (format != 0 && format != 1)
@@ -785,7 +816,7 @@ struct BlockStreams {
 };
 
 int block_check(const char* fn, const void* projected, int64_t ld_projected, const float* conv_weight,
-                const void* aux_bias, const void* convolved, int64_t b, int64_t t, int64_t h, int64_t chunk,
+                const void* aux_bias, const void* convolved, int64_t b, int64_t t, int64_t h, int64_t& chunk,
                 float floor, const BlockStreams& s) {
   if (h <= 0 || b < 0) return fail(BSSM_ERR_ARGUMENT, "%s: needs heads > 0 and batch >= 0", fn);
   if (ld_projected < 30 * h)
@@ -910,7 +941,7 @@ int bssm_mixer_block_backward(const void* projected, int64_t ld_projected, const
   bssm::FoldArgs f{};
   const float* parts[3] = {grad_conv_weight_partials, grad_norm_weight_partials, grad_aux_partials};
   void* outs[3] = {grad_conv_weight, grad_norm_weight, grad_aux_bias};
-  const int64_t rows[3] = {batch, batch * heads / 16, batch}, cols[3] = {16 * heads * 4, 8, 6 * heads};
+  const int64_t rows[3] = {batch, batch * ((heads + 15) / 16), batch}, cols[3] = {16 * heads * 4, 8, 6 * heads};
   for (int i = 0; i < 3; ++i) {
     if (outs[i] == nullptr) continue;
     f.part[f.count] = parts[i];

@@ -177,7 +177,7 @@ struct MixArgs {
   // the backward (y is not written).  Backward: gy is formed on chip from
   // gout (bf16 [B, T, H * 8]), yb and gate; ggate [B, T, H * 8] is written
   // bf16 (float32 when precise) and the weight gradient as per-wave partials
-  // gw_part [B * H / 16, 8].
+  // gw_part [B * ceil(H / 16), 8].
   const void* gate;
   int64_t ldg;
   const float* norm_w;
@@ -273,6 +273,18 @@ struct StatArgs {
 };
 int64_t stat_blocks(int64_t numel);
 hipError_t launch_value_stats(const StatArgs& a, float* partials, float* out, hipStream_t stream);
+
+// Whether any value of up to kMaxLargeStreams bf16 row views (rows[i] rows of
+// cols[i] elements, ld[i] apart; cols and ld multiples of 8, 16-byte aligned)
+// is NaN, infinite or at least 2^63 in magnitude: one flag per block.
+constexpr int kMaxLargeStreams = 8;
+constexpr int kLargeBlocks = 512;
+struct LargeArgs {
+  const void* ptr[kMaxLargeStreams];
+  int64_t ld[kMaxLargeStreams], cols[kMaxLargeStreams], rows[kMaxLargeStreams];
+  int count;
+};
+hipError_t launch_large_bf16(const LargeArgs& a, int* flags, hipStream_t stream);
 
 hipError_t launch_associative_scan(const float* k, const float* v, const float* q, const float* r,
                                    const float* m0, const float* c0, float* y, float* mT, float* cT,

@@ -313,6 +313,18 @@ int bssm_backward_chunked_narrow(int key_dim, int value_dim, int fixed, int form
                                  float* gm0, float* gc0,
                                  int64_t n, int64_t t, int64_t chunk, float denominator_floor, void* stream);
 
+/* Whether bf16 row views hold a NaN, an infinity or a magnitude of 2^63 or
+ * more: count (1 to 8) views, tensors[i] [rows[i], cols[i]] with row
+ * stride ld[i] (elements; cols and ld multiples of 8, 16-byte aligned).
+ * Writes one flag per block into flags [bssm_bf16_large_blocks()] (device
+ * memory), nonzero where the block saw one.  The array arguments are host
+ * memory.  Serves the mixer's argument check (the reference validates the
+ * layer's inputs, bayes_ssm/bayesian_layer.py:105-129); no counterpart in the
+ * reference library. */
+int bssm_bf16_large_blocks(void);
+int bssm_bf16_large(int count, const void* const* tensors, const int64_t* ld, const int64_t* cols,
+                    const int64_t* rows, int32_t* flags, void* stream);
+
 /* Host-side float32 -> float8 rounding of the float8 gradients (format as
  * above): round to nearest even; e4m3fn gives the NaN code 0x7f (with the
  * sign) for magnitudes that round past 448, for infinities and NaN; e5m2
@@ -389,9 +401,12 @@ int bssm_associative_static_scan_backward(const float* keys, const float* values
  * (contiguous), mean_final, cov_final, and the checkpoints bmean
  * [B*H, nb+1, 4, 8], bcov [B*H, nb+1, 4, 4] with nb = ceil(T / chunk).
  * Needs H % 16 == 0, T a positive multiple of 4, chunk ==
- * bssm_preferred_checkpoint(4);
+ * bssm_preferred_checkpoint(4), or, with BSSM_ANY_SHAPE or-ed into chunk, H a
+ * positive multiple of 4 and any T > 0 (in all six mixer entry points; the
+ * per-wave partial sums then have B * ceil(H / 16) rows);
  * otherwise BSSM_ERR_UNSUPPORTED.  No counterpart in the reference library:
  * its mixer materialises every transformed and permuted tensor in float32. */
+#define BSSM_ANY_SHAPE ((int64_t)1 << 32)
 int bssm_mixer_forward(const void* q_proj, int64_t ldq, const void* k_proj, int64_t ldk,
                        const void* v_proj, int64_t ldv, const void* decay_logits, int64_t ldd,
                        const void* noise, int64_t ldn,

@@ -57,6 +57,7 @@ _SIGNATURES = {
     "bssm_bf16_large": [_I, _P, _P, _P, _P, _P, _P],
     "bssm_value_stats_workspace": [_I, _P],
     "bssm_value_stats": [_I, _P, _P, _P, _P, _L, _P, _P],
+    "bssm_mixer_row_kernels": [_I, _L, _L, _L],
     "bssm_associative_static_scan": [_P] * 9 + [_L, _L, _I, _I, _P],
     "bssm_associative_static_scan_backward": [_P] * 16 + [_L, _L, _I, _I, _P],
     "bssm_mixer_forward": [_P, _L] * 5 + [_P] * 7 + [_L, _L, _L, _L, _F, _P],
@@ -79,6 +80,7 @@ _SIGNATURES = {
 }
 ABI_VERSION = 10
 ANY_SHAPE = 1 << 32  # or-ed into the mixer entry points' chunk (BSSM_ANY_SHAPE)
+ROW_KERNELS = 1 << 33  # the same (BSSM_ROW_KERNELS)
 
 _lock = threading.Lock()
 _lib: Optional[ctypes.CDLL] = None

@@ -76,10 +76,21 @@ def _whole_tiles(heads: int, t: int) -> bool:
     return heads % 16 == 0 and t % 4 == 0
 
 
-def _chunk_arg(heads: int, t: int) -> int:
-    """The checkpoint interval as the C entry points take it (with BSSM_ANY_SHAPE off whole tiles)."""
+def _chunk_arg(b: int, heads: int, t: int, backward: bool = False) -> int:
+    """The checkpoint interval as the C entry points take it: off whole tiles with BSSM_ANY_SHAPE, and with
+    BSSM_ROW_KERNELS where the small-batch kernels are the faster ones."""
     interval = _hip.preferred_checkpoint(KEY_DIM)
-    return interval if _whole_tiles(heads, t) else interval | _hip.ANY_SHAPE
+    if _whole_tiles(heads, t):
+        return interval
+    rows = _hip.load().bssm_mixer_row_kernels(int(backward), b, t, heads)
+    return interval | _hip.ANY_SHAPE | (_hip.ROW_KERNELS if rows else 0)
+
+
+def _partials(chunk: int, b: int, heads: int, device: torch.device) -> Tensor:
+    """Partial sums of the norm-weight gradient: a row, or with the small-batch kernels four, for each 16 heads of a
+    batch row."""
+    rows = b * (-(-heads // 16)) * (4 if chunk & _hip.ROW_KERNELS else 1)
+    return torch.empty(rows, VALUE_DIM, device=device, dtype=torch.float32)
 
 
 def _any_shape_call(heads: int, t: int, initial_mean: Optional[Tensor], initial_covariance: Optional[Tensor],
@@ -165,7 +176,7 @@ class _MixerCoreFunction(torch.autograd.Function):
         with _hip.on_device(dev):
             _hip.call("bssm_mixer_forward", P(q_proj), lds[0], P(k_proj), lds[1], P(v_proj), lds[2],
                       P(decay_logits), lds[3], P(noise), lds[4], P(initial_mean), P(initial_covariance), P(read),
-                      P(mean_t), P(cov_t), P(bmean), P(bcov), b, t, heads, _chunk_arg(heads, t),
+                      P(mean_t), P(cov_t), P(bmean), P(bcov), b, t, heads, _chunk_arg(b, heads, t),
                       float(denominator_floor),
                       _hip.stream_of(dev))
         ctx.save_for_backward(q_proj, k_proj, v_proj, decay_logits, noise, initial_mean, initial_covariance,
@@ -204,7 +215,7 @@ class _MixerCoreFunction(torch.autograd.Function):
             _hip.call("bssm_mixer_backward", P(q_proj), lds[0], P(k_proj), lds[1], P(v_proj), lds[2],
                       P(decay_logits), lds[3], P(noise), lds[4], P(mean0), P(cov0), P(bmean), P(bcov),
                       P(grad_read), P(gm), P(gc), P(gq), P(gk), P(gv), P(gdl), P(gnz), P(gm0), P(gc0), b, t, heads,
-                      _chunk_arg(heads, t), ctx.denominator_floor, 0, _hip.stream_of(dev))
+                      _chunk_arg(b, heads, t, backward=True), ctx.denominator_floor, 0, _hip.stream_of(dev))
         return (gq if need[0] else None, gk if need[1] else None, gv if need[2] else None,
                 gdl if need[3] else None, gnz if need[4] else None, gm0, gc0, None, None, None)
 
@@ -349,7 +360,7 @@ class _MixerReadoutFunction(torch.autograd.Function):
             _hip.call("bssm_mixer_gated_forward", P(q_proj), lds[0], P(k_proj), lds[1], P(v_proj), lds[2],
                       P(decay_logits), lds[3], P(noise), lds[4], P(gate), lds[5], P(w32), float(norm_eps),
                       P(initial_mean), P(initial_covariance), P(out), P(read_bf16), P(mean_t), P(cov_t), P(bmean),
-                      P(bcov), b, t, heads, _chunk_arg(heads, t), float(denominator_floor), 0, _hip.stream_of(dev))
+                      P(bcov), b, t, heads, _chunk_arg(b, heads, t), float(denominator_floor), 0, _hip.stream_of(dev))
         ctx.save_for_backward(q_proj, k_proj, v_proj, decay_logits, noise, gate, w32, initial_mean,
                               initial_covariance, bmean, bcov, read_bf16)
         ctx.heads = heads
@@ -383,7 +394,8 @@ class _MixerReadoutFunction(torch.autograd.Function):
         gdl = empty(decay_logits) if dyn else None
         gnz = empty(noise) if dyn else None
         ggate = empty(gate)
-        partials = torch.empty(b * (-(-heads // 16)), VALUE_DIM, device=dev, dtype=torch.float32)
+        chunk = _chunk_arg(b, heads, t, backward=True)
+        partials = _partials(chunk, b, heads, dev)
         gm0 = torch.empty_like(mean0) if need[7] else None
         gc0 = torch.empty_like(cov0) if need[8] else None
         P = _hip.ptr
@@ -391,7 +403,7 @@ class _MixerReadoutFunction(torch.autograd.Function):
             _hip.call("bssm_mixer_gated_backward", P(q_proj), lds[0], P(k_proj), lds[1], P(v_proj), lds[2],
                       P(decay_logits), lds[3], P(noise), lds[4], P(gate), lds[5], P(w32), ctx.norm_eps, P(mean0),
                       P(cov0), P(bmean), P(bcov), P(read_bf16), P(grad_out), P(gm), P(gc), P(gq), P(gk), P(gv),
-                      P(gdl), P(gnz), P(ggate), P(partials), P(gm0), P(gc0), b, t, heads, _chunk_arg(heads, t),
+                      P(gdl), P(gnz), P(ggate), P(partials), P(gm0), P(gc0), b, t, heads, chunk,
                       ctx.denominator_floor, 0, _hip.stream_of(dev))
         gw = partials.sum(0).to(ctx.weight_dtype) if need[6] else None
         return (gq if need[0] else None, gk if need[1] else None, gv if need[2] else None,
@@ -489,7 +501,7 @@ class _MixerBlockFunction(torch.autograd.Function):
         with _hip.on_device(dev):
             _hip.call("bssm_mixer_block_forward", P(projected), ld, P(cw32), P(bias), P(nw32), float(norm_eps),
                       P(mean0), P(cov0), P(convolved), P(out), P(read_bf16), P(mean_t), P(cov_t), P(bmean),
-                      P(bcov), b, t, heads, _chunk_arg(heads, t), float(denominator_floor), _hip.stream_of(dev))
+                      P(bcov), b, t, heads, _chunk_arg(b, heads, t), float(denominator_floor), _hip.stream_of(dev))
         ctx.save_for_backward(projected, cw32, bias, convolved, nw32, mean0, cov0, bmean, bcov, read_bf16)
         ctx.heads, ctx.ld = heads, ld
         ctx.norm_eps, ctx.denominator_floor = float(norm_eps), float(denominator_floor)
@@ -516,7 +528,8 @@ class _MixerBlockFunction(torch.autograd.Function):
         gproj = torch.empty(b, t, core + aux_w + heads * VALUE_DIM, device=dev, dtype=torch.bfloat16)
         gconv = torch.empty(b, t, core, device=dev, dtype=torch.bfloat16)
         cpart = torch.empty(b, core, 4, device=dev, dtype=torch.float32)
-        npart = torch.empty(b * (-(-heads // 16)), VALUE_DIM, device=dev, dtype=torch.float32)
+        chunk = _chunk_arg(b, heads, t, backward=True)
+        npart = _partials(chunk, b, heads, dev)
         apart = torch.empty(b, aux_w, device=dev, dtype=torch.float32) if need[3] else None
         # The weight gradients are summed from their partials in the same call,
         # in the parameters' dtype when all of them are bf16 (else float32).
@@ -533,7 +546,7 @@ class _MixerBlockFunction(torch.autograd.Function):
                       P(nw32), ctx.norm_eps, P(mean0), P(cov0), P(bmean), P(bcov), P(read_bf16), P(grad_out), P(gm),
                       P(gc), P(gconv), P(gproj), gproj.shape[-1], P(cpart), P(npart), P(apart), P(g_conv),
                       P(g_norm), P(g_bias), int(wdt == torch.bfloat16), P(gm0), P(gc0), b, t, heads,
-                      _chunk_arg(heads, t), ctx.denominator_floor, _hip.stream_of(dev))
+                      chunk, ctx.denominator_floor, _hip.stream_of(dev))
         if g_conv is not None and g_conv.dtype != ctx.conv_dtype:
             g_conv = g_conv.to(ctx.conv_dtype)
         if g_norm is not None and g_norm.dtype != ctx.norm_dtype:

@@ -186,7 +186,11 @@ int backward_impl(const char* fn, bool fixed, bool dyn, int d, int m, const floa
 // Shape and layout checks of the producer-fused mixer entry points.  The
 // kernels take 16 heads of one batch row per wave and address each batch
 // row of a stream through a 32-bit buffer range of T rows.
-// chunk: BSSM_ANY_SHAPE is taken out of it.
+bool takes_row_kernels(int64_t chunk, int64_t heads) {
+  return chunk > 0 && (chunk & BSSM_ROW_KERNELS) != 0 && heads % 4 == 0;
+}
+
+// chunk: BSSM_ANY_SHAPE and BSSM_ROW_KERNELS are taken out of it.
 int mixer_check(const char* fn, const void* const (&in)[5], const int64_t (&ld)[5], int64_t b, int64_t t, int64_t h,
                 int64_t& chunk, float floor) {
   static const int64_t kWidth[5] = {4, 4, 8, 4, 2};  // q, k, v, decay logits, noise (per head)
@@ -196,7 +200,7 @@ int mixer_check(const char* fn, const void* const (&in)[5], const int64_t (&ld)[
                 (long long)h);
   if (!(floor > 0.f)) return fail(BSSM_ERR_ARGUMENT, "%s: denominator_floor must be positive", fn);
   const bool any_shape = chunk > 0 && (chunk & BSSM_ANY_SHAPE) != 0;
-  if (any_shape) chunk &= ~BSSM_ANY_SHAPE;
+  if (chunk > 0) chunk &= ~(BSSM_ANY_SHAPE | BSSM_ROW_KERNELS);
   if (any_shape && (h <= 0 || h % 4 != 0 || t <= 0 || chunk != bssm::kRot4Chunk))
     return fail(BSSM_ERR_UNSUPPORTED, "%s: needs heads a positive multiple of 4, T > 0 and chunk == %d (got h=%lld "
                 "t=%lld chunk=%lld)", fn, bssm::kRot4Chunk, (long long)h, (long long)t, (long long)chunk);
@@ -648,6 +652,7 @@ int bssm_mixer_forward(const void* q_proj, int64_t ldq, const void* k_proj, int6
                        float* bmean, float* bcov, int64_t batch, int64_t t, int64_t heads, int64_t chunk,
                        float denominator_floor, void* stream) {
   const char* fn = "bssm_mixer_forward";
+  const bool row = takes_row_kernels(chunk, heads);
   if (int rc = mixer_check(fn, {q_proj, k_proj, v_proj, decay_logits, noise}, {ldq, ldk, ldv, ldd, ldn}, batch, t,
                            heads, chunk, denominator_floor))
     return rc;
@@ -664,6 +669,7 @@ int bssm_mixer_forward(const void* q_proj, int64_t ldq, const void* k_proj, int6
     if (p != nullptr && !aligned8(p)) return fail(BSSM_ERR_ARGUMENT, "%s: belief tensors must be 8-byte aligned", fn);
   if (read != nullptr && !aligned16(read)) return fail(BSSM_ERR_ARGUMENT, "%s: read must be 16-byte aligned", fn);
   bssm::MixArgs a{};
+  a.row = row;
   a.q = q_proj; a.k = k_proj; a.v = v_proj; a.dl = decay_logits; a.nz = noise;
   a.ldq = ldq; a.ldk = ldk; a.ldv = ldv; a.ldd = ldd; a.ldn = ldn;
   a.m0 = mean0; a.c0 = cov0; a.y = read; a.mT = mean_final; a.cT = cov_final; a.bm = bmean; a.bc = bcov;
@@ -680,6 +686,7 @@ int bssm_mixer_backward(const void* q_proj, int64_t ldq, const void* k_proj, int
                         int64_t batch, int64_t t, int64_t heads, int64_t chunk, float denominator_floor,
                         int grad_f32, void* stream) {
   const char* fn = "bssm_mixer_backward";
+  const bool row = takes_row_kernels(chunk, heads);
   if (int rc = mixer_check(fn, {q_proj, k_proj, v_proj, decay_logits, noise}, {ldq, ldk, ldv, ldd, ldn}, batch, t,
                            heads, chunk, denominator_floor))
     return rc;
@@ -702,6 +709,7 @@ int bssm_mixer_backward(const void* q_proj, int64_t ldq, const void* k_proj, int
     if (p != nullptr && !aligned16(p))
       return fail(BSSM_ERR_ARGUMENT, "%s: grad_read and the projection gradients must be 16-byte aligned", fn);
   bssm::MixArgs a{};
+  a.row = row;
   a.q = q_proj; a.k = k_proj; a.v = v_proj; a.dl = decay_logits; a.nz = noise;
   a.ldq = ldq; a.ldk = ldk; a.ldv = ldv; a.ldd = ldd; a.ldn = ldn;
   a.m0 = mean0; a.c0 = cov0; a.bmr = bmean; a.bcr = bcov; a.gy = grad_read; a.gmf = gmf; a.gcf = gcf;
@@ -720,6 +728,7 @@ int bssm_mixer_gated_forward(const void* q_proj, int64_t ldq, const void* k_proj
                              float* cov_final, float* bmean, float* bcov, int64_t batch, int64_t t, int64_t heads,
                              int64_t chunk, float denominator_floor, int precise, void* stream) {
   const char* fn = "bssm_mixer_gated_forward";
+  const bool row = takes_row_kernels(chunk, heads);
   if (int rc = mixer_check(fn, {q_proj, k_proj, v_proj, decay_logits, noise}, {ldq, ldk, ldv, ldd, ldn}, batch, t,
                            heads, chunk, denominator_floor))
     return rc;
@@ -735,6 +744,7 @@ int bssm_mixer_gated_forward(const void* q_proj, int64_t ldq, const void* k_proj
                         (const void*)bmean, (const void*)bcov})
     if (p != nullptr && !aligned8(p)) return fail(BSSM_ERR_ARGUMENT, "%s: belief tensors must be 8-byte aligned", fn);
   bssm::MixArgs a{};
+  a.row = row;
   a.q = q_proj; a.k = k_proj; a.v = v_proj; a.dl = decay_logits; a.nz = noise;
   a.ldq = ldq; a.ldk = ldk; a.ldv = ldv; a.ldd = ldd; a.ldn = ldn;
   a.m0 = mean0; a.c0 = cov0; a.mT = mean_final; a.cT = cov_final; a.bm = bmean; a.bc = bcov;
@@ -755,6 +765,7 @@ int bssm_mixer_gated_backward(const void* q_proj, int64_t ldq, const void* k_pro
                               int64_t batch, int64_t t, int64_t heads, int64_t chunk, float denominator_floor,
                               int precise, void* stream) {
   const char* fn = "bssm_mixer_gated_backward";
+  const bool row = takes_row_kernels(chunk, heads);
   if (int rc = mixer_check(fn, {q_proj, k_proj, v_proj, decay_logits, noise}, {ldq, ldk, ldv, ldd, ldn}, batch, t,
                            heads, chunk, denominator_floor))
     return rc;
@@ -779,6 +790,7 @@ int bssm_mixer_gated_backward(const void* q_proj, int64_t ldq, const void* k_pro
     if (p != nullptr && !aligned16(p))
       return fail(BSSM_ERR_ARGUMENT, "%s: the projection gradients must be 16-byte aligned", fn);
   bssm::MixArgs a{};
+  a.row = row;
   a.q = q_proj; a.k = k_proj; a.v = v_proj; a.dl = decay_logits; a.nz = noise;
   a.ldq = ldq; a.ldk = ldk; a.ldv = ldv; a.ldd = ldd; a.ldn = ldn;
   a.m0 = mean0; a.c0 = cov0; a.bmr = bmean; a.bcr = bcov; a.gmf = gmf; a.gcf = gcf;
@@ -840,6 +852,7 @@ int bssm_mixer_block_forward(const void* projected, int64_t ld_projected, const 
                              float* cov_final, float* bmean, float* bcov, int64_t batch, int64_t t, int64_t heads,
                              int64_t chunk, float denominator_floor, void* stream) {
   const char* fn = "bssm_mixer_block_forward";
+  const bool row = takes_row_kernels(chunk, heads);
   const BlockStreams s(projected, convolved, heads);
   if (int rc = block_check(fn, projected, ld_projected, conv_weight, aux_bias, convolved, batch, t, heads, chunk,
                            denominator_floor, s))
@@ -863,6 +876,7 @@ int bssm_mixer_block_forward(const void* projected, int64_t ld_projected, const 
   c.bf16 = 1;
   if (hipError_t e = bssm::launch_conv4_forward(c, st); e != hipSuccess) return launched(fn, e);
   bssm::MixArgs a{};
+  a.row = row;
   a.q = s.q; a.k = s.k; a.v = s.v; a.dl = s.dl; a.nz = s.nz;
   a.ldq = a.ldk = a.ldv = s.ldc; a.ldd = a.ldn = ld_projected; a.abias = aux_bias;
   a.m0 = mean0; a.c0 = cov0; a.mT = mean_final; a.cT = cov_final; a.bm = bmean; a.bc = bcov;
@@ -883,6 +897,7 @@ int bssm_mixer_block_backward(const void* projected, int64_t ld_projected, const
                               int64_t batch, int64_t t, int64_t heads, int64_t chunk, float denominator_floor,
                               void* stream) {
   const char* fn = "bssm_mixer_block_backward";
+  const bool row = takes_row_kernels(chunk, heads);
   const BlockStreams s(projected, convolved, heads);
   if (int rc = block_check(fn, projected, ld_projected, conv_weight, aux_bias, convolved, batch, t, heads, chunk,
                            denominator_floor, s))
@@ -913,6 +928,7 @@ int bssm_mixer_block_backward(const void* projected, int64_t ld_projected, const
   char* gp = static_cast<char*>(grad_projected);
   char* gc = static_cast<char*>(grad_convolved);
   bssm::MixArgs a{};
+  a.row = row;
   a.q = s.q; a.k = s.k; a.v = s.v; a.dl = s.dl; a.nz = s.nz;
   a.ldq = a.ldk = a.ldv = s.ldc; a.ldd = a.ldn = ld_projected; a.abias = aux_bias;
   a.m0 = mean0; a.c0 = cov0; a.bmr = bmean; a.bcr = bcov; a.gmf = gmf; a.gcf = gcf;
@@ -941,7 +957,8 @@ int bssm_mixer_block_backward(const void* projected, int64_t ld_projected, const
   bssm::FoldArgs f{};
   const float* parts[3] = {grad_conv_weight_partials, grad_norm_weight_partials, grad_aux_partials};
   void* outs[3] = {grad_conv_weight, grad_norm_weight, grad_aux_bias};
-  const int64_t rows[3] = {batch, batch * ((heads + 15) / 16), batch}, cols[3] = {16 * heads * 4, 8, 6 * heads};
+  const int64_t rows[3] = {batch, batch * ((heads + 15) / 16) * (a.row ? 4 : 1), batch};
+  const int64_t cols[3] = {16 * heads * 4, 8, 6 * heads};
   for (int i = 0; i < 3; ++i) {
     if (outs[i] == nullptr) continue;
     f.part[f.count] = parts[i];
@@ -955,6 +972,10 @@ int bssm_mixer_block_backward(const void* projected, int64_t ld_projected, const
 }
 
 int bssm_rotation_checkpoint(int key_dim) { return bssm::rotation_checkpoint(key_dim); }
+
+int bssm_mixer_row_kernels(int backward, int64_t batch, int64_t t, int64_t heads) {
+  return bssm::mixer_row_kernels(backward != 0, batch, t, heads);
+}
 
 int64_t bssm_small_batch_limit(int direction, int64_t limit) {
   if (direction < 0 || direction > 4) return -1;

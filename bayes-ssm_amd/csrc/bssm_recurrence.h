@@ -177,7 +177,7 @@ struct MixArgs {
   // the backward (y is not written).  Backward: gy is formed on chip from
   // gout (bf16 [B, T, H * 8]), yb and gate; ggate [B, T, H * 8] is written
   // bf16 (float32 when precise) and the weight gradient as per-wave partials
-  // gw_part [B * ceil(H / 16), 8].
+  // gw_part [B * ceil(H / 16), 8], or with row [4 B * ceil(H / 16), 8].
   const void* gate;
   int64_t ldg;
   const float* norm_w;
@@ -188,12 +188,16 @@ struct MixArgs {
   void* ggate;
   float* gw_part;
   int precise;
+  int row;  // take the row kernels (bssm_mixer_row.hip)
   // Aux bias (bf16 [6 H]: decay logits 4 H, then noise 2 H; null: none),
   // added to the decay-logit and noise pieces in bf16 (one rounding) as
   // they are read.
   const void* abias;
 };
 hipError_t launch_mixer_forward(const MixArgs& a, hipStream_t stream);
+bool mixer_row_kernels(bool backward, int64_t b, int64_t t, int64_t h);
+hipError_t launch_mixer_forward_row(const MixArgs& a, hipStream_t stream);
+hipError_t launch_mixer_backward_row(const MixArgs& a, hipStream_t stream);
 hipError_t launch_mixer_backward(const MixArgs& a, hipStream_t stream);
 
 // Rotation dynamics (bssm_rotation.hip): keys/queries [N, T, D], values,

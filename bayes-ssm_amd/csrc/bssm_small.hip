@@ -1,80 +1,16 @@
-// Row-per-sequence kernels for D = 4, M = 8 at small sequence counts, gfx950.
-//
-// The rotated-layout kernels (bssm_rot4.h) give a quad of 4 lanes to each
-// sequence, 16 sequences per wave.  Below about 1024 x 16 sequences their
-// waves do not fill the SIMDs, and each wave's time is its own instruction
-// stream: a wave issues the same instructions whatever number of its lanes
-// hold live sequences.  Here a 16-lane DPP row holds one sequence (4 per
-// wave) and every lane one entry of the covariance, so the per-token stream
-// is about 40 % shorter (four times as many waves, each doing a quarter of
-// the state).  The row layout spends about 2.4 times the lane work per
-// sequence, so once every SIMD holds several waves the rotated layout wins:
-// for the backward above about 8192 sequences, for the forward (which at
-// 16384 sequences still gains from its 4 waves per SIMD against the rotated
-// layout's one) above about 24576.
-//
-// Lane (i, j) of a sequence's row (i = row bits 3:2, j = bits 1:0) holds
-//   P[i][j]                    (the covariance, bitwise symmetric)
-//   M[j][2i], M[j][2i + 1]     (the mean, transposed: row j of M)
-// The forward keeps the lane's mean pair in its own order instead,
-// (M[j][c], M[j][c ^ 1]) with c = 2i + (j & 1): the lanes j, j ^ 1 of a quad
-// then hold the same column pair in opposite order, so a sum over j of a
-// column is an exchange between them and one quad step that leaves each lane
-// its own column's sum (and its partner the other's): a reduce-scatter in
-// place of two all-reduces for the readout and the innovations.  In the
-// backward the extra exchange lengthens the chained reverse; it keeps the
-// record order.
-// Sums over j are quad all-reduces (xor 1, xor 2); sums over i are
-// "column" all-reduces over the row: the pair (i, i ^ 1) through the half-row
-// mirror and a quad reversal, then the pairs through a row rotation by 8.
-// Both pair their four terms as ((a0 + a1) + (a2 + a3)), so a row sum and the
-// matching column sum of the symmetric covariance give the same bits, and
-// every quantity a lane needs in both orientations (u_i and u_j) is formed
-// from them identically: the covariance update stays bitwise symmetric.
-//
-// The equations are those of bssm_rot4.h (forward_step): u = d * (P (d * k))
-// + p k, s = r + k.u, beta = 1 / max(s, floor), e = v - (d * M)^T k,
-// M <- d * M + beta u e^T, P <- d d^T * P + p I - beta u u^T, y = M^T q.
+// Row-per-sequence kernels for D = 4, M = 8 at small sequence counts, gfx950
+// (the layout and the step's halves: bssm_row.h).
 
 #include <atomic>
 #include <cfloat>
 
-#include "bssm_rot4.h"
+#include "bssm_row.h"
 
-// No contraction: a sum like x + dpp(x) with x = a * b would otherwise be
-// fused into fma(a, b, dpp(x)), which rounds the two lanes of a pair
-// differently and breaks the bitwise agreement of row and column sums.
-// Every intended fused multiply-add is an explicit fmaf.
-#pragma clang fp contract(off)
+#pragma clang fp contract(off)  // as in bssm_row.h
 
 namespace bssm {
 namespace sn {
 namespace {
-
-constexpr int SPW = 4;   // sequences per wave
-constexpr int TT = 16;   // tokens per staged tile
-constexpr int kRowRor8 = 0x128;
-constexpr int kQuadRev = quad_perm(3, 2, 1, 0);
-
-using r4::Rsrc;
-using r4::make_rsrc;
-using r4::kOob;
-using r4::store_words;
-using r4::v4u;
-typedef float v2f __attribute__((ext_vector_type(2)));
-
-// Sum over the 4 lanes j of the quad; identical bits in the quad.
-__device__ __forceinline__ float quad_sum(float x) {
-  x += dpp<kXor1>(x);
-  return x + dpp<kXor2>(x);
-}
-// Sum over the 4 rows i of the 16-lane row at fixed j; identical bits in the
-// column, and equal to quad_sum of the transposed terms.
-__device__ __forceinline__ float col_sum(float x) {
-  const float m = dpp<kHalfMirror>(x);  // lane (i ^ 1, 3 - j)
-  x += dpp<kQuadRev>(m);                // + lane (i ^ 1, j)
-  return x + dpp<kRowRor8>(x);          // + rows i ^ 2, i ^ 3
-}
 
 // LDS tile of one wave: per sequence k, d, q [TT][4], v / y [TT][8], p, r
 // [TT], at a stride of 8 banks (mod 32), so that the 4 sequences' reads of
@@ -270,22 +206,6 @@ struct Bel {
   float P, M0, M1;
 };
 
-// The lane's mean pair between record order (columns 2i, 2i + 1) and its own
-// order (c, c ^ 1); the same swap both ways.
-__device__ __forceinline__ v2f own_order(v2f m, bool odd) {
-  v2f r;
-  r[0] = odd ? m[1] : m[0];
-  r[1] = odd ? m[0] : m[1];
-  return r;
-}
-
-// Sum over the quad of the lane's own column, given the lane's terms of its
-// own column (x0) and of the other (x1).
-__device__ __forceinline__ float own_sum(float x0, float x1) {
-  const float t = x0 + dpp<kXor1>(x1);
-  return t + dpp<kXor2>(t);
-}
-
 struct StepOut {
   float ui, uj, s;
   v2f e;
@@ -337,10 +257,6 @@ __device__ __forceinline__ void forward_step(Bel& b, const Tok& x, float delta, 
 // Readout of the lane's own column after the token (own order):
 // y_c = sum_j M[j][c] q_j.
 __device__ __forceinline__ float readout(const Bel& b, float qj) { return own_sum(b.M0 * qj, b.M1 * qj); }
-
-// Belief record offsets of lane (i, j) (bytes within one sequence's record).
-__device__ __forceinline__ uint32_t mean_off(int i, int j) { return static_cast<uint32_t>(j * 32 + i * 8); }
-__device__ __forceinline__ uint32_t cov_off(int i, int j) { return static_cast<uint32_t>(i * 16 + j * 4); }
 
 template <bool FIXED, int F>
 __global__ __launch_bounds__(kWave) void forward_kernel(FwdArgs a) {
@@ -476,54 +392,6 @@ __global__ __launch_bounds__(kWave) void forward_kernel(FwdArgs a) {
   store_ckpt(static_cast<uint32_t>(a.nb));
 }
 
-// ------------------------------------------------- two-wave forward (split)
-// At the smallest sequence counts the single-wave kernels leave SIMDs idle,
-// and each wave's time is its instruction stream.  The step splits into a
-// covariance half and a mean half that only talk one way: the mean update
-// needs the gain column bu_j = beta u_j, nothing else of the covariance
-// chain.  Here a workgroup of two waves holds the same 4 sequences: wave 0
-// runs the covariance chain (u, s, beta, P) one 16-token tile ahead and
-// leaves bu in LDS; wave 1 runs the innovations, the mean update and the
-// readouts of the tile before, from those bu.  One barrier per tile; each
-// wave stages and stores its own streams (wave 0: k, d, p, r, the covariance
-// checkpoints and final covariance; wave 1: v, q, the readouts, the mean
-// checkpoints and final mean).  The operations are those of forward_step, in
-// the same order, so the results are bitwise those of forward_kernel.
-struct STile {
-  // Input slot per sequence (3 slots: tile t + 1 lands while tiles t and
-  // t - 1 are read): k, d, q [TT][4], v [TT][8], p, r [TT].
-  static constexpr int K = 0, D = 64, Q = 128, V = 192, P = 320, R = 336, SEQ = 360, SLOT = SPW * SEQ;
-  // Readouts of a tile (2 slots) and the gain columns bu (2 slots).
-  static constexpr int YSEQ = 136, YSLOT = SPW * YSEQ, BSEQ = 72, BSLOT = SPW * BSEQ;
-  static constexpr int IN = 0, Y = 3 * SLOT, BU = Y + 2 * YSLOT, SIZE = BU + 2 * BSLOT;
-};
-
-// Covariance half of forward_step: P advanced, the gain column bu_j returned.
-__device__ __forceinline__ float cov_step(float& P, float ki, float kj, float di, float dj, float p, float r,
-                                          float delta, float floor) {
-  const float wki = di * ki, wkj = dj * kj;
-  const float zi = quad_sum(P * wkj);
-  const float zj = col_sum(P * wki);
-  const float ui = fmaf(di, zi, p * ki), uj = fmaf(dj, zj, p * kj);
-  const float s = quad_sum(kj * uj) + r;
-  const float beta = fast_rcp(fmaxf(s, floor));
-  const float bu = beta * uj;
-  const float dp = fmaf(p, delta, (di * dj) * P);
-  P = fmaf(-beta, ui * uj, dp);
-  return bu;
-}
-
-// Mean half (own order) and the readout of the lane's own column.
-__device__ __forceinline__ float mean_step(float& M0, float& M1, float kj, float dj, float qj, v2f v, float bu) {
-  const float wkj = dj * kj;
-  const float so = own_sum(M0 * wkj, M1 * wkj);
-  const float e0 = v[0] - so;
-  const float e1 = v[1] - dpp<kXor1>(so);
-  M0 = fmaf(bu, e0, dj * M0);
-  M1 = fmaf(bu, e1, dj * M1);
-  return own_sum(M0 * qj, M1 * qj);
-}
-
 // G groups of SPW sequences per workgroup, two waves each (covariance A, B,
 // then mean A, B): with G = 2 the four waves take the CU's four SIMDs, where
 // two two-wave workgroups on one CU leave a SIMD idle and make two waves share
@@ -623,50 +491,14 @@ __global__ __launch_bounds__(2 * G * kWave) void forward_split_kernel(FwdArgs a)
         float* bu = bu_slot(it);
         const int64_t t0 = it * TT;
         const int len = tile_len(it);
-        // Each token's inputs are read one token ahead, before the previous
-        // token's bu write (LDS reads may not pass that write).
-        struct In {
-          float ki, kj, di, dj, p, r;
-        };
-        auto read = [&](In& x, int tt) __attribute__((always_inline)) {
-          x.ki = b[STile::K + 4 * tt + i];
-          x.kj = b[STile::K + 4 * tt + j];
-          x.di = FIXED ? kFixedDecay : b[STile::D + 4 * tt + i];
-          x.dj = FIXED ? kFixedDecay : b[STile::D + 4 * tt + j];
-          x.p = FIXED ? kFixedProcess : b[STile::P + tt];
-          x.r = FIXED ? kFixedObservation : b[STile::R + tt];
-        };
-        auto ckpt_at = [&](int64_t t) __attribute__((always_inline)) {
-          if (t == next_ckpt) {
+        auto ckpt_at = [&](int tt) __attribute__((always_inline)) {
+          if (t0 + tt == next_ckpt) {
             r4::st32(rbc, P, cco, ckpt * 64u);
             ++ckpt;
             next_ckpt += a.chunk;
           }
         };
-        In cur, nxt;
-        read(cur, 0);
-        if (len == TT && a.chunk % 8 == 0) {
-          // Checkpoints can only fall on tokens 0 and 8 of a full tile: two
-          // straight 8-token runs.
-#pragma unroll
-          for (int h = 0; h < TT / 8; ++h) {
-            ckpt_at(t0 + 8 * h);
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-              const int tt = 8 * h + u;
-              if (tt + 1 < TT) read(nxt, tt + 1);
-              bu[4 * tt + j] = cov_step(P, cur.ki, cur.kj, cur.di, cur.dj, cur.p, cur.r, delta, a.floor);
-              cur = nxt;
-            }
-          }
-        } else {
-          for (int tt = 0; tt < len; ++tt) {
-            if (tt + 1 < len) read(nxt, tt + 1);
-            ckpt_at(t0 + tt);
-            bu[4 * tt + j] = cov_step(P, cur.ki, cur.kj, cur.di, cur.dj, cur.p, cur.r, delta, a.floor);
-            cur = nxt;
-          }
-        }
+        cov_tile<FIXED>(P, b, bu, i, j, len, len == TT && a.chunk % 8 == 0, delta, a.floor, ckpt_at);
       }
       __syncthreads();
     }
@@ -741,46 +573,13 @@ __global__ __launch_bounds__(2 * G * kWave) void forward_split_kernel(FwdArgs a)
         float* yb = y_slot(tl);
         const int64_t t0 = tl * TT;
         const int len = tile_len(tl);
-        struct In {
-          float kj, dj, qj, bu;
-          v2f v;
-        };
-        auto read = [&](In& x, int tt) __attribute__((always_inline)) {
-          x.kj = b[STile::K + 4 * tt + j];
-          x.dj = FIXED ? kFixedDecay : b[STile::D + 4 * tt + j];
-          x.qj = b[STile::Q + 4 * tt + j];
-          x.v[0] = b[STile::V + 8 * tt + co];
-          x.v[1] = b[STile::V + 8 * tt + (co ^ 1)];
-          x.bu = bu[4 * tt + j];
-        };
-        auto ckpt_at = [&](int64_t t) __attribute__((always_inline)) {
-          if (t == next_ckpt) {
+        auto ckpt_at = [&](int tt) __attribute__((always_inline)) {
+          if (t0 + tt == next_ckpt) {
             store_ckpt(ckpt++);
             next_ckpt += a.chunk;
           }
         };
-        In cur, nxt;
-        read(cur, 0);
-        if (len == TT && a.chunk % 8 == 0) {
-#pragma unroll
-          for (int h = 0; h < TT / 8; ++h) {
-            ckpt_at(t0 + 8 * h);
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-              const int tt = 8 * h + u;
-              if (tt + 1 < TT) read(nxt, tt + 1);
-              yb[8 * tt + co] = mean_step(M0, M1, cur.kj, cur.dj, cur.qj, cur.v, cur.bu);
-              cur = nxt;
-            }
-          }
-        } else {
-          for (int tt = 0; tt < len; ++tt) {
-            if (tt + 1 < len) read(nxt, tt + 1);
-            ckpt_at(t0 + tt);
-            yb[8 * tt + co] = mean_step(M0, M1, cur.kj, cur.dj, cur.qj, cur.v, cur.bu);
-            cur = nxt;
-          }
-        }
+        mean_tile<FIXED>(M0, M1, b, bu, yb, j, co, len, len == TT && a.chunk % 8 == 0, ckpt_at);
       }
       __syncthreads();
     }
@@ -1047,28 +846,6 @@ struct BTile {
   static constexpr int K = 0, D = 64, Q = 128, V = 192, GY = 320, P = 448, R = 464, SEQ = 488, SIZE = SPW * SEQ;
 };
 
-// Tokens len .. CAP - 1 of a sequence's LDS region (layout L) made neutral:
-// k = q = v = gy = 0, d = 1, p = 0, r = 1.  Their step leaves the belief as it
-// is (u = 0, e = 0) and their reverse leaves the carried adjoints as they are
-// (a = w = 0), bit for bit, so the unrolled chunks need no length test.  With
-// fixed dynamics d and p are constants and this does not hold for nonzero
-// carried adjoints: such calls (final-state gradients) take other kernels
-// when T ends inside a chunk.  Lane c of the sequence's 16.
-template <typename L, int CAP>
-__device__ __forceinline__ void neutral_tail(float* b, int len, int c) {
-  for (int t = len; t < CAP; ++t) {
-    if (c < 8) b[L::V + 8 * t + c] = b[L::GY + 8 * t + c] = 0.f;
-    if (c < 4) {
-      b[L::K + 4 * t + c] = b[L::Q + 4 * t + c] = 0.f;
-      b[L::D + 4 * t + c] = 1.f;
-    }
-    if (c == 0) {
-      b[L::P + t] = 0.f;
-      b[L::R + t] = 1.f;
-    }
-  }
-}
-
 struct BStage {
   v4f k, d, q, v0, v1, g0, g1, p, r;
 };
@@ -1209,15 +986,6 @@ __device__ __forceinline__ void read_ftok(Tok& x, const float* b, int tt, int i,
   }
 }
 
-// x at lane (i, i) of the row, given at every lane of quad i: the transpose
-// of a quantity indexed by the column j (constant down each column).
-__device__ __forceinline__ float diag_pick(float x, bool i1, bool i2) {
-  const float x0 = dpp<quad_perm(0, 0, 0, 0)>(x), x1 = dpp<quad_perm(1, 1, 1, 1)>(x);
-  const float x2 = dpp<quad_perm(2, 2, 2, 2)>(x), x3 = dpp<quad_perm(3, 3, 3, 3)>(x);
-  const float lo = i1 ? x1 : x0, hi = i1 ? x3 : x2;
-  return i2 ? hi : lo;
-}
-
 // Adjoint of one token, lane (i, j).  Carried: gM0, gM1 = dL/dM[j][2i],
 // dL/dM[j][2i + 1] and S = sym(dL/dP)[i][j], updated in place to their values
 // before the token.  With dL/dM_new including q gy^T (the equations of
@@ -1228,11 +996,6 @@ __device__ __forceinline__ float diag_pick(float x, bool i1, bool i2) {
 //   dL/dq = M_new gy,  H = S + sym(gu k^T)
 //   dL/dd = 2 (H * P_prev) d + sum_c (gM - k ge^T) * M_prev,  dL/dp = trace H
 //   S_prev = H * d d^T,  gM_prev = (gM - k ge^T) * d
-struct ROut {
-  float gk, gq, gd, gp, gs, gui, guj;
-  v2f ge;
-};
-
 template <bool DYN>
 __device__ __forceinline__ void reverse_step(const RTok& x, const Hist& h, float Mn0, float Mn1, float& gM0,
                                              float& gM1, float& S, float floor, float delta, bool i1, bool i2,
@@ -1270,11 +1033,6 @@ __device__ __forceinline__ void reverse_step(const RTok& x, const Hist& h, float
   o.ge[0] = ge0;
   o.ge[1] = ge1;
 }
-
-// What the initial-covariance adjoint needs of a sequence's first token.
-struct First {
-  float gui, guj, ki, kj, dd;
-};
 
 template <bool FIXED, bool DYN>
 __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
@@ -1433,105 +1191,6 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
   }
 }
 
-// ---------------------------------------------- three-wave backward (split)
-// A wave issues at most one instruction every ~6 cycles, so at the smallest
-// batches (one wave per SIMD or fewer) each wave's time is its instruction
-// count.  The backward splits three ways: the mean adjoint (gM, ge = dL/dv,
-// dL/dq) needs of the covariance side only u and beta; the covariance
-// adjoint (S, gu, dL/dk, dL/dd, dL/dp, dL/dr) needs of the mean side only
-// three column sums per token, a = gM e, A = M_prev ge and sum_c gb M_prev;
-// and the covariance replay feeds both.  A workgroup of three waves holds the
-// same 4 sequences and walks the checkpoint chunks (8 tokens) last to first
-// in steps, one barrier per step.  With x the chunk's position in that
-// order, at step x:
-//   wave 0 replays the covariance of chunk x (its records P, u, s go to
-//          LDS, and u_j and beta for the mean wave);
-//   wave 2 replays and reverses the mean of chunk x - 1 (from u and beta)
-//          and leaves the three sums;
-//   wave 1 reverses the covariance of chunk x - 2 (from the records and the
-//          sums).
-// Wave 0 also moves every stream of the loop: it stages k, d, p, r, q, v, gy
-// and both checkpoints one step ahead and stores the gradients (gq, gv one
-// step after wave 2 leaves them, gk, gd, gp, gr one step after wave 1), so
-// the two long waves never wait for global memory (a wait for loads is also a
-// wait for the stores issued with them).  The operations are those of
-// backward_kernel in its order: the results are bitwise the same.
-struct SBTile {
-  static constexpr int CH = 8;
-  // Chunk slot per sequence (5 slots: a chunk is staged one step before its
-  // replay and its last gradients leave three steps after): k, d, q [CH][4],
-  // v, gy [CH][8], p, r [CH], and the mean checkpoint (2 per lane).
-  static constexpr int K = 0, D = 32, Q = 64, V = 96, GY = 160, P = 224, R = 232, MC = 264, SEQ = 296,
-                       SLOT = SPW * SEQ;
-  static constexpr int NSLOT = 5;
-  // Covariance to mean (2 slots): u_j [CH][4], beta [CH].
-  static constexpr int USEQ = 40, USLOT = SPW * USEQ;
-  // Mean to covariance (2 slots): a, A, sum_c gb M_prev [CH][4] each.
-  static constexpr int ASEQ = 104, ASLOT = SPW * ASEQ;
-  // Covariance records (3 slots: written at step x, read at step x + 2):
-  // [CH][64 lanes] of (P, u_i, u_j, s).
-  static constexpr int RSLOT = CH * kWave * 4;
-  static constexpr int IN = 0, U = NSLOT * SLOT, A = U + 2 * USLOT, REC = A + 2 * ASLOT, SIZE = REC + 3 * RSLOT;
-};
-
-// Covariance record of one replayed token (one 16-byte LDS word per lane).
-struct PRec {
-  float P, ui, uj, s;
-};
-__device__ __forceinline__ v4f pack(const PRec& r) { return v4f{r.P, r.ui, r.uj, r.s}; }
-__device__ __forceinline__ PRec unpack(v4f x) { return PRec{x[0], x[1], x[2], x[3]}; }
-// Mean record of one replayed token (record order, as backward_kernel).
-struct MRec {
-  float M0, M1;
-  v2f e;
-};
-
-// Mean half of the reverse (reverse_step's gM, ge, a, A, C, gb, Bv).
-template <bool DYN>
-__device__ __forceinline__ void mean_reverse(float kj, float dj, float qj, v2f gy, const MRec& h, float uj, float beta,
-                                             float Mn0, float Mn1, float& gM0, float& gM1, float& a_out,
-                                             float& A_out, float& Bv_out, float& gq, float& ge0, float& ge1) {
-  gM0 = fmaf(qj, gy[0], gM0);
-  gM1 = fmaf(qj, gy[1], gM1);
-  ge0 = beta * quad_sum(gM0 * uj);
-  ge1 = beta * quad_sum(gM1 * uj);
-  a_out = col_sum(fmaf(gM1, h.e[1], gM0 * h.e[0]));
-  A_out = col_sum(fmaf(h.M1, ge1, h.M0 * ge0));
-  gq = col_sum(fmaf(Mn1, gy[1], Mn0 * gy[0]));
-  const float gb0 = fmaf(-kj, ge0, gM0), gb1 = fmaf(-kj, ge1, gM1);
-  gM0 = gb0 * dj;
-  gM1 = gb1 * dj;
-  Bv_out = DYN ? col_sum(fmaf(gb1, h.M1, gb0 * h.M0)) : 0.f;
-}
-
-// Covariance half of the reverse (reverse_step's w, z, gs, gu, gk, H, gd,
-// gp, S).
-template <bool DYN>
-__device__ __forceinline__ void cov_reverse(float ki, float kj, float di, float dj, float p, const PRec& h, float a,
-                                            float A, float Bv, float& S, float floor, float delta, bool i1, bool i2,
-                                            ROut& o) {
-  const float beta = fast_rcp(fmaxf(h.s, floor));
-  const float w = col_sum(S * h.ui);
-  const float z = quad_sum(h.uj * (a - w));
-  const float gs = h.s > floor ? -z * beta * beta : 0.f;
-  const float guj = fmaf(beta, fmaf(-2.f, w, a), gs * kj);
-  const float gui = diag_pick(guj, i1, i2);
-  const float dd = di * dj;
-  const float pb = fmaf(p, delta, dd * h.P);
-  o.gk = fmaf(-dj, A, gs * h.uj) + col_sum(pb * gui);
-  const float H = fmaf(0.5f, gui * kj + guj * ki, S);
-  if constexpr (DYN) {
-    o.gd = fmaf(2.f, col_sum((H * di) * h.P), Bv);
-    o.gp = col_sum(quad_sum(delta * H));
-  } else {
-    o.gd = o.gp = 0.f;
-  }
-  S = H * dd;
-  o.gs = gs;
-  o.gui = gui;
-  o.guj = guj;
-}
-
 // G groups of SPW sequences per workgroup, three waves each, one barrier for
 // all.  A workgroup's waves go to the CU's SIMDs in the cyclic order 0, 2, 1,
 // 3 (an HW_ID probe on MI355X), and two workgroups on one CU start at varying
@@ -1681,9 +1340,6 @@ __global__ __launch_bounds__(3 * G * kWave) void backward_split_kernel(BwdArgs a
       if (nb > 1) load(1);
     }
     __syncthreads();
-    struct In {
-      float ki, kj, di, dj, p, r;
-    };
     for (int64_t x = 0; x <= nb + 1; ++x) {
       r4::vm_wait<0>();
       float Pc = Pload;
@@ -1695,48 +1351,13 @@ __global__ __launch_bounds__(3 * G * kWave) void backward_split_kernel(BwdArgs a
       if (x >= 2) store_mean(x - 2);
       if (x >= 3) store_cov(x - 3);
       if (x < nb) {
-        const float* pb = slot(x);
-        float* ub = uslot(x);
-        float* rec = rslot(x);
-        auto read = [&](In& y, int k) __attribute__((always_inline)) {
-          y.ki = pb[SBTile::K + 4 * k + i];
-          y.kj = pb[SBTile::K + 4 * k + j];
-          y.di = FIXED ? kFixedDecay : pb[SBTile::D + 4 * k + i];
-          y.dj = FIXED ? kFixedDecay : pb[SBTile::D + 4 * k + j];
-          y.p = FIXED ? kFixedProcess : pb[SBTile::P + k];
-          y.r = FIXED ? kFixedObservation : pb[SBTile::R + k];
-        };
-        In cur, nxt;
-        read(cur, 0);
-#pragma unroll
-        for (int k = 0; k < CH; ++k) {
-          if (k + 1 < CH) read(nxt, k + 1);
-          // forward_step's covariance operations, in its order.
-          PRec h;
-          h.P = Pc;
-          const float wki = cur.di * cur.ki, wkj = cur.dj * cur.kj;
-          const float zi = quad_sum(Pc * wkj);
-          const float zj = col_sum(Pc * wki);
-          const float ui = fmaf(cur.di, zi, cur.p * cur.ki), uj = fmaf(cur.dj, zj, cur.p * cur.kj);
-          const float sv = quad_sum(cur.kj * uj) + cur.r;
-          const float beta = fast_rcp(fmaxf(sv, a.floor));
-          const float dp = fmaf(cur.p, delta, (cur.di * cur.dj) * Pc);
-          Pc = fmaf(-beta, ui * uj, dp);
-          h.ui = ui;
-          h.uj = uj;
-          h.s = sv;
-          *reinterpret_cast<v4f*>(rec + k * 4 * kWave) = pack(h);
-          ub[4 * k + j] = uj;
-          ub[4 * CH + k] = beta;
-          cur = nxt;
-        }
+        replay_chunk<FIXED>(Pc, slot(x), uslot(x), rslot(x), i, j, delta, a.floor);
       }
       __syncthreads();
     }
     if (nb > 0) store_cov(nb - 1);
   } else if (role == 1) {
     // ------------------------------------------------ covariance reverse wave
-    const bool i1 = (i & 1) != 0, i2 = (i & 2) != 0;
     const uint32_t cvo = static_cast<uint32_t>(s) * 64u + cov_off(i, j);
     float S;
     {
@@ -1747,49 +1368,9 @@ __global__ __launch_bounds__(3 * G * kWave) void backward_split_kernel(BwdArgs a
     }
     First first = {0.f, 0.f, 0.f, 0.f, 0.f};
     __syncthreads();
-    struct In {
-      float ki, kj, di, dj, p, a, A, Bv;
-      v4f rec;
-    };
     for (int64_t x = 0; x <= nb + 1; ++x) {
       if (x >= 2) {
-        float* rb = slot(x - 2);
-        const float* ab = aslot(x - 2);
-        const float* rec = rslot(x - 2);
-        auto read = [&](In& y, int u) __attribute__((always_inline)) {
-          y.ki = rb[SBTile::K + 4 * u + i];
-          y.kj = rb[SBTile::K + 4 * u + j];
-          y.di = FIXED ? kFixedDecay : rb[SBTile::D + 4 * u + i];
-          y.dj = FIXED ? kFixedDecay : rb[SBTile::D + 4 * u + j];
-          y.p = FIXED ? kFixedProcess : rb[SBTile::P + u];
-          y.a = ab[4 * u + j];
-          y.A = ab[4 * CH + 4 * u + j];
-          y.Bv = DYN ? ab[8 * CH + 4 * u + j] : 0.f;
-          y.rec = *reinterpret_cast<const v4f*>(rec + u * 4 * kWave);
-        };
-        In cur, nxt;
-        read(cur, CH - 1);
-#pragma unroll
-        for (int u = CH - 1; u >= 0; --u) {
-          if (u > 0) read(nxt, u - 1);
-          ROut o;
-          cov_reverse<DYN>(cur.ki, cur.kj, cur.di, cur.dj, cur.p, unpack(cur.rec), cur.a, cur.A, cur.Bv, S, a.floor,
-                           delta, i1, i2, o);
-          rb[SBTile::K + 4 * u + j] = o.gk;
-          if constexpr (DYN) {
-            rb[SBTile::D + 4 * u + j] = o.gd;
-            rb[SBTile::P + u] = o.gp;
-            rb[SBTile::R + u] = o.gs;
-          }
-          if (u == 0) {
-            first.gui = o.gui;
-            first.guj = o.guj;
-            first.ki = cur.ki;
-            first.kj = cur.kj;
-            first.dd = cur.di * cur.dj;
-          }
-          cur = nxt;
-        }
+        reverse_chunk<FIXED, DYN>(S, first, slot(x - 2), aslot(x - 2), rslot(x - 2), i, j, delta, a.floor);
       }
       __syncthreads();
     }
@@ -1812,59 +1393,7 @@ __global__ __launch_bounds__(3 * G * kWave) void backward_split_kernel(BwdArgs a
     __syncthreads();
     for (int64_t x = 0; x <= nb + 1; ++x) {
       if (x >= 1 && x <= nb) {
-        float* b = slot(x - 1);
-        const float* ub = uslot(x - 1);
-        float* ab = aslot(x - 1);
-        MRec h[CH];
-        const v2f Mc = *reinterpret_cast<const v2f*>(b + SBTile::MC + 2 * c);  // checkpoint of the chunk
-        float M0 = Mc[0], M1 = Mc[1];
-#pragma unroll
-        for (int k = 0; k < CH; ++k) {
-          const float kj = b[SBTile::K + 4 * k + j];
-          const float dj = FIXED ? kFixedDecay : b[SBTile::D + 4 * k + j];
-          const v2f v = *reinterpret_cast<const v2f*>(b + SBTile::V + 8 * k + 2 * i);
-          const float uj = ub[4 * k + j], beta = ub[4 * CH + k];
-          // forward_step's mean operations, in its order.
-          h[k].M0 = M0;
-          h[k].M1 = M1;
-          const float wkj = dj * kj;
-          const float e0 = v[0] - quad_sum(M0 * wkj);
-          const float e1 = v[1] - quad_sum(M1 * wkj);
-          const float bu = beta * uj;
-          M0 = fmaf(bu, e0, dj * M0);
-          M1 = fmaf(bu, e1, dj * M1);
-          h[k].e[0] = e0;
-          h[k].e[1] = e1;
-        }
-        struct In {
-          float kj, dj, qj, uj, beta;
-          v2f gy;
-        };
-        auto read = [&](In& y, int u) __attribute__((always_inline)) {
-          y.kj = b[SBTile::K + 4 * u + j];
-          y.dj = FIXED ? kFixedDecay : b[SBTile::D + 4 * u + j];
-          y.qj = b[SBTile::Q + 4 * u + j];
-          y.gy = *reinterpret_cast<const v2f*>(b + SBTile::GY + 8 * u + 2 * i);
-          y.uj = ub[4 * u + j];
-          y.beta = ub[4 * CH + u];
-        };
-        In cur, nxt;
-        read(cur, CH - 1);
-#pragma unroll
-        for (int u = CH - 1; u >= 0; --u) {
-          if (u > 0) read(nxt, u - 1);
-          const float Mn0 = u < CH - 1 ? h[u < CH - 1 ? u + 1 : u].M0 : M0;
-          const float Mn1 = u < CH - 1 ? h[u < CH - 1 ? u + 1 : u].M1 : M1;
-          float av, Av, Bv, gq, ge0, ge1;
-          mean_reverse<DYN>(cur.kj, cur.dj, cur.qj, cur.gy, h[u], cur.uj, cur.beta, Mn0, Mn1, gM0, gM1, av, Av, Bv,
-                            gq, ge0, ge1);
-          ab[4 * u + j] = av;
-          ab[4 * CH + 4 * u + j] = Av;
-          if constexpr (DYN) ab[8 * CH + 4 * u + j] = Bv;
-          b[SBTile::Q + 4 * u + j] = gq;
-          b[SBTile::V + 8 * u + 2 * i + (j & 1)] = (j & 1) ? ge1 : ge0;
-          cur = nxt;
-        }
+        mean_chunk<FIXED, DYN>(gM0, gM1, slot(x - 1), uslot(x - 1), aslot(x - 1), i, j, c);
       }
       __syncthreads();
     }

@@ -407,6 +407,14 @@ int bssm_associative_static_scan_backward(const float* keys, const float* values
  * otherwise BSSM_ERR_UNSUPPORTED.  No counterpart in the reference library:
  * its mixer materialises every transformed and permuted tensor in float32. */
 #define BSSM_ANY_SHAPE ((int64_t)1 << 32)
+/* Or-ed into chunk: the small-batch kernels (a workgroup per 4 heads, another
+ * rounding).  grad_norm_weight_partials then has 4 B * ceil(H / 16) rows, all
+ * written.  bssm_mixer_row_kernels says where they are the faster ones (1, else
+ * 0): off whole tiles (H % 16 or T % 4 not 0), up to twice the forward's and
+ * three times the backward's limit of bssm_small_batch_limit(2) and (3) in
+ * B * H. */
+#define BSSM_ROW_KERNELS ((int64_t)1 << 33)
+int bssm_mixer_row_kernels(int backward, int64_t batch, int64_t t, int64_t heads);
 int bssm_mixer_forward(const void* q_proj, int64_t ldq, const void* k_proj, int64_t ldk,
                        const void* v_proj, int64_t ldv, const void* decay_logits, int64_t ldd,
                        const void* noise, int64_t ldn,

@@ -69,8 +69,20 @@ def test_core_matches_oracle(cuda_device, monkeypatch, b, t, h, final_grads):
         _bf16_close(got, want.reshape(got.shape), what)
 
 
+@pytest.fixture
+def large_batch_kernels():
+    """The small-batch kernels (test_gpu_mixer_row.py), which round differently, off."""
+    from bayes_ssm import _hip
+
+    lib = _hip.load()
+    old = [lib.bssm_small_batch_limit(d, 0) for d in (2, 3)]
+    yield
+    for d, n in zip((2, 3), old):
+        lib.bssm_small_batch_limit(d, n)
+
+
 @pytest.mark.parametrize("b,t,h", SHAPES)
-def test_readout_is_the_whole_tile_kernels(cuda_device, monkeypatch, b, t, h):
+def test_readout_is_the_whole_tile_kernels(cuda_device, monkeypatch, large_batch_kernels, b, t, h):
     """Bit for bit the whole-tile kernels on inputs padded with zeros to a multiple of 16 heads and of 4 tokens: heads
     are independent, and tokens past T whose gradient is zero leave the others' results alone."""
     from bayes_ssm import mixer

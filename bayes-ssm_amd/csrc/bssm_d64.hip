@@ -8,8 +8,7 @@
 // checkpoint interval kBlk = kD64Checkpoint = 8, bssm_recurrence.h): a
 // workgroup of W waves per sequence, thread (w, l) holding 64 / W columns of
 // covariance row l and the same rows of mean column l; row sums over j are W
-// partial sums exchanged through LDS, sums over lanes go through a
-// wave-private LDS transpose.  Inputs are staged per 8-token block through
+// partial sums exchanged through LDS, sums over lanes stay in registers.  Inputs are staged per 8-token block through
 // LDS.  The backward replays each chunk once, its history in registers.
 //
 // One wave per sequence (the backward at other chunks): lane l owns row l of
@@ -543,7 +542,7 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
 // carried by all W waves with identical bits.  Sums over j of a row
 // (P~ wk, M^T wk, M^T q, ...) are W partial sums exchanged through LDS (one
 // barrier) and added in the same order by every wave; sums over the lanes of
-// a wave's KB rows go through a wave-private LDS transpose.  u_j and gu_j of
+// a wave's KB rows are a reduce-scatter in registers.  u_j and gu_j of
 // J_w are read from their lanes (v_readlane).
 //
 // Inputs are staged per block of kBlk tokens in a double-buffered LDS stage,
@@ -600,39 +599,32 @@ __device__ __forceinline__ float tree(const float (&x)[W]) {
   else return ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
 }
 
-// Sum over the wave's 64 lanes of each of the lane's KB values x[ii]: the
-// total of row ii lands in the G = 64 / KB lanes G ii .. G ii + G - 1.
-// `tile` is wave-private, 64 rows of KB floats with the 16-byte pieces of row
-// r permuted by tile_rot(r): the 16-byte row writes of any 8 (or 16)
-// consecutive lanes then cover all 32 (64) banks, and the column reads of a
-// row sum touch 64 consecutive words.  A wave's LDS operations complete in
-// issue order, so no barrier separates the writes from the reads.
-template <int KB>
-__device__ __forceinline__ int tile_rot(int r) {
-  return ((r >> 1) ^ (r >> 3)) & (KB / 4 - 1);
-}
-template <int KB>
-__device__ __forceinline__ float lane_rowsum(float* tile, int l, const float (&x)[KB]) {
-  constexpr int G = kWave / KB, NP = KB / 4;
-  float* row = tile + l * KB;
-  const int rot = tile_rot<KB>(l);
+// Sum over the wave's 64 lanes of each of the lane's eight values x[ii]: the
+// total of row ii lands in the lanes 8 ii .. 8 ii + 7.  A reduce-scatter in
+// registers: the row swaps hand half of the rows to the lanes 32 (16) away,
+// an exchange by 8 halves them again, three DPP steps add the last eight
+// lanes.  18 VALU instructions and no LDS; a transpose through LDS took 12 and
+// 10 LDS instructions with bank conflicts (four of these sums a token were
+// 60 % of the backward's LDS instructions).
+__device__ __forceinline__ float lane_rowsum(const float (&x)[8], int l) {
+  float y[8];
 #pragma unroll
-  for (int c = 0; c < NP; ++c)
-    *reinterpret_cast<v4f*>(&row[4 * (c ^ rot)]) = v4f{x[4 * c], x[4 * c + 1], x[4 * c + 2], x[4 * c + 3]};
-  __builtin_amdgcn_wave_barrier();
-  const int ii = l / G, g = l % G;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < 8; ++i) y[i] = x[i];
+  asm volatile(
+      "s_nop 1\n\tv_permlane32_swap_b32 %0, %4\n\tv_permlane32_swap_b32 %1, %5\n\t"
+      "v_permlane32_swap_b32 %2, %6\n\tv_permlane32_swap_b32 %3, %7"
+      : "+v"(y[0]), "+v"(y[1]), "+v"(y[2]), "+v"(y[3]), "+v"(y[4]), "+v"(y[5]), "+v"(y[6]), "+v"(y[7]));
 #pragma unroll
-  for (int m = 0; m < KB; ++m) {
-    const int r = G * m + g;
-    acc[m & 3] += tile[r * KB + 4 * ((ii >> 2) ^ tile_rot<KB>(r)) + (ii & 3)];
-  }
-  __builtin_amdgcn_wave_barrier();
-  float t = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+  for (int i = 0; i < 4; ++i) y[i] += y[i + 4];  // rows i | i + 4 by the half wave
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %2\n\tv_permlane16_swap_b32 %1, %3"
+               : "+v"(y[0]), "+v"(y[1]), "+v"(y[2]), "+v"(y[3]));
+#pragma unroll
+  for (int i = 0; i < 2; ++i) y[i] += y[i + 2];
+  const bool odd = (l & 8) != 0;
+  float t = (odd ? y[1] : y[0]) + dpp<0x128>(odd ? y[0] : y[1]);  // row_ror:8
   t = add_rn(t, dpp<kXor1>(t));
   t = add_rn(t, dpp<kXor2>(t));
-  if constexpr (G == 8) t = add_rn(t, dpp<kHalfMirror>(t));
-  return t;
+  return add_rn(t, dpp<kHalfMirror>(t));
 }
 
 // LDS stage of one block (floats): rows of k, v, q, gy, d (kBlk x 64 each),
@@ -957,18 +949,17 @@ __global__ __launch_bounds__(W * kWave) void forward_group_kernel(FwdArgs a) {
 // registers, then reversed token by token (the reverse of
 // persistent_bayes_chunked.cu:303-343 in the conventions of the one-wave
 // kernel above: symmetrized gu k^T adjoint, first-token mirror correction).
-// Barriers per token: one in the replay, two in the reverse.
+// Barriers per token: one in the replay, one in the reverse, and one per chunk.
 template <int W, bool FIXED, bool DYN>
 __global__ __launch_bounds__(W * kWave) __attribute__((amdgpu_waves_per_eu(W / 4, W / 4)))
 void backward_group_kernel(BwdArgs a) {
   constexpr int KB = D / W, NT = W * kWave, G = kWave / KB;
   __shared__ v2f xz[2][W * kWave];
-  __shared__ v2f xb[W * kWave], xc[W * kWave];
-  __shared__ float ra[D], rkm[D], rdm[D];
-  __shared__ __attribute__((aligned(16))) float tiles[W * kWave * KB];
+  // Of the reverse, double-buffered by the token: one barrier per token.
+  __shared__ v2f xb[2][W * kWave], xc[2][W * kWave];
+  __shared__ float ra[2][D], rkm[2][D], rdm[2][D];
   __shared__ __attribute__((aligned(16))) float stage[2][kStage];
   const int tid = static_cast<int>(threadIdx.x), w = wave_index(), l = tid & (kWave - 1), j0 = KB * w;
-  float* tile = tiles + w * kWave * KB;
   const int64_t n = blockIdx.x;
   const int T = static_cast<int>(a.t);
   const int64_t nbp = a.nb + 1;
@@ -1073,6 +1064,27 @@ void backward_group_kernel(BwdArgs a) {
           }
         }
       }
+      // Phase 3 of token t: dL/dk and dL/dd from the partials that its phase 2
+      // left (P' gu = 2 P' hg) and the lane's own terms gk0 and gd0.  Nothing of
+      // it is carried, so it runs behind the next token's barrier instead of
+      // one of its own.
+      float gk0 = 0.f, gd0 = 0.f;
+      auto finish = [&](int t, int buf) __attribute__((always_inline)) {
+        if (w != 0) return;
+        float pgs[W], gds[W];
+#pragma unroll
+        for (int i = 0; i < W; ++i) {
+          const v2f v = xc[buf][i * kWave + l];
+          pgs[i] = v[0];
+          gds[i] = v[1];
+        }
+        gkp[t * D + l] = fmaf(2.f, tree<W>(pgs), gk0) - rkm[buf][l];
+        if constexpr (DYN) {
+          if (gdp) gdp[t * D + l] = fmaf(2.f, gd0 + tree<W>(gds), rdm[buf][l]);
+        } else {
+          if (gdp) gdp[t * D + l] = 0.f;
+        }
+      };
 #pragma unroll
       for (int tt = HI - 1; tt >= LO; --tt) {
         if (tt < len) {
@@ -1101,13 +1113,14 @@ void backward_group_kernel(BwdArgs a) {
             va[ii] = gM[ii] * o.e;
           }
           {
-            const float rq = lane_rowsum<KB>(tile, l, vq);
+            const float rq = lane_rowsum(vq, l);
             if (l % G == 0) gqp[t * D + j0 + l / G] = rq;
-            const float r_a = lane_rowsum<KB>(tile, l, va);
-            if (l % G == 0) ra[j0 + l / G] = r_a;
+            const float r_a = lane_rowsum(va, l);
+            if (l % G == 0) ra[tt & 1][j0 + l / G] = r_a;
           }
-          xb[w * kWave + l] = v2f{(am[0] + am[1]) + (am[2] + am[3]), (aw[0] + aw[1]) + (aw[2] + aw[3])};
+          xb[tt & 1][w * kWave + l] = v2f{(am[0] + am[1]) + (am[2] + am[3]), (aw[0] + aw[1]) + (aw[2] + aw[3])};
           __syncthreads();
+          if (tt + 1 < HI && tt + 1 < len) finish(t + 1, (tt + 1) & 1);
           // Phase 2: ge, gs, gu; row sums of (d M) ge and (gM - k ge^T) M;
           // partials of P' gu and of the decay's covariance term.  gu enters
           // halved (hg = gu / 2, exact), which gives the symmetrized outer
@@ -1115,12 +1128,12 @@ void backward_group_kernel(BwdArgs a) {
           float gms[W], ws[W];
 #pragma unroll
           for (int i = 0; i < W; ++i) {
-            const v2f v = xb[i * kWave + l];
+            const v2f v = xb[tt & 1][i * kWave + l];
             gms[i] = v[0];
             ws[i] = v[1];
           }
           const float gmu = tree<W>(gms), wl = tree<W>(ws);
-          const float a_l = ra[l];
+          const float a_l = ra[tt & 1][l];
           const float ge = o.beta * gmu;
           const float z = wave_total(fmaf(o.e, gmu, -(o.u * wl)));
           const float gs = o.clamped ? 0.f : -z * o.beta * o.beta;
@@ -1135,11 +1148,11 @@ void backward_group_kernel(BwdArgs a) {
             gM[ii] = g * x.dJ[ii];
           }
           {
-            const float r_k = lane_rowsum<KB>(tile, l, vk);
-            if (l % G == 0) rkm[j0 + l / G] = r_k;
+            const float r_k = lane_rowsum(vk, l);
+            if (l % G == 0) rkm[tt & 1][j0 + l / G] = r_k;
             if constexpr (DYN) {
-              const float r_d = lane_rowsum<KB>(tile, l, vd);
-              if (l % G == 0) rdm[j0 + l / G] = r_d;
+              const float r_d = lane_rowsum(vd, l);
+              if (l % G == 0) rdm[tt & 1][j0 + l / G] = r_d;
             }
           }
           float ap[4] = {0.f, 0.f, 0.f, 0.f}, gdc = 0.f;
@@ -1157,43 +1170,24 @@ void backward_group_kernel(BwdArgs a) {
           }
           const float hd = add_rn(Sd, add_rn(mul_rn(hg, x.k), mul_rn(hg, x.k)));
           Sd = hd * mul_rn(x.d, x.d);
-          xc[w * kWave + l] = v2f{(ap[0] + ap[1]) + (ap[2] + ap[3]), gdc};
-          if (tt == 0 && c > 0) {  // publish the next chunk's stage
-            if (!FIXED && tid < 2 * kBlk) stage[(c - 1) & 1][kSP + tid] = pr;
-            r4::vm_wait<0>();
-          }
-          __syncthreads();
-          // Phase 3: dL/dk, dL/dd, dL/dp, dL/dr of the token (P' gu = 2 P' hg).
-          float pgs[W], gds[W];
-#pragma unroll
-          for (int i = 0; i < W; ++i) {
-            const v2f v = xc[i * kWave + l];
-            pgs[i] = v[0];
-            gds[i] = v[1];
-          }
-          const float pgu = 2.f * tree<W>(pgs);
-          const float gk = -rkm[l] + fmaf(gs, o.u, fmaf(fmaf(hbt.pd, mul_rn(x.d, x.d), x.p), gu, pgu));
+          xc[tt & 1][w * kWave + l] = v2f{(ap[0] + ap[1]) + (ap[2] + ap[3]), gdc};
+          gk0 = fmaf(gs, o.u, fmaf(hbt.pd, mul_rn(x.d, x.d), x.p) * gu);
+          gd0 = hd * hbt.pd * x.d;
+          const float gp = DYN ? wave_total(hd) : 0.f;
           if (w == 0) {
-            gkp[t * D + l] = gk;
             gvp[t * D + l] = ge;
-          }
-          if constexpr (DYN) {
-            const float gdl = fmaf(hd * hbt.pd, x.d, tree<W>(gds));
-            const float gd = fmaf(2.f, gdl, rdm[l]);
-            const float gp = wave_total(hd);
-            if (w == 0) {
-              if (gdp) gdp[t * D + l] = gd;
-              if (l == 0) {
-                if (gpp) gpp[t] = gp;
-                if (grp) grp[t] = gs;
-              }
-            }
-          } else if (w == 0) {
-            if (gdp) gdp[t * D + l] = 0.f;
             if (l == 0) {
-              if (gpp) gpp[t] = 0.f;
-              if (grp) grp[t] = 0.f;
+              if (gpp) gpp[t] = gp;
+              if (grp) grp[t] = DYN ? gs : 0.f;
             }
+          }
+          if (tt == 0) {  // publish the next chunk's stage
+            if (c > 0) {
+              if (!FIXED && tid < 2 * kBlk) stage[(c - 1) & 1][kSP + tid] = pr;
+              r4::vm_wait<0>();
+            }
+            __syncthreads();
+            finish(t, 0);
           }
         }
       }

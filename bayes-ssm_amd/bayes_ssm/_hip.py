@@ -66,6 +66,7 @@ _SIGNATURES = {
     "bssm_rotation_checkpoint": [_I],
     "bssm_small_batch_limit": [_I, _L],
     "bssm_forward_chunked_rotation": [_I, _I] + [_P] * 9 + [_P] * 5 + [_L, _L, _L, _F, _P],
+    "bssm_forward_chunked_rotation_checked": [_I, _I] + [_P] * 9 + [_P] * 5 + [_L, _L, _L, _F, _P, _P, _P],
     "bssm_backward_chunked_rotation": [_I, _I] + [_P] * 9 + [_P] * 5 + [_P] * 9 + [_L, _L, _L, _F, _P],
     "bssm_causal_conv4_forward": [_I, _P, _L, _P, _P, _L, _L, _L, _P],
     "bssm_causal_conv4_backward": [_I, _P, _L, _P, _P, _P, _P, _L, _L, _L, _P],

@@ -150,6 +150,10 @@ class _DeferredChecks:
             return
         self._pending.append((name, kind, x.detach()))
 
+    @property
+    def pending(self) -> bool:
+        return bool(self._pending)
+
     def finite(self, x: Tensor, name: str) -> None:
         self._add(x, name, None)
 
@@ -163,13 +167,19 @@ class _DeferredChecks:
             return
         self._pending.append((message, torch.tensor(float(bound), dtype=x.dtype).item(), x.detach()))
 
-    def flush(self) -> None:
+    def flush(self, probe=None) -> None:
+        """``probe``: a ``RotationProbe`` whose kernel may have checked the tensors of its names already."""
         pending, self._pending = self._pending, []
         if not pending:
             return
+        bits = probe.BITS if probe is not None and probe.checked else {}
         rows: dict[torch.device, list[tuple[int, Tensor]]] = {}
         fused: dict[torch.device, list[int]] = {}
-        for i, (_, kind, x) in enumerate(pending):
+        if bits:
+            rows[probe.faults.device] = [(-1, probe.faults.double().expand(3))]
+        for i, (name, kind, x) in enumerate(pending):
+            if name in bits:
+                continue
             # The kernel keeps float64 values only to float32 precision (signs exact): a float64 lower bound
             # other than zero is tested on torch's exact minimum.
             if _stats_kernel_takes(x) and not (isinstance(kind, float) and x.dtype == torch.float64):
@@ -184,9 +194,18 @@ class _DeferredChecks:
                 out = _device_value_stats([pending[i][2] for i in part]).double()
                 rows.setdefault(dev, []).extend((i, out[j]) for j, i in enumerate(part))
         values: list = [None] * len(pending)
+        faults = 0
         for entries in rows.values():
             for (i, _), triple in zip(entries, torch.stack([t for _, t in entries]).tolist()):
-                values[i] = triple
+                if i < 0:
+                    faults = int(triple[0])
+                else:
+                    values[i] = triple
+        for i, (name, _, _) in enumerate(pending):
+            if name in bits:
+                bad, sign = bits[name]
+                lo = -1.0 if faults & sign else 1.0
+                values[i] = (lo, lo, float(faults & bad))
         for (name, kind, _), (lo, hi, bad) in zip(pending, values):
             finite = not bad and math.isfinite(lo) and math.isfinite(hi)
             if isinstance(kind, float):
@@ -602,14 +621,16 @@ def bayesian_layer(
                                       denominator_floor=floor)
         if rotation:
             if device.type == "cuda" and len(batch_shape) == 1 and t > 0:
-                from .fused_cuda import fused_rotation_bayesian
+                from .fused_cuda import RotationProbe, fused_rotation_bayesian
 
+                probe = RotationProbe(device) if checks.pending else None
                 fused = fused_rotation_bayesian(keys, values, queries,
                                                 rotation_radii.expand(*batch_shape, t, d // 2),
                                                 rotation_angles.expand(*batch_shape, t, d // 2), process_variances,
-                                                observation_variances, mean, cov, denominator_floor=floor)
+                                                observation_variances, mean, cov, denominator_floor=floor,
+                                                _probe=probe)
                 if fused is not None:
-                    checks.flush()
+                    checks.flush(probe)
                     return fused
             checks.flush()
             outs = []

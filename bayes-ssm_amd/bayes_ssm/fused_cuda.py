@@ -39,6 +39,7 @@ way.  Other shapes widen first and take the float32 path.
 """
 from __future__ import annotations
 
+import ctypes
 import os
 from typing import Optional
 
@@ -567,6 +568,19 @@ def fused_diagonal_bayesian(
     )
 
 
+class RotationProbe:
+    """The rotation forward's value checks: ``checked`` tells whether its kernel made them, ``faults`` (int32 [1] on the
+    device) holds their bits then (``bssm_forward_chunked_rotation_checked``)."""
+
+    # Argument name -> (bit of an entry that is not finite, bit of a variance of the wrong sign).
+    BITS = {"keys": (1, 0), "values": (2, 0), "queries": (4, 0), "rotation_radii": (8, 0), "rotation_angles": (16, 0),
+            "process_variances": (32, 128), "observation_variances": (64, 256)}
+
+    def __init__(self, device: torch.device) -> None:
+        self.faults = torch.zeros(1, device=device, dtype=torch.int32)
+        self.checked = False
+
+
 class _ChunkedRotationFunction(torch.autograd.Function):
     """Rotation dynamics on the HIP kernels (C ABI ``bssm_*_chunked_rotation``).
 
@@ -577,10 +591,11 @@ class _ChunkedRotationFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, keys, values, queries, radii, angles, process, observation, initial_mean, initial_covariance,
-                denominator_floor):
+                denominator_floor, probe=None):
         n, t, d = keys.shape
         m = values.shape[-1]
         interval = int(_hip.load().bssm_rotation_checkpoint(d))
+        checked = ctypes.c_int(0)
         nb = -(-t // interval)
         dev = keys.device
         out = torch.empty(n, t, m, device=dev, dtype=torch.float32)
@@ -590,9 +605,12 @@ class _ChunkedRotationFunction(torch.autograd.Function):
         bcov = torch.empty(n, nb + 1, d, d, device=dev, dtype=torch.float32)
         P = _hip.ptr
         with _hip.on_device(dev):
-            _hip.call("bssm_forward_chunked_rotation", d, m, P(keys), P(values), P(queries), P(radii), P(angles),
-                      P(process), P(observation), P(initial_mean), P(initial_covariance), P(out), P(mean_t),
-                      P(cov_t), P(bmean), P(bcov), n, t, interval, float(denominator_floor), _hip.stream_of(dev))
+            _hip.call("bssm_forward_chunked_rotation_checked", d, m, P(keys), P(values), P(queries), P(radii),
+                      P(angles), P(process), P(observation), P(initial_mean), P(initial_covariance), P(out), P(mean_t),
+                      P(cov_t), P(bmean), P(bcov), n, t, interval, float(denominator_floor),
+                      None if probe is None else P(probe.faults), ctypes.addressof(checked), _hip.stream_of(dev))
+        if probe is not None:
+            probe.checked = bool(checked.value)
         ctx.save_for_backward(keys, values, queries, radii, angles, process, observation, initial_mean,
                               initial_covariance, bmean, bcov)
         ctx.interval = interval
@@ -619,7 +637,7 @@ class _ChunkedRotationFunction(torch.autograd.Function):
                       P(process), P(observation), P(mean0), P(cov0), P(bmean), P(bcov), P(grad_output), P(gm),
                       P(gc), *map(P, grads), P(gm0), P(gc0), n, t, ctx.interval, ctx.denominator_floor,
                       _hip.stream_of(keys.device))
-        return (*(g if need[i] else None for i, g in enumerate(grads)), gm0, gc0, None)
+        return (*(g if need[i] else None for i, g in enumerate(grads)), gm0, gc0, None, None)
 
 
 _ROTATION_SHAPES = ((2, 8), (4, 8), (8, 8))
@@ -637,6 +655,7 @@ def fused_rotation_bayesian(
     initial_covariance: Tensor,
     *,
     denominator_floor: float,
+    _probe: RotationProbe | None = None,
 ) -> tuple[Tensor, Tensor, Tensor] | None:
     """Rotation-dynamics core on the HIP kernels; ``None`` means "use the torch path".
 
@@ -656,7 +675,7 @@ def fused_rotation_bayesian(
     if any(tuple(x.shape) != e for x, e in zip(tensors, expect)):
         return None
     _hip.load()
-    return _ChunkedRotationFunction.apply(*(x.contiguous() for x in tensors), float(denominator_floor))
+    return _ChunkedRotationFunction.apply(*(x.contiguous() for x in tensors), float(denominator_floor), _probe)
 
 
 __all__ = ["fused_diagonal_bayesian", "fused_rotation_bayesian"]

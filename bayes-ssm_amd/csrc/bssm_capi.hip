@@ -996,13 +996,13 @@ int rotation_common(const char* fn, int d, int m, int64_t n, int64_t t, int64_t 
 }
 }  // namespace
 
-int bssm_forward_chunked_rotation(int key_dim, int value_dim, const float* keys, const float* values,
-                                  const float* queries, const float* radii, const float* angles,
-                                  const float* process, const float* observation, const float* mean0,
-                                  const float* cov0, float* out, float* mean_final, float* cov_final, float* bmean,
-                                  float* bcov, int64_t n, int64_t t, int64_t chunk, float denominator_floor,
-                                  void* stream) {
-  const char* fn = "bssm_forward_chunked_rotation";
+namespace {
+int rotation_forward(const char* fn, int key_dim, int value_dim, const float* keys, const float* values,
+                     const float* queries, const float* radii, const float* angles,
+                     const float* process, const float* observation, const float* mean0,
+                     const float* cov0, float* out, float* mean_final, float* cov_final, float* bmean,
+                     float* bcov, int64_t n, int64_t t, int64_t chunk, float denominator_floor,
+                     int* faults, int* checked, void* stream) {
   if (int rc = rotation_common(fn, key_dim, value_dim, n, t, chunk, denominator_floor)) return rc;
   BSSM_REQUIRE_T(keys);
   BSSM_REQUIRE_T(values);
@@ -1023,8 +1023,38 @@ int bssm_forward_chunked_rotation(int key_dim, int value_dim, const float* keys,
   a.m0 = mean0; a.c0 = cov0; a.y = out; a.mT = mean_final; a.cT = cov_final; a.bm = bmean; a.bc = bcov;
   a.n = n; a.t = t; a.chunk = chunk; a.nb = (t + chunk - 1) / chunk; a.floor = denominator_floor;
   a.base16 = all_aligned16({keys, values, queries, radii, angles, process, observation, out});
+  a.row = bssm::rotation_row_forward(key_dim, a);
+  if (checked != nullptr) {
+    *checked = n > 0 && a.row && faults != nullptr;
+    a.faults = *checked ? faults : nullptr;
+  }
   if (n == 0) return ok();
   return launched(fn, bssm::launch_rotation_forward(key_dim, a, static_cast<hipStream_t>(stream)));
+}
+}  // namespace
+
+int bssm_forward_chunked_rotation(int key_dim, int value_dim, const float* keys, const float* values,
+                                  const float* queries, const float* radii, const float* angles,
+                                  const float* process, const float* observation, const float* mean0,
+                                  const float* cov0, float* out, float* mean_final, float* cov_final, float* bmean,
+                                  float* bcov, int64_t n, int64_t t, int64_t chunk, float denominator_floor,
+                                  void* stream) {
+  return rotation_forward("bssm_forward_chunked_rotation", key_dim, value_dim, keys, values, queries, radii, angles, process, observation, mean0,
+                          cov0, out, mean_final, cov_final, bmean, bcov, n, t, chunk, denominator_floor, nullptr, nullptr,
+                          stream);
+}
+
+int bssm_forward_chunked_rotation_checked(int key_dim, int value_dim, const float* keys, const float* values,
+                                          const float* queries, const float* radii, const float* angles,
+                                          const float* process, const float* observation, const float* mean0,
+                                          const float* cov0, float* out, float* mean_final, float* cov_final, float* bmean,
+                                          float* bcov, int64_t n, int64_t t, int64_t chunk, float denominator_floor,
+                                          int* faults, int* checked, void* stream) {
+  const char* fn = "bssm_forward_chunked_rotation_checked";
+  if (checked == nullptr) return fail(BSSM_ERR_ARGUMENT, "%s: checked is null", fn);
+  return rotation_forward(fn, key_dim, value_dim, keys, values, queries, radii, angles, process, observation, mean0,
+                          cov0, out, mean_final, cov_final, bmean, bcov, n, t, chunk, denominator_floor, faults, checked,
+                          stream);
 }
 
 int bssm_backward_chunked_rotation(int key_dim, int value_dim, const float* keys, const float* values,

@@ -213,8 +213,17 @@ struct RotArgs {
   int64_t n, t, chunk, nb;
   float floor;
   int base16;
+  // Forward: take the row kernel (rotation_row_forward, read once per call);
+  // fault bits of the inputs (RotFault), or null.
+  int row;
+  int* faults;
 };
+// Bits of an input that is not finite, in the order k, v, q, rad, ang, p, r;
+// of a negative process and of an observation variance that is not positive.
+enum RotFault { kFaultK = 1, kFaultV = 2, kFaultQ = 4, kFaultRad = 8, kFaultAng = 16, kFaultP = 32, kFaultR = 64,
+                kFaultNegP = 128, kFaultNonPosR = 256 };
 int rotation_checkpoint(int key_dim);
+bool rotation_row_forward(int key_dim, const RotArgs& a);
 hipError_t launch_rotation_forward(int key_dim, const RotArgs& a, hipStream_t stream);
 // Row-per-sequence rotation forward for D = 4, M = 8 (bssm_small.hip): used
 // with 16-byte aligned stream bases and 8-byte aligned mean tensors, for n up

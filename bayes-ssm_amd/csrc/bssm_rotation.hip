@@ -1003,11 +1003,14 @@ int rotation_checkpoint(int key_dim) {
   }
 }
 
+bool rotation_row_forward(int key_dim, const RotArgs& a) {
+  auto al8 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; };
+  return key_dim == 4 && a.base16 && a.t > 0 && a.n <= small_batch_limit(4) && al8(a.m0) && al8(a.mT) && al8(a.bm);
+}
+
 hipError_t launch_rotation_forward(int key_dim, const RotArgs& a, hipStream_t stream) {
   if (a.n == 0) return hipSuccess;
-  auto al8 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; };
-  if (key_dim == 4 && a.base16 && a.t > 0 && a.n <= small_batch_limit(4) && al8(a.m0) && al8(a.mT) && al8(a.bm))
-    return launch_rotation_forward_small(a, stream);
+  if (a.row) return launch_rotation_forward_small(a, stream);
   switch (key_dim) {
     case 2: return rot::fwd<2>(a, stream);
     case 4: return rot::fwd<4>(a, stream);

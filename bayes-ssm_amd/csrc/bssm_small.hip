@@ -620,7 +620,13 @@ struct RTile {
   static constexpr int K = 0, Q = 64, V = 128, CS = 256, PP = 384, R = 448, SEQ = 488, SIZE = SPW * SEQ;
 };
 
-template <int F = kInF32>
+//
+// CHECK: the inputs' value checks (finite entries, signs of the variances) on
+// the staged pieces, 36 of about 800 VALU instructions a tile: 16384 x 512
+// tokens take 265 us with them and 247 without; the pass of bssm_checks.hip over
+// the same 772 MB took 117
+// us.
+template <bool CHECK>
 __global__ __launch_bounds__(kWave) void rotation_forward_kernel(RotArgs a) {
   __shared__ float tile[RTile::SIZE];
   const int lane = threadIdx.x;
@@ -694,6 +700,27 @@ __global__ __launch_bounds__(kWave) void rotation_forward_kernel(RotArgs a) {
     x.p = r4::ld128<false>(rp, c < 8 ? static_cast<uint32_t>(s) * row2 + t0 * 8u + c * 16u : kOob);
     const uint32_t o1 = c < 4 ? static_cast<uint32_t>(s) * row1 + t0 * 4u + c * 16u : kOob;
     x.r = r4::ld128<false>(rr, o1);
+  };
+  // x * 0 sums to NaN once any x is not finite.  Lanes without a piece hold
+  // zeros, which only the observation variances' sign has to leave out.
+  float fk = 0.f, fv = 0.f, fq = 0.f, frad = 0.f, fang = 0.f, fp = 0.f, fr = 0.f, lo_p = 0.f, lo_r = FLT_MAX;
+  auto tally = [&](const RStage& x, int64_t t0) __attribute__((always_inline)) {
+    const bool mine = c < 4 && static_cast<uint32_t>(s) < valid;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      fk = fmaf(x.k[e], 0.f, fk);
+      fq = fmaf(x.q[e], 0.f, fq);
+      fv = fmaf(x.v0[e], 0.f, fmaf(x.v1[e], 0.f, fv));
+      fp = fmaf(x.p[e], 0.f, fp);
+      fr = fmaf(x.r[e], 0.f, fr);
+      lo_p = fminf(lo_p, x.p[e]);
+      lo_r = fminf(lo_r, mine && t0 + 4 * c + e < T ? x.r[e] : FLT_MAX);
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      frad = fmaf(x.rad[e], 0.f, frad);
+      fang = fmaf(x.ang[e], 0.f, fang);
+    }
   };
   auto put = [&](const RStage& x) __attribute__((always_inline)) {
     float* b = tile + s * RTile::SEQ;
@@ -777,6 +804,7 @@ __global__ __launch_bounds__(kWave) void rotation_forward_kernel(RotArgs a) {
     }
     r4::vm_wait<0>();
     put(x);
+    if constexpr (CHECK) tally(x, t0);
     if (ti > 0) {
       const uint32_t o8 = static_cast<uint32_t>(s) * row8 + (t0 - TT) * 32u + c * 16u;
       r4::st128<r4::kNtStore>(ry, ys0, o8, 0);
@@ -829,6 +857,13 @@ __global__ __launch_bounds__(kWave) void rotation_forward_kernel(RotArgs a) {
   r4::st64(rmT, own_order(m, odd), mo, 0);
   r4::st32(rcT, P, cvo, 0);
   store_ckpt(static_cast<uint32_t>(a.nb));
+  if constexpr (CHECK) {
+    const float sums[7] = {fk, fv, fq, frad, fang, fp, fr};  // the order of RotFault
+    int bits = (lo_p < 0.f ? kFaultNegP : 0) | (lo_r <= 0.f ? kFaultNonPosR : 0);
+#pragma unroll
+    for (int e = 0; e < 7; ++e) bits |= sums[e] != sums[e] ? 1 << e : 0;
+    if (bits != 0) atomicOr(a.faults, bits);
+  }
 }
 
 // ----------------------------------------------------------------- backward
@@ -1510,7 +1545,9 @@ hipError_t launch_backward_small(bool fixed, bool dyn, const BwdArgs& a, hipStre
 hipError_t launch_rotation_forward_small(const RotArgs& a, hipStream_t stream) {
   const int64_t blocks = (a.n + sn::SPW - 1) / sn::SPW;
   if (blocks == 0) return hipSuccess;
-  hipLaunchKernelGGL((sn::rotation_forward_kernel<>), dim3(static_cast<unsigned>(blocks)), dim3(kWave), 0, stream, a);
+  const dim3 grid(static_cast<unsigned>(blocks)), block(kWave);
+  if (a.faults) hipLaunchKernelGGL((sn::rotation_forward_kernel<true>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((sn::rotation_forward_kernel<false>), grid, block, 0, stream, a);
   return hipGetLastError();
 }
 

@@ -462,6 +462,21 @@ int bssm_forward_chunked_rotation(int key_dim, int value_dim,
                                   float* bmean, float* bcov,
                                   int64_t n, int64_t t, int64_t chunk, float denominator_floor,
                                   void* stream);
+/* The same call with the value checks of bayesian_layer on the way: *checked
+ * (host) is set to 1 where the kernel makes them (D = 4's row kernel, see
+ * bssm_small_batch_limit), else to 0, and then faults (device, 4 bytes that the
+ * caller cleared) receives a bit for each input with an entry that is not
+ * finite (1 keys, 2 values, 4 queries, 8 radii, 16 angles, 32 process, 64
+ * observation), 128 for a negative process variance and 256 for an
+ * observation variance that is not positive.  faults NULL: no checks. */
+int bssm_forward_chunked_rotation_checked(int key_dim, int value_dim,
+                                          const float* keys, const float* values, const float* queries,
+                                          const float* radii, const float* angles, const float* process,
+                                          const float* observation, const float* mean0, const float* cov0,
+                                          float* out, float* mean_final, float* cov_final,
+                                          float* bmean, float* bcov,
+                                          int64_t n, int64_t t, int64_t chunk, float denominator_floor,
+                                          int* faults, int* checked, void* stream);
 
 /* Reverse: all seven input gradients (g_radii is zero where the radius clamp
  * is active) and, when non-NULL, gm0 and the asymmetric gc0 (the convention
@@ -490,8 +505,7 @@ int bssm_rotation_checkpoint(int key_dim);
  * waves of the latter do not fill the GPU and each wave's time is its own
  * instruction stream, which the row layout shortens; at large N the row
  * layout's extra lane work costs more than it saves (the backward first).
- * The backward also needs T a multiple of 16 and the preferred checkpoint
- * chunk.  Direction 2 (3): the largest N, within direction 0's (1's), for
+ * The backward also needs the preferred checkpoint chunk.  Direction 2 (3): the largest N, within direction 0's (1's), for
  * which the row forward (backward) runs as two (three) waves per 4
  * sequences, the covariance and mean halves (the covariance replay, the
  * covariance reverse and the mean) on separate SIMDs, bitwise the one-wave
@@ -500,7 +514,7 @@ int bssm_rotation_checkpoint(int key_dim);
  * (widened on chip, bitwise the float32 split kernels on the widened values).
  * Direction 4: the largest N for which the D = 4 rotation forward
  * (bssm_forward_chunked_rotation) uses its row-per-sequence kernel (16-byte
- * aligned streams, T a multiple of 4).  Defaults: 24576, 8192, 2048, 2048,
+ * aligned streams).  Defaults: 24576, 8192, 2048, 2048,
  * 32768, the measured crossovers.
  * Sets the limit when limit >= 0 and returns the previous one; limit < 0
  * only reads it; -1 for any other direction.  Results of the row and

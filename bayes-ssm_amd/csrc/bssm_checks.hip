@@ -131,28 +131,37 @@ __global__ __launch_bounds__(kThreads) void fold_kernel(StatArgs a, const float*
   }
 }
 
-// A wave takes whole rows, its lanes the 16-byte pieces of a row.  The pieces
-// are read once: bound by HBM (46 MB of projections, 32 x 511 x 64 heads).
+// Lanes over all pieces of a tensor (16 bytes each, rows of a power of two or
+// any other number of them), four loads of a lane in flight: 46 MB of
+// projections (32 x 511 x 64 heads) in 11.5 us, against 21 us with a wave to a
+// row, where the rows of 16 and 32 pieces left most of its lanes idle.
 __global__ __launch_bounds__(kThreads) void large_bf16_kernel(LargeArgs a, int* __restrict__ flags) {
   typedef uint32_t v4 __attribute__((ext_vector_type(4)));
   __shared__ int any;
   if (threadIdx.x == 0) any = 0;
   __syncthreads();
-  constexpr int kWaves = kThreads / kWave;
-  const int lane = threadIdx.x % kWave;
+  constexpr int kAhead = 4;
+  const int64_t step = static_cast<int64_t>(gridDim.x) * kThreads;
   uint32_t bad = 0;
   for (int i = 0; i < a.count; ++i) {
-    const int64_t pieces = a.cols[i] / 8;
-    for (int64_t row = static_cast<int64_t>(blockIdx.x) * kWaves + threadIdx.x / kWave; row < a.rows[i];
-         row += static_cast<int64_t>(gridDim.x) * kWaves) {
-      const v4* p = reinterpret_cast<const v4*>(static_cast<const uint16_t*>(a.ptr[i]) + row * a.ld[i]);
-      for (int64_t c = lane; c < pieces; c += kWave) {
-        const v4 x = p[c];
+    const int64_t pieces = a.cols[i] / 8, total = a.rows[i] * pieces;
+    const uint16_t* base = static_cast<const uint16_t*>(a.ptr[i]);
+    for (int64_t at = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; at < total; at += kAhead * step) {
+      v4 x[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int64_t e = at + u * step < total ? at + u * step : at;
+        const int64_t row = total <= 0xffffffff
+                                ? static_cast<uint32_t>(e) / static_cast<uint32_t>(pieces) : e / pieces;
+        x[u] = *reinterpret_cast<const v4*>(base + row * a.ld[i] + (e - row * pieces) * 8);
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
           // Exponent field 127 + 63 = 0xbe or more, of either half.
-          bad |= (x[w] & 0x7f80u) >= 0x5f00u;
-          bad |= (x[w] & 0x7f800000u) >= 0x5f000000u;
+          bad |= (x[u][w] & 0x7f80u) >= 0x5f00u;
+          bad |= (x[u][w] & 0x7f800000u) >= 0x5f000000u;
         }
       }
     }

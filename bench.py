@@ -61,7 +61,7 @@ def dispatched_kernels(d: int, m: int, n: int, t: int, interval: int) -> tuple[s
     (D4M8: the row-per-sequence kernels up to the library's small-batch limits, else the rotated layout)."""
     from bayes_ssm import _hip
 
-    if (d, m) != (4, 8) or t % 4:
+    if (d, m) != (4, 8):
         return f"bssm forward kernel (D{d}M{m})", f"bssm backward kernel (D{d}M{m})"
     lib = _hip.load()
     lim = [lib.bssm_small_batch_limit(k, -1) for k in range(4)]
@@ -72,14 +72,15 @@ def dispatched_kernels(d: int, m: int, n: int, t: int, interval: int) -> tuple[s
         fwd = "bssm::sn::forward_kernel<false, 0> (row layout, 16 lanes per sequence)"
     else:
         fwd = "bssm::r4::forward_kernel<false, 0> (rotated layout, 4 lanes per sequence)"
-    row_bwd = t % 16 == 0 and interval == _hip.preferred_checkpoint(4)
+    row_bwd = interval == _hip.preferred_checkpoint(4)
     if row_bwd and n <= lim[3]:
         bwd = f"bssm::sn::backward_split_kernel<false, true, 0, {groups}> (row layout, three waves per 4 sequences)"
     elif row_bwd and n <= lim[1]:
         bwd = "bssm::sn::backward_kernel<false, true> (row layout, 16 lanes per sequence)"
     else:
-        bwd = (f"bssm::r4::backward_tile_kernel<false, true, 0, {interval}> (rotated layout, 4 lanes per sequence, "
-               "16-token tiles)")
+        ragged = "true" if t % 4 else "false"  # T ends inside a 4-token piece
+        bwd = (f"bssm::r4::backward_tile_kernel<false, true, 0, {interval}, {ragged}> (rotated layout, "
+               "4 lanes per sequence, 16-token tiles)")
     return fwd, bwd
 
 

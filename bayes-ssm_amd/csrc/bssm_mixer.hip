@@ -37,6 +37,8 @@
 // row's last head.  32 x 511 x 64 heads, gated, forward and backward: 770 us,
 // against 6010 us as torch ops around the layer kernels, where such shapes fell.
 
+#include <cfloat>
+
 #include "bssm_mixer.h"
 
 namespace bssm {
@@ -231,6 +233,7 @@ struct MixEpi {
   Rsrc gate, out, yb, gout, ggate;
   uint32_t rg, cg;    // gate row bytes; lane byte offset in a row
   uint32_t ro, co;    // contiguous bf16 rows (H * 16 bytes); lane byte offset
+  uint32_t tro;       // bytes of a batch row of them
   uint32_t rgg;       // ggate row bytes (bf16 layout)
   float w[4], eps;
   bool precise;
@@ -243,7 +246,8 @@ struct MixEpi {
     ro = static_cast<uint32_t>(a.h) * 16u;
     co = cg;
     rgg = static_cast<uint32_t>(a.ldgg ? a.ldgg : 8 * a.h) * 2u;
-    const uint32_t tro = static_cast<uint32_t>(T) * ro, trw = precise ? 2u * tro : tro;
+    tro = static_cast<uint32_t>(T) * ro;
+    const uint32_t trw = precise ? 2u * tro : tro;
     const uint32_t trg = (precise ? 2u : 1u) * static_cast<uint32_t>(T) * rgg;
     gate = make_rsrc(as_f(a.gate, bb * T * rg), static_cast<uint32_t>(T) * rg);
     yb = make_rsrc(as_f(a.yb, bb * tro), tro);
@@ -372,8 +376,9 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1, 1))) v
 }
 
 // RAG: T is not a multiple of 4 (the last chunk is filled up with neutral
-// tokens; a template parameter, so that the register-bound loop of the other
-// case stays as it is).
+// tokens), or the epilogue's eps is zero and tokens or heads are missing from
+// the last tile or wave (a template parameter, so that the register-bound loop
+// of the other case stays as it is).
 template <bool DYN, bool EPI, bool BIAS, bool RAG>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1, 1))) void mixer_backward_kernel(
     MixArgs a) {
@@ -448,13 +453,17 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1, 1))) v
   // (n = y r, h = n w, out = h silu(z)):
   //   dL/dh = gout silu(z),  dL/dz = gout h silu'(z),  dL/dw += dL/dh n,
   //   gy = r (dL/dn - n mean(dL/dn n)) with dL/dn = dL/dh w.
+  // Tokens at or past T and heads past the wave's last read zeros: with
+  // eps = 0 their r would be infinite and n = 0 r not a number, so r is zero
+  // there (RAG; see the launch).
   auto put_epi = [&](const EpiHalf& x, int64_t J, int h) __attribute__((always_inline)) {
     v4f dw = dwl[lane];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int I = 4 * h + i;
       const v4f y = widen4(x.yb[i]), z = widen4(x.gt[i]), go = widen4(x.go[i]);
-      const float r = ep.inv_rms(y);
+      const uint32_t t = static_cast<uint32_t>(J * 2 * SUB + mm.y_tok[I]);
+      const float rms = ep.inv_rms(y), r = !RAG || t * ep.ro + ep.co < ep.tro ? rms : 0.f;
       v4f gz, gn, n;
       float dot = 0.f;
 #pragma unroll
@@ -473,7 +482,6 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(1, 1))) v
 #pragma unroll
       for (int c = 0; c < 4; ++c) gy[c] = r * fmaf(-n[c], dot * 0.125f, gn[c]);
       *reinterpret_cast<v4f*>(&tile[BwdTile::GY + mm.y_lds[I]]) = gy;
-      const uint32_t t = static_cast<uint32_t>(J * 2 * SUB + mm.y_tok[I]);
       ep.put4(ep.ggate, t * ep.rgg + ep.co, gz);
     }
     dwl[lane] = dw;
@@ -673,7 +681,12 @@ hipError_t launch_mixer_backward(const MixArgs& a, hipStream_t stream) {
   const int64_t blocks = a.b * ((a.h + r4::SPW - 1) / r4::SPW);
   if (blocks == 0) return hipSuccess;
   const dim3 grid(static_cast<unsigned>(blocks));
-  if (a.t % 4 != 0) launch_mixer_backward_rag<true>(a, grid, stream);
+  // With eps = 0 the missing tokens and heads of a last tile or wave need the
+  // RAG kernels' mask (below the smallest normal number 1 / sqrt(eps) may be
+  // infinite).  In the other kernels, whose registers are all taken, the mask
+  // cost 8 % (256 x 512 x 64 heads, gated, forward and backward: 834 -> 906 us).
+  const bool mask = a.gate != nullptr && a.norm_eps < FLT_MIN && (a.t % 16 != 0 || a.h % r4::SPW != 0);
+  if (a.t % 4 != 0 || mask) launch_mixer_backward_rag<true>(a, grid, stream);
   else launch_mixer_backward_rag<false>(a, grid, stream);
   return hipGetLastError();
 }

@@ -448,13 +448,14 @@ __global__ __launch_bounds__(4 * G * kWave) void mixer_backward_row_kernel(MixAr
       v4f gy;
       if constexpr (EPI) {
         // gy of the readout's epilogue, its gate gradient and weight-gradient
-        // share (the equations of bssm_mixer.hip's put_epi).
+        // share (the equations of bssm_mixer.hip's put_epi; r = 0 for tokens
+        // past T, as there).
         const v4f y = widen4(xy), z = widen4(xg), go = widen4(xo);
         float ss = y[0] * y[0];
 #pragma unroll
         for (int k = 1; k < 4; ++k) ss = fmaf(y[k], y[k], ss);
         ss += dpp<kRowRor8>(ss);
-        const float r = __builtin_amdgcn_rsqf(fmaf(ss, 0.125f, a.norm_eps));
+        const float rms = __builtin_amdgcn_rsqf(fmaf(ss, 0.125f, a.norm_eps)), r = x == 0 && tk >= len0 ? 0.f : rms;
         v4f gz, gn, nn;
         float dot = 0.f;
 #pragma unroll

@@ -486,15 +486,21 @@ class _ChunkedBayesianBF16Function(torch.autograd.Function):
                 gd if need[3] else None, gp if need[4] else None, gr if need[5] else None, gm0, gc0, None, None)
 
 
-def _bf16_kernels_apply(keys: Tensor, values: Tensor, queries: Tensor, fixed: bool) -> bool:
+def _bf16_kernels_apply(keys: Tensor, values: Tensor, queries: Tensor, dynamics: tuple[Tensor, ...],
+                        belief: tuple[Tensor, ...], fixed: bool) -> bool:
     """The D4M8 kernels read these bfloat16 / float8 streams directly (else: widen, float32 path).
 
-    With fixed dynamics and T not a multiple of 4 the backward kernels take
-    no final-state gradients; whether there will be any is not known here.
+    They need every stream on a 16-byte boundary and the belief on an 8-byte
+    one, which a slice of a batch need not be: process and observation rows
+    are T floats apart.  With fixed dynamics (no stream of theirs is read) and
+    T not a multiple of 4 the backward kernels take no final-state gradients;
+    whether there will be any is not known here.
     """
     n, t, d = keys.shape
+    streams = (keys, values, queries) if fixed else (keys, values, queries, *dynamics)
     return ((d, values.shape[-1]) == (4, 8) and t > 0 and (t % 4 == 0 or not fixed)
-            and _hip.preferred_checkpoint(d) > 0 and all(x.data_ptr() % 16 == 0 for x in (keys, values, queries)))
+            and _hip.preferred_checkpoint(d) > 0 and all(x.data_ptr() % 16 == 0 for x in streams)
+            and all(x.data_ptr() % 8 == 0 for x in belief))
 
 
 def fused_diagonal_bayesian(
@@ -557,7 +563,8 @@ def fused_diagonal_bayesian(
         x if x.is_contiguous() else x.contiguous()
         for x in (keys, values, queries, decay, process, observation, initial_mean, initial_covariance))
     if bf16:
-        if _bf16_kernels_apply(keys, values, queries, bool(fixed_dynamics)):
+        if _bf16_kernels_apply(keys, values, queries, (decay, process, observation),
+                               (initial_mean, initial_covariance), bool(fixed_dynamics)):
             return _ChunkedBayesianBF16Function.apply(
                 keys, values, queries, decay, process, observation, initial_mean, initial_covariance,
                 float(denominator_floor), bool(fixed_dynamics))

@@ -138,6 +138,13 @@ def ptr(x: Optional[Tensor]) -> Optional[int]:
     return None if x is None else x.data_ptr()
 
 
+def aligned(x: Tensor) -> Tensor:
+    """``x`` contiguous with a 16-byte aligned base: a contiguous view at an unaligned offset (a slice of a flattened
+    buffer, a gradient that a concatenation hands back) is copied."""
+    x = x.contiguous()
+    return x if x.data_ptr() % 16 == 0 else x.clone()
+
+
 def stream_of(device: torch.device) -> int:
     """The ``hipStream_t`` of torch's current stream on ``device``."""
     index = device.index if device.index is not None else torch.cuda.current_device()

@@ -465,9 +465,9 @@ class _ChunkedBayesianBF16Function(torch.autograd.Function):
         if grad_output is None:
             grad_output = torch.zeros(n, t, m, device=keys.device, dtype=torch.float32)
         else:
-            grad_output = grad_output.contiguous()
-        gm = None if grad_mean is None else grad_mean.contiguous()
-        gc = None if grad_covariance is None else grad_covariance.contiguous()
+            grad_output = _hip.aligned(grad_output)
+        gm = None if grad_mean is None else _hip.aligned(grad_mean)
+        gc = None if grad_covariance is None else _hip.aligned(grad_covariance)
         gk, gv, gq = torch.empty_like(keys), torch.empty_like(values), torch.empty_like(queries)
         dyn = any(need[3:6])
         gd = torch.empty_like(decay) if dyn else None

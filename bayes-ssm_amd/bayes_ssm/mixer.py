@@ -53,13 +53,6 @@ NOISE_FLOOR = 1e-4  # softplus(noise) + 1e-4 (train_6layer.py:667-668)
 _WIDTHS = (KEY_DIM, KEY_DIM, VALUE_DIM, KEY_DIM, 2)
 
 
-def _aligned(x: Tensor) -> Tensor:
-    """``x`` contiguous with a 16-byte aligned base (the C ABI's requirement for weights, biases and belief
-    tensors): a contiguous view at an unaligned offset, e.g. a slice of a flattened parameter buffer, is copied."""
-    x = x.contiguous()
-    return x if x.data_ptr() % 16 == 0 else x.clone()
-
-
 def _row_stride(x: Tensor, t: int) -> Optional[int]:
     """Row stride (elements) of a [B, T, W] view the kernels can address, else None."""
     if x.ndim != 3 or x.stride(2) != 1:
@@ -197,9 +190,9 @@ class _MixerCoreFunction(torch.autograd.Function):
         if grad_read is None:
             grad_read = torch.zeros(b, t, heads, VALUE_DIM, device=dev, dtype=torch.float32)
         else:
-            grad_read = grad_read.float().contiguous()
-        gm = None if grad_mean is None else grad_mean.float().contiguous()
-        gc = None if grad_covariance is None else grad_covariance.float().contiguous()
+            grad_read = _hip.aligned(grad_read.float())
+        gm = None if grad_mean is None else _hip.aligned(grad_mean.float())
+        gc = None if grad_covariance is None else _hip.aligned(grad_covariance.float())
 
         def empty(x: Tensor) -> Tensor:
             return torch.empty(x.shape, device=dev, dtype=torch.bfloat16)
@@ -250,7 +243,7 @@ def _initial_state(initial_mean: Optional[Tensor], initial_covariance: Optional[
         cov0 = torch.eye(KEY_DIM, device=device, dtype=torch.float32).expand(n, KEY_DIM, KEY_DIM)
     else:
         cov0 = initial_covariance.to(device=device, dtype=torch.float32).expand(n, KEY_DIM, KEY_DIM)
-    return _aligned(mean0), _aligned(cov0)
+    return _hip.aligned(mean0), _hip.aligned(cov0)
 
 
 def mixer_layer_inputs(q_proj: Tensor, k_proj: Tensor, v_proj: Tensor, decay_logits: Tensor, noise: Tensor,
@@ -354,7 +347,7 @@ class _MixerReadoutFunction(torch.autograd.Function):
         cov_t = torch.empty(n, KEY_DIM, KEY_DIM, device=dev, dtype=torch.float32)
         bmean = torch.empty(n, nb + 1, KEY_DIM, VALUE_DIM, device=dev, dtype=torch.float32)
         bcov = torch.empty(n, nb + 1, KEY_DIM, KEY_DIM, device=dev, dtype=torch.float32)
-        w32 = _aligned(norm_weight.detach().float())
+        w32 = _hip.aligned(norm_weight.detach().float())
         P = _hip.ptr
         with _hip.on_device(dev):
             _hip.call("bssm_mixer_gated_forward", P(q_proj), lds[0], P(k_proj), lds[1], P(v_proj), lds[2],
@@ -382,9 +375,9 @@ class _MixerReadoutFunction(torch.autograd.Function):
         if grad_out is None:
             grad_out = torch.zeros(b, t, heads * VALUE_DIM, device=dev, dtype=torch.bfloat16)
         else:
-            grad_out = grad_out.to(torch.bfloat16).contiguous()
-        gm = None if grad_mean is None else grad_mean.float().contiguous()
-        gc = None if grad_covariance is None else grad_covariance.float().contiguous()
+            grad_out = _hip.aligned(grad_out.to(torch.bfloat16))
+        gm = None if grad_mean is None else _hip.aligned(grad_mean.float())
+        gc = None if grad_covariance is None else _hip.aligned(grad_covariance.float())
 
         def empty(x: Tensor) -> Tensor:
             return torch.empty(x.shape, device=dev, dtype=torch.bfloat16)
@@ -486,7 +479,7 @@ class _MixerBlockFunction(torch.autograd.Function):
         dev = projected.device
         # The kernels add the aux bias as they read the aux columns, in bf16
         # as the reference does (one rounding).
-        bias = None if aux_bias is None else _aligned(aux_bias.detach())
+        bias = None if aux_bias is None else _hip.aligned(aux_bias.detach())
         convolved = torch.empty(b, t, core, device=dev, dtype=torch.bfloat16)
         out = torch.empty(b, t, heads * VALUE_DIM, device=dev, dtype=torch.bfloat16)
         read_bf16 = torch.empty_like(out)
@@ -495,8 +488,8 @@ class _MixerBlockFunction(torch.autograd.Function):
         cov_t = torch.empty(n, KEY_DIM, KEY_DIM, device=dev, dtype=torch.float32)
         bmean = torch.empty(n, nb + 1, KEY_DIM, VALUE_DIM, device=dev, dtype=torch.float32)
         bcov = torch.empty(n, nb + 1, KEY_DIM, KEY_DIM, device=dev, dtype=torch.float32)
-        cw32 = _aligned(conv_weight.detach().reshape(core, 4).float())
-        nw32 = _aligned(norm_weight.detach().float())
+        cw32 = _hip.aligned(conv_weight.detach().reshape(core, 4).float())
+        nw32 = _hip.aligned(norm_weight.detach().float())
         P = _hip.ptr
         with _hip.on_device(dev):
             _hip.call("bssm_mixer_block_forward", P(projected), ld, P(cw32), P(bias), P(nw32), float(norm_eps),
@@ -522,9 +515,9 @@ class _MixerBlockFunction(torch.autograd.Function):
         if grad_out is None:
             grad_out = torch.zeros(b, t, heads * VALUE_DIM, device=dev, dtype=torch.bfloat16)
         else:
-            grad_out = grad_out.to(torch.bfloat16).contiguous()
-        gm = None if grad_mean is None else grad_mean.float().contiguous()
-        gc = None if grad_covariance is None else grad_covariance.float().contiguous()
+            grad_out = _hip.aligned(grad_out.to(torch.bfloat16))
+        gm = None if grad_mean is None else _hip.aligned(grad_mean.float())
+        gc = None if grad_covariance is None else _hip.aligned(grad_covariance.float())
         gproj = torch.empty(b, t, core + aux_w + heads * VALUE_DIM, device=dev, dtype=torch.bfloat16)
         gconv = torch.empty(b, t, core, device=dev, dtype=torch.bfloat16)
         cpart = torch.empty(b, core, 4, device=dev, dtype=torch.float32)
@@ -628,9 +621,9 @@ def bayes_mixer_block(
         if not whole:
             # The layer's inputs come of the core and aux columns, the filter's taps and the bias (the taps as rows
             # of 8: core is a multiple of 64).
-            views = [projected[..., :core + aux], _aligned(conv_weight.detach().reshape(1, -1, 8))]
+            views = [projected[..., :core + aux], _hip.aligned(conv_weight.detach().reshape(1, -1, 8))]
             if aux_bias is not None:
-                views.append(_aligned(aux_bias.detach()).view(1, 1, aux))
+                views.append(_hip.aligned(aux_bias.detach()).view(1, 1, aux))
             scan = _LargeScan(tuple(views))
         mean0, cov0 = _initial_state(initial_mean, initial_covariance, b * heads, projected.device)
         outs = _MixerBlockFunction.apply(projected, conv_weight, norm_weight, aux_bias, mean0, cov0, int(heads), eps,

@@ -58,7 +58,7 @@ def _row_stride(x: Tensor, t: int) -> Optional[int]:
     if x.ndim != 3 or x.stride(2) != 1:
         return None
     ld = x.stride(1)
-    if ld % 8 != 0 or x.data_ptr() % 16 != 0:
+    if ld % 8 != 0 or ld < x.shape[2] or x.data_ptr() % 16 != 0:
         return None
     if x.shape[0] > 1 and x.stride(0) != t * ld:
         return None

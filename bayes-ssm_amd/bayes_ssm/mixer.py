@@ -23,7 +23,8 @@ which is what autograd through the reference's ``.float()`` widening yields.
 
 Heads a multiple of 16 with T a multiple of 4 ("whole tiles") always run the
 kernels.  Heads a multiple of 4 with any T run them when the call is one that
-the op chain would take without complaint (see ``_any_shape_call``): the op
+the op chain would take without complaint (see ``_any_shape_call``) and its
+rows are within the kernels' 32-bit offsets (``_in_limits``): the op
 chain validates the layer's inputs, so the projections are scanned on the
 device first, and a call with a non-finite (or enormous) value is left to the
 op chain, which raises or computes as it always has.  Other shapes (and other
@@ -96,6 +97,12 @@ def _any_shape_call(heads: int, t: int, initial_mean: Optional[Tensor], initial_
                                           and chunk_length > 0))
             and os.environ.get("BAYES_SSM_DISABLE_FUSED_CUDA", "0") != "1"
             and not (torch.is_grad_enabled() and _replay_enabled()))
+
+
+def _in_limits(t: int, heads: int, *lds: int) -> bool:
+    """The entry points address a batch row's streams (row strides ``lds``, checkpoint records) with 32-bit offsets."""
+    records = -(-t // _hip.preferred_checkpoint(KEY_DIM)) + 1
+    return max(records * 2048, t * heads * 32, *((t + 16) * ld * 2 for ld in lds)) < 1 << 31
 
 
 class _LargeScan:
@@ -312,8 +319,9 @@ def bayes_mixer_core(
             raise ValueError(f"{name} must have shape [B, T, H*{w}] = {(b, t, w * heads)}, got {tuple(x.shape)}")
     lds = _fused_eligible(projections, heads, whole=False)
     whole = _whole_tiles(heads, t)
-    if lds is not None and (whole or _any_shape_call(heads, t, initial_mean, initial_covariance, chunk_length,
-                                                     denominator_floor, optimized)):
+    if lds is not None and (whole or (_any_shape_call(heads, t, initial_mean, initial_covariance, chunk_length,
+                                                      denominator_floor, optimized)
+                                      and _in_limits(t, heads, *lds))):
         _hip.load()  # on a GPU the fused path never degrades silently
         scan = None if whole else _LargeScan(projections)
         mean0, cov0 = _initial_state(initial_mean, initial_covariance, b * heads, q_proj.device)
@@ -448,6 +456,7 @@ def bayes_mixer_readout(
     whole = _whole_tiles(heads, t)
     if lds is not None and ldg is not None and (whole or (
             _any_shape_call(heads, t, initial_mean, initial_covariance, chunk_length, denominator_floor, optimized)
+            and _in_limits(t, heads, *lds, ldg)
             and denominator_floor > 0 and eps >= 0 and norm_weight.dtype == torch.bfloat16
             and norm_weight.device == q_proj.device)):
         _hip.load()
@@ -608,6 +617,7 @@ def bayes_mixer_block(
     fused = (ld is not None and t > 0
              and (whole or (_any_shape_call(heads, t, initial_mean, initial_covariance, chunk_length,
                                             denominator_floor, optimized)
+                            and _in_limits(t, heads, ld)
                             and conv_weight.dtype == norm_weight.dtype == torch.bfloat16
                             and (norm_eps is None or norm_eps >= 0)))
              and conv_weight.device == projected.device and norm_weight.device == projected.device

@@ -95,9 +95,9 @@ __device__ __forceinline__ void put_v(float* dst, v4f v0, v4f v1, int c) {
 // The reverse: gradients in a region of TOK x 4 / TOK x 8 floats leave as
 // 16-byte pieces of format F (bfloat16: round to nearest even; float8:
 // narrow_f8, torch's rounding), at the loaders' offsets.
-// With len < TOK only the first len tokens' values are stored (a row that
+// RAG: with len < TOK only the first len tokens' values are stored (a row that
 // ends inside the block: the piece across its end leaves word by word).
-template <int F, int TOK>
+template <int F, int TOK, bool RAG>
 __device__ __forceinline__ void store_kq(Rsrc r, uint32_t row, int s, int c, uint32_t t0, int len,
                                          const float* src) {
   const uint32_t off = static_cast<uint32_t>(s) * row + t0 * kq_bytes<F>() + static_cast<uint32_t>(c) * 16u;
@@ -114,10 +114,10 @@ __device__ __forceinline__ void store_kq(Rsrc r, uint32_t row, int s, int c, uin
     for (int u = 0; u < 4; ++u) w[u] = narrow_f8<F>(*reinterpret_cast<const v4f*>(src + 16 * cc + 4 * u));
     x = __builtin_bit_cast(v4f, w);
   }
-  if (len == TOK) r4::st128<r4::kNtStore>(r, x, o, 0);
+  if (!RAG || len == TOK) r4::st128<r4::kNtStore>(r, x, o, 0);
   else store_words(r, x, off, c < kq_lanes<F, TOK>() ? len * static_cast<int>(kq_bytes<F>() / 4) - 4 * c : 0);
 }
-template <int F, int TOK>
+template <int F, int TOK, bool RAG>
 __device__ __forceinline__ void store_v(Rsrc r, uint32_t row, int s, int c, uint32_t t0, int len,
                                         const float* src) {
   static_assert(TOK * 2 * kq_bytes<F>() <= 256u, "one piece per lane");
@@ -136,7 +136,7 @@ __device__ __forceinline__ void store_v(Rsrc r, uint32_t row, int s, int c, uint
     for (int u = 0; u < 4; ++u) w[u] = narrow_f8<F>(*reinterpret_cast<const v4f*>(src + 16 * cc + 4 * u));
     x = __builtin_bit_cast(v4f, w);
   }
-  if (len == TOK) r4::st128<r4::kNtStore>(r, x, o, 0);
+  if (!RAG || len == TOK) r4::st128<r4::kNtStore>(r, x, o, 0);
   else store_words(r, x, off, c < lanes ? len * static_cast<int>(kq_bytes<F>() / 2) - 4 * c : 0);
 }
 
@@ -947,11 +947,11 @@ __device__ __forceinline__ void get_grads(GStage& g, const float* tl, int s, int
   }
 }
 
-template <bool DYN>
+template <bool DYN, bool RAG>
 __device__ __forceinline__ void store_grads(const GStage& g, const BStreams& st, const BwdArgs& a, int s, int c,
                                             uint32_t t0) {
   // Tokens of the tile below T; a partial (last) tile drops the others' pieces.
-  const int len = static_cast<int>(a.t - t0) < TT ? static_cast<int>(a.t - t0) : TT;
+  const int len = RAG && static_cast<int>(a.t - t0) < TT ? static_cast<int>(a.t - t0) : TT;
   const uint32_t o4 = c < len ? static_cast<uint32_t>(s) * st.row4 + (t0 + c) * 16u : kOob;
   r4::st128<r4::kNtStore>(st.gk, g.k, o4, 0);
   r4::st128<r4::kNtStore>(st.gq, g.q, o4, 0);
@@ -1069,7 +1069,8 @@ __device__ __forceinline__ void reverse_step(const RTok& x, const Hist& h, float
   o.ge[1] = ge1;
 }
 
-template <bool FIXED, bool DYN>
+// RAG: T is not a multiple of 16 (a template parameter, as in the kernels below).
+template <bool FIXED, bool DYN, bool RAG>
 __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
   __shared__ float tile[BTile::SIZE];
   const int lane = threadIdx.x;
@@ -1194,8 +1195,8 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
     r4::vm_wait<0>();
     const Bel k0 = nk0, k1 = nk1;
     put_btile<FIXED>(x, tile, s, c);
-    if (t0 + TT > T) neutral_tail<BTile, TT>(mine, static_cast<int>(T - t0), c);
-    if (ti + 1 < ntiles) store_grads<DYN>(go, st, a, s, c, t0 + TT);
+    if (RAG && t0 + TT > T) neutral_tail<BTile, TT>(mine, static_cast<int>(T - t0), c);
+    if (ti + 1 < ntiles) store_grads<DYN, RAG>(go, st, a, s, c, t0 + TT);
     if (ti > 0) {
       load_btile<FIXED>(x, st, s, c, t0 - TT);
       load_ckpt(nk0, 2 * ti - 2);
@@ -1208,7 +1209,7 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
   if (ntiles > 0) {
     r4::lds_wait();
     get_grads<DYN>(go, tile, s, c);
-    store_grads<DYN>(go, st, a, s, c, 0);
+    store_grads<DYN, RAG>(go, st, a, s, c, 0);
   }
   if (a.gm0) {
     const Rsrc rgm0 = make_rsrc(a.gm0 + n0 * 32, valid * 128u);
@@ -1233,7 +1234,10 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
 // share a SIMD.  With G = 2 the six waves are ordered reverse A, reverse B,
 // mean A, mean B, replay A, replay B: waves 4 and 5 share the SIMDs of waves 0
 // and 1, and every long wave has its SIMD alone or with a replay wave.
-template <bool FIXED, bool DYN, int F, int G>
+// RAG: T is not a multiple of 8.  A template parameter: the tail's stores and
+// tests in the replay wave's loop cost 8 % of the bfloat16 step (512 x 512,
+// forward and backward: 156 -> 169 us).
+template <bool FIXED, bool DYN, int F, int G, bool RAG>
 __global__ __launch_bounds__(3 * G * kWave) void backward_split_kernel(BwdArgs a) {
   __shared__ float lds_all[G * SBTile::SIZE];
   constexpr int CH = SBTile::CH;
@@ -1256,7 +1260,7 @@ __global__ __launch_bounds__(3 * G * kWave) void backward_split_kernel(BwdArgs a
   const int64_t nb = (T + CH - 1) / CH;  // chunks; position x is chunk nb - 1 - x
   // Tokens of chunk position x (position 0 holds the row's end).
   const int len0 = static_cast<int>(T - (nb - 1) * CH);
-  auto clen = [&](int64_t x) __attribute__((always_inline)) { return x == 0 ? len0 : CH; };
+  auto clen = [&](int64_t x) __attribute__((always_inline)) { return RAG && x == 0 ? len0 : CH; };
   // Ring slots of step position x (T / 8 positions: 32-bit arithmetic).
   auto slot = [&](int64_t x) __attribute__((always_inline)) {
     return lds + SBTile::IN + static_cast<int>(static_cast<uint32_t>(x) % SBTile::NSLOT) * SBTile::SLOT +
@@ -1325,7 +1329,7 @@ __global__ __launch_bounds__(3 * G * kWave) void backward_split_kernel(BwdArgs a
       put_v<F, CH>(b + SBTile::V, sv, sv1, c);
       *reinterpret_cast<v4f*>(b + SBTile::GY + 4 * c) = sg;
       *reinterpret_cast<v2f*>(b + SBTile::MC + 2 * c) = sm;
-      if (x == 0 && len0 < CH) neutral_tail<SBTile, CH>(b, len0, c);
+      if (RAG && x == 0) neutral_tail<SBTile, CH>(b, len0, c);
     };
     auto ckpt = [&](int64_t x) __attribute__((always_inline)) {
       return r4::ld32(rbc, cco + static_cast<uint32_t>(nb - 1 - x) * 64u, 0);
@@ -1343,8 +1347,8 @@ __global__ __launch_bounds__(3 * G * kWave) void backward_split_kernel(BwdArgs a
       const float* b = slot(x);
       const uint32_t t0 = tok0(x);
       const int len = clen(x);
-      store_kq<F, CH>(rgq, row4n, s, c, t0, len, b + SBTile::Q);
-      store_v<F, CH>(rgv, row8n, s, c, t0, len, b + SBTile::V);
+      store_kq<F, CH, RAG>(rgq, row4n, s, c, t0, len, b + SBTile::Q);
+      store_v<F, CH, RAG>(rgv, row8n, s, c, t0, len, b + SBTile::V);
     };
     auto store_cov = [&](int64_t x) __attribute__((always_inline)) {
       const float* b = slot(x);
@@ -1353,7 +1357,7 @@ __global__ __launch_bounds__(3 * G * kWave) void backward_split_kernel(BwdArgs a
       const uint32_t q4 = c < len ? o4 + t0 * 16u : kOob, q1 = c < CH / 4 ? o1 + t0 * 4u : kOob;
       const v4f zero = v4f{0.f, 0.f, 0.f, 0.f};
       const int c8 = c & (CH - 1), c2 = c & (CH / 4 - 1);
-      store_kq<F, CH>(rgk, row4n, s, c, t0, len, b + SBTile::K);
+      store_kq<F, CH, RAG>(rgk, row4n, s, c, t0, len, b + SBTile::K);
       if (a.gd) r4::st128<r4::kNtStore>(rgd, DYN ? *reinterpret_cast<const v4f*>(b + SBTile::D + 4 * c8) : zero, q4, 0);
       const v4f xp = DYN ? *reinterpret_cast<const v4f*>(b + SBTile::P + 4 * c2) : zero;
       const v4f xr = DYN ? *reinterpret_cast<const v4f*>(b + SBTile::R + 4 * c2) : zero;
@@ -1502,19 +1506,34 @@ hipError_t launch_forward_small(bool fixed, const FwdArgs& a, hipStream_t stream
 }
 
 namespace {
-template <int F, int G>
+template <int F, int G, bool RAG>
 void launch_backward_split_g(bool fixed, bool dyn, const BwdArgs& a, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>((a.n + G * sn::SPW - 1) / (G * sn::SPW))), block(3 * G * kWave);
-  if (fixed) hipLaunchKernelGGL((sn::backward_split_kernel<true, false, F, G>), grid, block, 0, stream, a);
-  else if (dyn) hipLaunchKernelGGL((sn::backward_split_kernel<false, true, F, G>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((sn::backward_split_kernel<false, false, F, G>), grid, block, 0, stream, a);
+  if (fixed) hipLaunchKernelGGL((sn::backward_split_kernel<true, false, F, G, RAG>), grid, block, 0, stream, a);
+  else if (dyn) hipLaunchKernelGGL((sn::backward_split_kernel<false, true, F, G, RAG>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((sn::backward_split_kernel<false, false, F, G, RAG>), grid, block, 0, stream, a);
 }
 // One group per workgroup while every workgroup has a CU of its own; beyond
 // that two groups per workgroup (one workgroup per CU up to 2048 sequences).
+template <int F, bool RAG>
+void launch_backward_split_rag(bool fixed, bool dyn, const BwdArgs& a, hipStream_t stream) {
+  if (a.n > static_cast<int64_t>(kSplitGroupsAbove)) launch_backward_split_g<F, 2, RAG>(fixed, dyn, a, stream);
+  else launch_backward_split_g<F, 1, RAG>(fixed, dyn, a, stream);
+}
 template <int F>
-void launch_backward_split(bool fixed, bool dyn, const BwdArgs& a, dim3, hipStream_t stream) {
-  if (a.n > static_cast<int64_t>(kSplitGroupsAbove)) launch_backward_split_g<F, 2>(fixed, dyn, a, stream);
-  else launch_backward_split_g<F, 1>(fixed, dyn, a, stream);
+void launch_backward_split(bool fixed, bool dyn, const BwdArgs& a, hipStream_t stream) {
+  // Two float32 groups run the ragged form at every T: it schedules 1 % better
+  // (2048 x 512, forward and backward: 166.5 us, against 168.5).
+  const bool two = a.n > kSplitGroupsAbove;
+  if (a.t % sn::SBTile::CH != 0 || (F == kInF32 && two)) launch_backward_split_rag<F, true>(fixed, dyn, a, stream);
+  else launch_backward_split_rag<F, false>(fixed, dyn, a, stream);
+}
+template <bool RAG>
+void launch_backward_row(bool fixed, bool dyn, const BwdArgs& a, dim3 grid, hipStream_t stream) {
+  const dim3 block(kWave);
+  if (fixed) hipLaunchKernelGGL((sn::backward_kernel<true, false, RAG>), grid, block, 0, stream, a);
+  else if (dyn) hipLaunchKernelGGL((sn::backward_kernel<false, true, RAG>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((sn::backward_kernel<false, false, RAG>), grid, block, 0, stream, a);
 }
 }  // namespace
 
@@ -1524,21 +1543,19 @@ hipError_t launch_backward_small(bool fixed, bool dyn, const BwdArgs& a, hipStre
   if (a.chunk != kRot4Chunk) return hipErrorInvalidValue;
   const int64_t blocks = (a.n + sn::SPW - 1) / sn::SPW;
   if (blocks == 0) return hipSuccess;
-  const dim3 grid(static_cast<unsigned>(blocks));
   switch (a.in_fmt) {
-    case kInBf16: launch_backward_split<kInBf16>(fixed, dyn, a, grid, stream); return hipGetLastError();
-    case kInE4M3: launch_backward_split<kInE4M3>(fixed, dyn, a, grid, stream); return hipGetLastError();
-    case kInE5M2: launch_backward_split<kInE5M2>(fixed, dyn, a, grid, stream); return hipGetLastError();
+    case kInBf16: launch_backward_split<kInBf16>(fixed, dyn, a, stream); return hipGetLastError();
+    case kInE4M3: launch_backward_split<kInE4M3>(fixed, dyn, a, stream); return hipGetLastError();
+    case kInE5M2: launch_backward_split<kInE5M2>(fixed, dyn, a, stream); return hipGetLastError();
     default: break;
   }
   if (a.n <= small_batch_limit(3)) {
-    launch_backward_split<kInF32>(fixed, dyn, a, grid, stream);
+    launch_backward_split<kInF32>(fixed, dyn, a, stream);
     return hipGetLastError();
   }
-  const dim3 block(kWave);
-  if (fixed) hipLaunchKernelGGL((sn::backward_kernel<true, false>), grid, block, 0, stream, a);
-  else if (dyn) hipLaunchKernelGGL((sn::backward_kernel<false, true>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((sn::backward_kernel<false, false>), grid, block, 0, stream, a);
+  const dim3 grid(static_cast<unsigned>(blocks));
+  if (a.t % sn::TT != 0) launch_backward_row<true>(fixed, dyn, a, grid, stream);
+  else launch_backward_row<false>(fixed, dyn, a, grid, stream);
   return hipGetLastError();
 }
 

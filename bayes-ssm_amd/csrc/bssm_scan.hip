@@ -20,7 +20,8 @@
 // 64 lanes in the factorization and a suffix pass of one thread per entry, took
 // 1400 and 1366 + 210 + 35 us.  (Step 1 on the VALU, lanes over the entries:
 // 185 us forward.)  Bound by the instruction stream of a wave, one to a SIMD:
-// 250 workgroups; step 1 grows with T^2 / 64.
+// 250 workgroups; step 1 grows with T^2 / 64.  Short sequences take a wave per
+// token (short_sequences has the line).
 //
 // The key dimension is a template parameter (runtime D is padded up to the
 // next instantiated size: the padded block of every matrix is the identity
@@ -646,6 +647,76 @@ __global__ __launch_bounds__(kWaves* kWave) void scan_backward_suffix_kernel(Ws 
     if (lane < len && e0 + i < entries) ws.at(b, t0, e0 + i)[len - 1 - lane] = x[i];
 }
 
+// The prior's gradients: SL_0 (lane i < D: row i), SN_0 (lane c < M: column c;
+// also row-major in sn), inv(P0) again (as in the forward), then gM0 = inv(P0)
+// SN_0 and gP0 = -inv(P0)^T (SL_0 + SN_0 M0^T) inv(P0)^T.  One wave; mat, idg and
+// tmp ([D][D]) are its LDS.
+template <int D>
+__device__ __forceinline__ void prior_grads(const ScanIn& a, int64_t b, int Dr, int lane, const float (&sl)[D],
+                                            const float (&snc)[D], const float* sn, float* mat, float* idg,
+                                            float* tmp, float* __restrict__ gm0, float* __restrict__ gc0) {
+  const int M = a.m;
+  const bool row_lane = lane < Dr, col_lane = lane < M;
+  const int rl = row_lane ? lane : 0;
+  float f[D], inv_diag = 1.f;
+  const float* P0 = a.c0 + (b * Dr + rl) * Dr;
+#pragma unroll
+  for (int j = 0; j < D; ++j) {
+    const float v = ld_or_zero(P0, j, Dr);
+    f[j] = row_lane ? v : (lane == j ? 1.f : 0.f);
+  }
+  chol_rows<D>(f, inv_diag, lane, mat, idg);
+  float lam0[D];
+#pragma unroll
+  for (int j = 0; j < D; ++j) lam0[j] = lane == j ? 1.f : 0.f;
+  chol_solve<D>(mat, idg, lam0);  // lane i < D: column i of inv(P0)
+  rows_to_lds<D>(lam0, mat, lane);  // mat = inv(P0)^T, row i = column i of inv(P0)
+  if (col_lane) {
+    // gM0[i][c] = sum_k inv(P0)[i][k] SN[k][c]
+#pragma unroll
+    for (int i = 0; i < D; ++i) {
+      float s = 0.f;
+#pragma unroll
+      for (int j = 0; j < D; ++j) s = fmaf(mat[j * D + i], snc[j], s);
+      if (i < Dr) gm0[(b * Dr + i) * M + lane] = s;
+    }
+  }
+  // gA = SL_0 + SN_0 M0^T (row owners, row i), then gP0 = -inv(P0)^T gA inv(P0)^T.
+  float ga[D];
+  const float* M0 = a.m0 + b * Dr * M;
+#pragma unroll
+  for (int j = 0; j < D; ++j) {
+    float s = sl[j];
+    if (row_lane && j < Dr)
+      for (int c = 0; c < M; ++c) s = fmaf(sn[lane * kMaxM + c], M0[j * M + c], s);
+    ga[j] = s;
+  }
+  float ta[D];
+#pragma unroll
+  for (int j = 0; j < D; ++j) {
+    // (gA inv(P0)^T)[i][j] = sum_k gA[i][k] inv(P0)[j][k]
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < D; ++i) s = fmaf(ga[i], mat[i * D + j], s);
+    ta[j] = s;
+  }
+  if (lane < D) {
+#pragma unroll
+    for (int j = 0; j < D; ++j) tmp[lane * D + j] = ta[j];
+  }
+  wave_fence();
+  if (row_lane) {
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      // gP0[i][j] = -sum_k inv(P0)[k][i] (gA inv(P0)^T)[k][j]
+      float s = 0.f;
+#pragma unroll
+      for (int i = 0; i < D; ++i) s = fmaf(mat[lane * D + i], tmp[i * D + j], s);
+      if (j < Dr) gc0[(b * Dr + lane) * Dr + j] = -s;
+    }
+  }
+}
+
 template <int D, bool VEC>
 __global__ __launch_bounds__(kWaves* kWave) void scan_backward_input_kernel(ScanIn a, Ws ws, float* __restrict__ gk,
                                                                            float* __restrict__ gv,
@@ -725,8 +796,6 @@ __global__ __launch_bounds__(kWaves* kWave) void scan_backward_input_kernel(Scan
   if (wave == 0 && valid)
     gr[t] = -static_cast<float>((zsum[0][lane] + zsum[1][lane]) + (zsum[2][lane] + zsum[3][lane])) * rinv * rinv;
   if (t0 != 0 || wave != 0) return;
-  // The prior: SL_0 and SN_0 of token 0, inv(P0) again (as in the forward), then
-  // gM0 = inv(P0) SN_0 and gP0 = -inv(P0)^T (SL_0 + SN_0 M0^T) inv(P0)^T.
   const bool row_lane = lane < Dr, col_lane = lane < M;
   const int rl = row_lane ? lane : 0;
   float sl[D], snc[D];
@@ -743,65 +812,340 @@ __global__ __launch_bounds__(kWaves* kWave) void scan_backward_input_kernel(Scan
     for (int i = 0; i < D; ++i) sn[i * kMaxM + lane] = snc[i];
   }
   wave_fence();
-  float f[D], inv_diag = 1.f;
+  // tmp takes the place of carry, which no other wave reads now.
+  prior_grads<D>(a, b, Dr, lane, sl, snc, sn, mat, idg, reinterpret_cast<float*>(carry), gm0, gc0);
+}
+
+// ------------------------------------------------------- short sequences
+// One wave per (b, t): a workgroup of 64 tokens takes the time of 64 whatever
+// part of them its row has.  Two lane roles: row owners (lane i < D) hold row i
+// of the precision, then of its factor; column owners (lane c < M) hold column c
+// of the natural parameter and solve for column c of the mean.  The prefix is
+// summed token by token (rows s are uniform across the wave and load as scalars),
+// eight to a partial sum.  EXACT: the key dimension equals D.  At D = M = 16 a
+// batch of 2048 rows of 8 tokens takes 322 us backward, against 484 us with a
+// workgroup per 64 tokens; 8192 of one token, forward and backward through the
+// API, 381 against 2612 us.
+// On return LDS mat / idg hold the factor of L_t and 1 / its diagonal, and the
+// column owners column c of M_t = L_t^{-1} N_t in x.
+template <int D, bool EXACT>
+__device__ __forceinline__ void token_state(const ScanIn& a, int64_t b, int64_t t, int lane, float* mat, float* tr,
+                                            float* idg, float (&x)[D]) {
+  const int Dr = EXACT ? D : a.d, M = a.m;
+  const bool row_lane = lane < Dr, col_lane = lane < M;
+  const int rl = row_lane ? lane : 0, cl = col_lane ? lane : 0;
+  // inv(P0): factor P0 (padded with the identity), then lane c < D solves for
+  // column c of the identity; column c of inv(P0) is its row c (symmetric).
+  float l[D], inv_diag = 1.f, lam0[D];
   const float* P0 = a.c0 + (b * Dr + rl) * Dr;
 #pragma unroll
   for (int j = 0; j < D; ++j) {
     const float v = ld_or_zero(P0, j, Dr);
-    f[j] = row_lane ? v : (lane == j ? 1.f : 0.f);
+    l[j] = row_lane ? v : (lane == j ? 1.f : 0.f);
   }
-  chol_rows<D>(f, inv_diag, lane, mat, idg);
-  float lam0[D];
+  chol_rows<D>(l, inv_diag, lane, mat, idg);
 #pragma unroll
   for (int j = 0; j < D; ++j) lam0[j] = lane == j ? 1.f : 0.f;
-  chol_solve<D>(mat, idg, lam0);  // lane i < D: column i of inv(P0)
-  rows_to_lds<D>(lam0, mat, lane);  // mat = inv(P0)^T, row i = column i of inv(P0)
-  if (col_lane) {
-    // gM0[i][c] = sum_k inv(P0)[i][k] SN[k][c]
+  chol_solve<D>(mat, idg, lam0);
+  wave_fence();
+  rows_to_lds<D>(lam0, mat, lane);  // mat = inv(P0)
+  // N_t column c starts at inv(P0) M0[:, c].
+  float m0c[D];
+  const float* M0 = a.m0 + b * Dr * M + cl;
 #pragma unroll
-    for (int i = 0; i < D; ++i) {
-      float s = 0.f;
+  for (int k = 0; k < D; ++k) {
+    const float v = M0[(k < Dr ? k : 0) * M];
+    m0c[k] = (col_lane && k < Dr) ? v : 0.f;
+  }
 #pragma unroll
-      for (int j = 0; j < D; ++j) s = fmaf(mat[j * D + i], snc[j], s);
-      if (i < Dr) gm0[(b * Dr + i) * M + lane] = s;
+  for (int i = 0; i < D; ++i) {
+    float li[D];
+    lds_row<D>(mat, i, li);
+    float n0 = 0.f;
+#pragma unroll
+    for (int k = 0; k < D; ++k) n0 = fmaf(li[k], m0c[k], n0);
+    x[i] = n0;
+  }
+  // Prefix sums over s < t: row owners row i of sum k (k / r)^T, column
+  // owners column c of sum (k / r) v^T.  The token's own term, often far larger,
+  // is added by one fma (as in the 64-token kernels).
+  float acc[D], ks[D], own, vc, rinv;
+#pragma unroll
+  for (int j = 0; j < D; ++j) acc[j] = 0.f;
+  const float* kb = a.k + b * a.T * Dr;
+  const float* vb = a.v + b * a.T * M + cl;
+  const float* rb = a.r + b * a.T;
+  auto token = [&](int64_t s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < D; ++j) ks[j] = ld_or_zero(kb + s * Dr, j, Dr);
+    rinv = 1.0f / rb[s];
+    const float kown = kb[s * Dr + rl], vown = vb[s * M];
+    own = row_lane ? kown * rinv : 0.f;
+    vc = col_lane ? vown : 0.f;
+  };
+  for (int64_t s0 = 0; s0 < t; s0 += 8) {
+    float pa[D], px[D];
+#pragma unroll
+    for (int j = 0; j < D; ++j) pa[j] = px[j] = 0.f;
+    const int64_t end = s0 + 8 < t ? s0 + 8 : t;
+#pragma unroll 4
+    for (int64_t s = s0; s < end; ++s) {
+      token(s);
+#pragma unroll
+      for (int j = 0; j < D; ++j) {
+        pa[j] = fmaf(own, ks[j], pa[j]);
+        px[j] = fmaf(ks[j] * rinv, vc, px[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      acc[j] += pa[j];
+      x[j] += px[j];
     }
   }
-  // gA = SL_0 + SN_0 M0^T (row owners, row i), then gP0 = -inv(P0)^T gA inv(P0)^T.
-  float ga[D];
-  const float* M0 = a.m0 + b * Dr * M;
+  token(t);
 #pragma unroll
-  for (int j = 0; j < D; ++j) {
-    float s = sl[j];
-    if (row_lane && j < Dr)
-      for (int c = 0; c < M; ++c) s = fmaf(sn[lane * kMaxM + c], M0[j * M + c], s);
-    ga[j] = s;
-  }
-  float ta[D];
+  for (int j = 0; j < D; ++j) x[j] = fmaf(ks[j] * rinv, vc, x[j]);
+  // L_t = inv(P0) + prefix, symmetrized through LDS, on the row owners.
+  // Padded rows (lanes Dr .. D - 1) keep the identity.
+  float lam[D];
 #pragma unroll
-  for (int j = 0; j < D; ++j) {
-    // (gA inv(P0)^T)[i][j] = sum_k gA[i][k] inv(P0)[j][k]
-    float s = 0.f;
-#pragma unroll
-    for (int i = 0; i < D; ++i) s = fmaf(ga[i], mat[i * D + j], s);
-    ta[j] = s;
-  }
-  // The rows of gA inv(P0)^T go where carry stood, which no other wave reads now.
-  float* tmp = reinterpret_cast<float*>(carry);
+  for (int j = 0; j < D; ++j) lam[j] = fmaf(own, ks[j], lam0[j] + acc[j]);
   if (lane < D) {
 #pragma unroll
-    for (int j = 0; j < D; ++j) tmp[lane * D + j] = ta[j];
+    for (int j = 0; j < D; ++j) tr[j * D + lane] = lam[j];
+  }
+  wave_fence();
+  if (lane < D) {
+#pragma unroll
+    for (int j = 0; j < D; ++j) lam[j] = (lam[j] + tr[lane * D + j]) * 0.5f;
+  }
+  wave_fence();
+  chol_rows<D>(lam, inv_diag, lane, mat, idg);  // mat = factor of L_t
+  chol_solve<D>(mat, idg, x);
+}
+
+template <int D, bool EXACT>
+__global__ __launch_bounds__(kWave) void scan_forward_short_kernel(ScanIn a, float* __restrict__ out,
+                                                                   float* __restrict__ mT, float* __restrict__ cT) {
+  __shared__ float mat[D * D], tr[D * D], idg[D];
+  const int Dr = EXACT ? D : a.d, M = a.m, lane = threadIdx.x;
+  const int64_t b = blockIdx.y, t = blockIdx.x;
+  float x[D];
+  token_state<D, EXACT>(a, b, t, lane, mat, tr, idg, x);
+  const bool last = t == a.T - 1;
+  if (lane < M) {
+    const float* qt = a.q + (b * a.T + t) * Dr;
+    float y = 0.f;
+#pragma unroll
+    for (int i = 0; i < D; ++i) y = fmaf(x[i], ld_or_zero(qt, i, Dr), y);
+    out[(b * a.T + t) * M + lane] = y;
+    if (last) {
+#pragma unroll
+      for (int i = 0; i < D; ++i)
+        if (i < Dr) mT[(b * Dr + i) * M + lane] = x[i];
+    }
+  }
+  if (last) {
+    // P_T = L_T^{-1}: lane c solves for column c of the identity.
+    float e[D];
+#pragma unroll
+    for (int i = 0; i < D; ++i) e[i] = lane == i ? 1.f : 0.f;
+    chol_solve<D>(mat, idg, e);
+    if (lane < Dr) {
+#pragma unroll
+      for (int i = 0; i < D; ++i)
+        if (i < Dr) cT[(b * Dr + i) * Dr + lane] = e[i];
+    }
+  }
+}
+
+// The backward's passes (above) with a wave per token: gL_t [D, D] and gN_t [D,
+// M], token by token in the workspace (in this order), their suffix sums in place
+// (a thread an entry), then a wave per token again.  Sums as above: float64
+// where gr would show their rounding.
+template <int D, bool EXACT>
+__global__ __launch_bounds__(kWave) void scan_backward_short_token_kernel(ScanIn a, const float* __restrict__ gy,
+                                                                          const float* __restrict__ gmT,
+                                                                          const float* __restrict__ gcT,
+                                                                          float* __restrict__ ws_gl,
+                                                                          float* __restrict__ ws_gn,
+                                                                          float* __restrict__ gq) {
+  __shared__ float mat[D * D], idg[D];
+  __shared__ double tr[D * D];      // transpose staging
+  __shared__ float mt[D * kMaxM];   // M_t, row-major
+  __shared__ float gn[D * kMaxM];   // gN_t, row-major
+  __shared__ float pt[D * D];       // P_T (last token); token_state's staging before it
+  __shared__ float gys[kMaxM];
+  const int Dr = EXACT ? D : a.d, M = a.m, lane = threadIdx.x;
+  const int64_t b = blockIdx.y, t = blockIdx.x, row = b * a.T + t;
+  const bool row_lane = lane < Dr, col_lane = lane < M, last = t == a.T - 1;
+  float x[D];
+  token_state<D, EXACT>(a, b, t, lane, mat, pt, idg, x);
+  // Column owners: G[:, c] = q_t gy_t[c] (+ gM_T[:, c]), then gN[:, c] = L_t^{-1} G[:, c].
+  float g[D];
+  const float gyc = col_lane ? gy[row * M + lane] : 0.f;
+#pragma unroll
+  for (int i = 0; i < D; ++i) {
+    float v = ld_or_zero(a.q + row * Dr, i, Dr) * gyc;
+    if (last && gmT != nullptr && col_lane && i < Dr) v += gmT[(b * Dr + i) * M + lane];
+    g[i] = col_lane ? v : 0.f;
+  }
+  chol_solve<D>(mat, idg, g);
+  if (col_lane) {
+    gys[lane] = gyc;
+#pragma unroll
+    for (int i = 0; i < D; ++i) {
+      mt[i * kMaxM + lane] = x[i];
+      gn[i * kMaxM + lane] = g[i];
+      if (i < Dr) ws_gn[(row * Dr + i) * M + lane] = g[i];
+    }
+  }
+  if (last && gcT != nullptr) {
+    float e[D];
+#pragma unroll
+    for (int i = 0; i < D; ++i) e[i] = lane == i ? 1.f : 0.f;
+    chol_solve<D>(mat, idg, e);  // lane c < D: column c of P_T (= row c)
+    if (lane < D) {
+#pragma unroll
+      for (int i = 0; i < D; ++i) pt[lane * D + i] = e[i];
+    }
+  }
+  wave_fence();
+  // Row owners: gq_t[i] = sum_c M_t[i, c] gy_t[c] and row i of -gN_t M_t^T.
+  double gl[D];
+  if (lane < D) {
+    double acc = 0.;
+#pragma unroll
+    for (int j = 0; j < D; ++j) gl[j] = 0.;
+    for (int c = 0; c < M; ++c) {
+      acc = fma(static_cast<double>(mt[lane * kMaxM + c]), static_cast<double>(gys[c]), acc);
+      const double gc = -static_cast<double>(gn[lane * kMaxM + c]);
+#pragma unroll
+      for (int j = 0; j < D; ++j) gl[j] = fma(gc, static_cast<double>(mt[j * kMaxM + c]), gl[j]);
+    }
+    if (row_lane) gq[row * Dr + lane] = static_cast<float>(acc);
+  }
+  if (last && gcT != nullptr && lane < D) {
+    // -(P_T gP_T P_T)[i][:]: row i of A = P_T gP_T in registers, then A P_T
+    // (gP_T and the padded block of P_T: zero and the identity).
+    float ar[D];
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      float acc = 0.f;
+#pragma unroll
+      for (int k = 0; k < D; ++k) {
+        const float gkj = (k < Dr && j < Dr) ? gcT[(b * Dr + k) * Dr + j] : 0.f;
+        acc = fmaf(pt[lane * D + k], gkj, acc);
+      }
+      ar[j] = acc;
+    }
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      float acc = 0.f;
+#pragma unroll
+      for (int k = 0; k < D; ++k) acc = fmaf(ar[k], pt[k * D + j], acc);
+      gl[j] -= acc;
+    }
+  }
+  // Symmetrize through LDS and store row i of gL_t.
+  if (lane < D) {
+#pragma unroll
+    for (int j = 0; j < D; ++j) tr[j * D + lane] = gl[j];
   }
   wave_fence();
   if (row_lane) {
 #pragma unroll
-    for (int j = 0; j < D; ++j) {
-      // gP0[i][j] = -sum_k inv(P0)[k][i] (gA inv(P0)^T)[k][j]
-      float s = 0.f;
-#pragma unroll
-      for (int i = 0; i < D; ++i) s = fmaf(mat[lane * D + i], tmp[i * D + j], s);
-      if (j < Dr) gc0[(b * Dr + lane) * Dr + j] = -s;
-    }
+    for (int j = 0; j < D; ++j)
+      if (j < Dr) ws_gl[(row * Dr + lane) * Dr + j] = static_cast<float>((gl[j] + tr[lane * D + j]) * 0.5);
   }
+}
+
+// Loads run kSuffixBatch tokens ahead of the dependent sum.
+constexpr int kSuffixBatch = 8;
+__global__ __launch_bounds__(256) void scan_backward_short_suffix_kernel(float* __restrict__ ws_gl,
+                                                                         float* __restrict__ ws_gn, int64_t T,
+                                                                         int e_gl, int e_gn) {
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  if (e >= e_gl + e_gn) return;
+  const int64_t b = blockIdx.y;
+  const bool gl = e < e_gl;
+  const int w = gl ? e_gl : e_gn;
+  float* p = gl ? ws_gl + b * T * e_gl + e : ws_gn + b * T * e_gn + (e - e_gl);
+  double acc = 0.;
+  int64_t t = T;
+  while (t > 0) {
+    const int n = t >= kSuffixBatch ? kSuffixBatch : static_cast<int>(t);
+    float x[kSuffixBatch];
+#pragma unroll
+    for (int i = 0; i < kSuffixBatch; ++i) x[i] = i < n ? p[(t - 1 - i) * w] : 0.f;
+#pragma unroll
+    for (int i = 0; i < kSuffixBatch; ++i) {
+      if (i < n) {
+        acc += x[i];
+        p[(t - 1 - i) * w] = static_cast<float>(acc);
+      }
+    }
+    t -= n;
+  }
+}
+
+template <int D, bool EXACT>
+__global__ __launch_bounds__(kWave) void scan_backward_short_input_kernel(ScanIn a, const float* __restrict__ ws_gl,
+                                                                          const float* __restrict__ ws_gn,
+                                                                          float* __restrict__ gk,
+                                                                          float* __restrict__ gv,
+                                                                          float* __restrict__ gr,
+                                                                          float* __restrict__ gm0,
+                                                                          float* __restrict__ gc0) {
+  __shared__ float mat[D * D], tmp[D * D], idg[D], sn[D * kMaxM];  // sn: SN_s, row-major
+  __shared__ double part[kWave];
+  const int Dr = EXACT ? D : a.d, M = a.m, lane = threadIdx.x;
+  const int64_t b = blockIdx.y, s = blockIdx.x, row = b * a.T + s;
+  const bool row_lane = lane < Dr, col_lane = lane < M;
+  const int rl = row_lane ? lane : 0;
+  // Suffix sums over t >= s: row owners row i of SL, column owners column c of SN.
+  float sl[D], snc[D];
+  const float* glt = ws_gl + (row * Dr + rl) * Dr;
+  const float* gnt = ws_gn + row * Dr * M + (col_lane ? lane : 0);
+#pragma unroll
+  for (int j = 0; j < D; ++j) {
+    const float l = glt[j < Dr ? j : 0], n = gnt[(j < Dr ? j : 0) * M];
+    sl[j] = (row_lane && j < Dr) ? l : 0.f;
+    snc[j] = (col_lane && j < Dr) ? n : 0.f;
+  }
+  if (col_lane) {
+#pragma unroll
+    for (int i = 0; i < D; ++i) sn[i * kMaxM + lane] = snc[i];
+  }
+  wave_fence();
+  const float* ks = a.k + row * Dr;
+  const float* vs = a.v + row * M;
+  const float rinv = 1.0f / a.r[row];
+  // gk_s[i] = (2 (SL k)_i + (SN v)_i) / r;  k^T SL k and k^T SN v for gr.
+  double contrib = 0.;
+  if (row_lane) {
+    double l = 0., n = 0.;
+#pragma unroll
+    for (int j = 0; j < D; ++j) l = fma(static_cast<double>(sl[j]), static_cast<double>(ld_or_zero(ks, j, Dr)), l);
+    for (int c = 0; c < M; ++c) n = fma(static_cast<double>(sn[lane * kMaxM + c]), static_cast<double>(vs[c]), n);
+    gk[row * Dr + lane] = static_cast<float>(2. * l + n) * rinv;
+    contrib = (l + n) * ks[lane];
+  }
+  part[lane] = contrib;
+  if (col_lane) {
+    double acc = 0.;
+#pragma unroll
+    for (int i = 0; i < D; ++i) acc = fma(static_cast<double>(snc[i]), static_cast<double>(ld_or_zero(ks, i, Dr)), acc);
+    gv[row * M + lane] = static_cast<float>(acc) * rinv;
+  }
+  wave_fence();
+  if (lane == 0) {
+    double z = 0.;
+    for (int i = 0; i < Dr; ++i) z += part[i];
+    gr[row] = -static_cast<float>(z) * rinv * rinv;
+  }
+  if (s == 0) prior_grads<D>(a, b, Dr, lane, sl, snc, sn, mat, idg, tmp, gm0, gc0);
 }
 
 // Key dimensions 17..32: the general kernel with the matrices in LDS (a
@@ -932,8 +1276,59 @@ __global__ void copy_prior_kernel(const float* __restrict__ mean0, const float* 
   if (i < nc) cT[i] = cov0[i];
 }
 
+// Whether the kernels with a wave per token are the faster ones: fits of both
+// sides' times at 24 pairs of batch (1 to 2048) and T (1 to 96) for each of 15
+// key and value dimensions, at most 13 % off the faster side.  A workgroup of 64
+// tokens takes the same time whatever T; it grows with the value columns, which
+// its waves take in turn and a wave per token in lanes, as the latter grows with
+// T.  While every token's wave has a SIMD of its own (1024; for twice as many the
+// line is halved) the column solves decide: D = M = 16 forward, 16 x 16 tokens
+// 16.9 against 22.3 us, 16 x 64 32.9 against 22.6; backward, 16 x 32 52.0 against
+// 58.8, 16 x 64 69.1 against 59.5.  With more waves their work does: forward 2048
+// x 4 59.5 against 103 us, 2048 x 8 132 against 103; backward 2048 x 8 322 against
+// 484, 2048 x 16 668 against 496.  A key dimension that is padded costs the wave
+// per token its branches.
+bool short_sequences(bool backward, int64_t b, int64_t t, int d, int m) {
+  const bool wide = d > 8, padded = d == 3 || (d > 4 && d != 8 && d != 16);
+  int64_t idle, busy;
+  if (backward) {
+    idle = wide ? 22 + 2 * m : 4 + 7 * m / 10;
+    if (padded) idle = idle * 3 / 5;
+    busy = (wide ? 9 : 4) + m / 10;
+  } else {
+    idle = wide ? 12 + 6 * m / 5 : 1 + 7 * m / 10;
+    if (padded) idle = idle * 7 / 20;
+    busy = 4 + m / 8;
+  }
+  const int64_t waves = b * t;
+  return t <= (waves <= 1024 ? idle : waves <= 2048 && idle / 2 > busy ? idle / 2 : busy);
+}
+
+template <int D, bool EXACT>
+void launch_scan_backward_short(const ScanIn& a, const float* gy, const float* gmT, const float* gcT, float* ws,
+                                float* gk, float* gv, float* gq, float* gr, float* gm0, float* gc0, int64_t b,
+                                hipStream_t stream) {
+  const dim3 grid(static_cast<unsigned>(a.T), static_cast<unsigned>(b)), block(kWave);
+  float* ws_gl = ws;
+  float* ws_gn = ws + b * a.T * a.d * a.d;
+  hipLaunchKernelGGL((scan_backward_short_token_kernel<D, EXACT>), grid, block, 0, stream, a, gy, gmT, gcT, ws_gl,
+                     ws_gn, gq);
+  const int e_gl = a.d * a.d, e_gn = a.d * a.m;
+  hipLaunchKernelGGL(scan_backward_short_suffix_kernel,
+                     dim3(static_cast<unsigned>((e_gl + e_gn + 255) / 256), static_cast<unsigned>(b)), dim3(256), 0,
+                     stream, ws_gl, ws_gn, a.T, e_gl, e_gn);
+  hipLaunchKernelGGL((scan_backward_short_input_kernel<D, EXACT>), grid, block, 0, stream, a, ws_gl, ws_gn, gk, gv,
+                     gr, gm0, gc0);
+}
+
 template <int D>
 hipError_t launch_scan(const ScanIn& a, float* y, float* mT, float* cT, int64_t b, hipStream_t stream) {
+  if (short_sequences(false, b, a.T, a.d, a.m)) {
+    const dim3 grid(static_cast<unsigned>(a.T), static_cast<unsigned>(b)), block(kWave);
+    if (a.d == D) hipLaunchKernelGGL((scan_forward_short_kernel<D, true>), grid, block, 0, stream, a, y, mT, cT);
+    else hipLaunchKernelGGL((scan_forward_short_kernel<D, false>), grid, block, 0, stream, a, y, mT, cT);
+    return hipGetLastError();
+  }
   const dim3 grid(static_cast<unsigned>((a.T + kTok - 1) / kTok), static_cast<unsigned>(b)), block(kWaves * kWave);
   if (a.d == D && D % 4 == 0 && a.m % 4 == 0)
     hipLaunchKernelGGL((scan_forward_kernel<D, (D % 4 == 0)>), grid, block, 0, stream, a, y, mT, cT);
@@ -959,6 +1354,11 @@ template <int D>
 hipError_t launch_scan_backward(const ScanIn& a, const float* gy, const float* gmT, const float* gcT, float* ws,
                                 float* gk, float* gv, float* gq, float* gr, float* gm0, float* gc0, int64_t b,
                                 hipStream_t stream) {
+  if (short_sequences(true, b, a.T, a.d, a.m)) {
+    if (a.d == D) launch_scan_backward_short<D, true>(a, gy, gmT, gcT, ws, gk, gv, gq, gr, gm0, gc0, b, stream);
+    else launch_scan_backward_short<D, false>(a, gy, gmT, gcT, ws, gk, gv, gq, gr, gm0, gc0, b, stream);
+    return hipGetLastError();
+  }
   const Ws w{ws, a.T, a.d, a.m};
   if (a.d == D && D % 4 == 0 && a.m % 4 == 0)
     launch_scan_backward_vec<D, (D % 4 == 0)>(a, gy, gmT, gcT, w, gk, gv, gq, gr, gm0, gc0, b, stream);

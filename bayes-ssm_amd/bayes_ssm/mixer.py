@@ -87,11 +87,13 @@ def _partials(chunk: int, b: int, heads: int, device: torch.device) -> Tensor:
     return torch.empty(rows, VALUE_DIM, device=device, dtype=torch.float32)
 
 
-def _any_shape_call(heads: int, t: int, initial_mean: Optional[Tensor], initial_covariance: Optional[Tensor],
-                    chunk_length: Optional[int], denominator_floor: float, optimized: bool) -> bool:
+def _any_shape_call(b: int, heads: int, t: int, initial_mean: Optional[Tensor],
+                    initial_covariance: Optional[Tensor], chunk_length: Optional[int], denominator_floor: float,
+                    optimized: bool) -> bool:
     """Off whole tiles the kernels take calls that the op chain's own argument checks would pass (the values aside):
-    the default prior, a valid chunk length and floor, the optimized core, no switch that selects another core."""
-    return (heads > 0 and heads % 4 == 0 and t > 0 and optimized and initial_mean is None
+    a batch, the default prior, a valid chunk length and floor, the optimized core, no switch that selects another
+    core."""
+    return (b > 0 and heads > 0 and heads % 4 == 0 and t > 0 and optimized and initial_mean is None
             and initial_covariance is None and isinstance(denominator_floor, Real) and math.isfinite(denominator_floor)
             and (chunk_length is None or (isinstance(chunk_length, int) and not isinstance(chunk_length, bool)
                                           and chunk_length > 0))
@@ -319,7 +321,7 @@ def bayes_mixer_core(
             raise ValueError(f"{name} must have shape [B, T, H*{w}] = {(b, t, w * heads)}, got {tuple(x.shape)}")
     lds = _fused_eligible(projections, heads, whole=False)
     whole = _whole_tiles(heads, t)
-    if lds is not None and (whole or (_any_shape_call(heads, t, initial_mean, initial_covariance, chunk_length,
+    if lds is not None and (whole or (_any_shape_call(b, heads, t, initial_mean, initial_covariance, chunk_length,
                                                       denominator_floor, optimized)
                                       and _in_limits(t, heads, *lds))):
         _hip.load()  # on a GPU the fused path never degrades silently
@@ -455,7 +457,7 @@ def bayes_mixer_readout(
     ldg = _row_stride(gate, t) if gate.dtype == torch.bfloat16 and gate.device == q_proj.device else None
     whole = _whole_tiles(heads, t)
     if lds is not None and ldg is not None and (whole or (
-            _any_shape_call(heads, t, initial_mean, initial_covariance, chunk_length, denominator_floor, optimized)
+            _any_shape_call(b, heads, t, initial_mean, initial_covariance, chunk_length, denominator_floor, optimized)
             and _in_limits(t, heads, *lds, ldg)
             and denominator_floor > 0 and eps >= 0 and norm_weight.dtype == torch.bfloat16
             and norm_weight.device == q_proj.device)):
@@ -615,7 +617,7 @@ def bayes_mixer_block(
     ld = _row_stride(projected, t) if projected.is_cuda and projected.dtype == torch.bfloat16 else None
     whole = _whole_tiles(heads, t)
     fused = (ld is not None and t > 0
-             and (whole or (_any_shape_call(heads, t, initial_mean, initial_covariance, chunk_length,
+             and (whole or (_any_shape_call(b, heads, t, initial_mean, initial_covariance, chunk_length,
                                             denominator_floor, optimized)
                             and _in_limits(t, heads, ld)
                             and conv_weight.dtype == norm_weight.dtype == torch.bfloat16

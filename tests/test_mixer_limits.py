@@ -40,6 +40,12 @@ def test_limits_are_the_entry_points(name, heads, ld, t):
     assert mixer._in_limits(t, heads, ld) == _entry_takes(name, t, heads, ld)
 
 
+def test_an_empty_batch_is_left_to_the_op_chain():
+    """The block's weight gradients would come back unwritten from a call without work."""
+    assert mixer._any_shape_call(1, 8, 7, None, None, None, 1e-6, True)
+    assert not mixer._any_shape_call(0, 8, 7, None, None, None, 1e-6, True)
+
+
 class _OpChain(Exception):
     pass
 

@@ -139,13 +139,13 @@ class _LargeScan:
         return not self._flags.any()
 
 
-def _fused_eligible(projections: tuple[Tensor, ...], heads: int, whole: bool = True) -> Optional[tuple[int, ...]]:
-    """Row strides of projections the kernels can address (with ``whole``: in whole tiles), else None."""
+def _fused_eligible(projections: tuple[Tensor, ...], heads: int) -> Optional[tuple[int, ...]]:
+    """Row strides of projections the kernels can address, else None."""
     q = projections[0]
     if q.device.type != "cuda" or q.ndim != 3:
         return None
     b, t, _ = q.shape
-    if t <= 0 or (not _whole_tiles(heads, t) if whole else heads % 4 != 0):
+    if t <= 0 or heads % 4 != 0:
         return None
     lds = []
     for x, w in zip(projections, _WIDTHS):
@@ -319,7 +319,7 @@ def bayes_mixer_core(
     for x, w, name in zip(projections, _WIDTHS, ("q_proj", "k_proj", "v_proj", "decay_logits", "noise")):
         if tuple(x.shape) != (b, t, w * heads):
             raise ValueError(f"{name} must have shape [B, T, H*{w}] = {(b, t, w * heads)}, got {tuple(x.shape)}")
-    lds = _fused_eligible(projections, heads, whole=False)
+    lds = _fused_eligible(projections, heads)
     whole = _whole_tiles(heads, t)
     if lds is not None and (whole or (_any_shape_call(b, heads, t, initial_mean, initial_covariance, chunk_length,
                                                       denominator_floor, optimized)
@@ -453,7 +453,7 @@ def bayes_mixer_readout(
         raise ValueError("norm_weight must have shape [8]")
     eps = torch.finfo(torch.float32).eps if norm_eps is None else float(norm_eps)
     projections = (q_proj, k_proj, v_proj, decay_logits, noise)
-    lds = _fused_eligible(projections, heads, whole=False)
+    lds = _fused_eligible(projections, heads)
     ldg = _row_stride(gate, t) if gate.dtype == torch.bfloat16 and gate.device == q_proj.device else None
     whole = _whole_tiles(heads, t)
     if lds is not None and ldg is not None and (whole or (

@@ -205,8 +205,8 @@ int mixer_check(const char* fn, const void* const (&in)[5], const int64_t (&ld)[
     return fail(BSSM_ERR_UNSUPPORTED, "%s: needs heads a positive multiple of 4, T > 0 and chunk == %d (got h=%lld "
                 "t=%lld chunk=%lld)", fn, bssm::kRot4Chunk, (long long)h, (long long)t, (long long)chunk);
   if (!any_shape && (h % 16 != 0 || t <= 0 || t % 4 != 0 || chunk != bssm::kRot4Chunk))
-    return fail(BSSM_ERR_UNSUPPORTED, "%s: needs heads %% 16 == 0, T a positive multiple of 4 and chunk == %d (got h=%lld t=%lld "
-                "chunk=%lld)", fn, bssm::kRot4Chunk, (long long)h, (long long)t, (long long)chunk);
+    return fail(BSSM_ERR_UNSUPPORTED, "%s: needs heads %% 16 == 0, T a positive multiple of 4 and chunk == %d "
+                "(got h=%lld t=%lld chunk=%lld)", fn, bssm::kRot4Chunk, (long long)h, (long long)t, (long long)chunk);
   if (b * ((h + 15) / 16) > 0x7fffffff) return fail(BSSM_ERR_ARGUMENT, "%s: batch * heads too large", fn);
   const int64_t nb = (t + chunk - 1) / chunk;
   if ((nb + 1) * 128 * 16 >= ((int64_t)1 << 31) || t * h * 32 >= ((int64_t)1 << 31))
@@ -1039,22 +1039,22 @@ int bssm_forward_chunked_rotation(int key_dim, int value_dim, const float* keys,
                                   const float* cov0, float* out, float* mean_final, float* cov_final, float* bmean,
                                   float* bcov, int64_t n, int64_t t, int64_t chunk, float denominator_floor,
                                   void* stream) {
-  return rotation_forward("bssm_forward_chunked_rotation", key_dim, value_dim, keys, values, queries, radii, angles, process, observation, mean0,
-                          cov0, out, mean_final, cov_final, bmean, bcov, n, t, chunk, denominator_floor, nullptr, nullptr,
-                          stream);
+  return rotation_forward("bssm_forward_chunked_rotation", key_dim, value_dim, keys, values, queries, radii, angles,
+                          process, observation, mean0, cov0, out, mean_final, cov_final, bmean, bcov, n, t, chunk,
+                          denominator_floor, nullptr, nullptr, stream);
 }
 
 int bssm_forward_chunked_rotation_checked(int key_dim, int value_dim, const float* keys, const float* values,
                                           const float* queries, const float* radii, const float* angles,
                                           const float* process, const float* observation, const float* mean0,
-                                          const float* cov0, float* out, float* mean_final, float* cov_final, float* bmean,
-                                          float* bcov, int64_t n, int64_t t, int64_t chunk, float denominator_floor,
-                                          int* faults, int* checked, void* stream) {
+                                          const float* cov0, float* out, float* mean_final, float* cov_final,
+                                          float* bmean, float* bcov, int64_t n, int64_t t, int64_t chunk,
+                                          float denominator_floor, int* faults, int* checked, void* stream) {
   const char* fn = "bssm_forward_chunked_rotation_checked";
   if (checked == nullptr) return fail(BSSM_ERR_ARGUMENT, "%s: checked is null", fn);
   return rotation_forward(fn, key_dim, value_dim, keys, values, queries, radii, angles, process, observation, mean0,
-                          cov0, out, mean_final, cov_final, bmean, bcov, n, t, chunk, denominator_floor, faults, checked,
-                          stream);
+                          cov0, out, mean_final, cov_final, bmean, bcov, n, t, chunk, denominator_floor, faults,
+                          checked, stream);
 }
 
 int bssm_backward_chunked_rotation(int key_dim, int value_dim, const float* keys, const float* values,

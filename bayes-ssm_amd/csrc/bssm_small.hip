@@ -611,21 +611,18 @@ __global__ __launch_bounds__(2 * G * kWave) void forward_split_kernel(FwdArgs a)
 // (sin and cos by sincos_rad) and stored with both signs of s, so that a lane
 // reads its row's (R_ii, R_{i,i^1}) as one pair; the process variances are
 // stored beside zeros, which the lanes off the even diagonal read (adding a
-// zero instead of selecting).  The mean pair is
-// kept in the lane's own column order as in forward_kernel; its row mixing
-// is one quad exchange.
+// zero instead of selecting).  The mean pair is kept in the lane's own column
+// order as in forward_kernel; its row mixing is one quad exchange.
 struct RTile {
   // k, q [TT][4], v / y [TT][8], (c0, -s0, c0, s0, c1, -s1, c1, s1) [TT][8],
   // (p0, 0, p1, 0) [TT][4], r [TT]; sequences 8 banks apart (488 mod 32).
   static constexpr int K = 0, Q = 64, V = 128, CS = 256, PP = 384, R = 448, SEQ = 488, SIZE = SPW * SEQ;
 };
 
-//
 // CHECK: the inputs' value checks (finite entries, signs of the variances) on
 // the staged pieces, 36 of about 800 VALU instructions a tile: 16384 x 512
-// tokens take 265 us with them and 247 without; the pass of bssm_checks.hip over
-// the same 772 MB took 117
-// us.
+// tokens take 265 us with them and 247 without; the pass of bssm_checks.hip
+// over the same 772 MB took 117 us.
 template <bool CHECK>
 __global__ __launch_bounds__(kWave) void rotation_forward_kernel(RotArgs a) {
   __shared__ float tile[RTile::SIZE];
@@ -869,8 +866,9 @@ __global__ __launch_bounds__(kWave) void rotation_forward_kernel(RotArgs a) {
 // ----------------------------------------------------------------- backward
 // A 16-token tile holds two checkpoint chunks of 8 tokens; tiles are visited
 // last to first, and in each the chunk 2J + 1 before the chunk 2J.  The last
-// tile's tokens at and past T are filled with neutral ones (neutral_tail).  A chunk is replayed from its checkpoint, keeping each
-// token's belief and step intermediates in registers, and then reversed.
+// tile's tokens at and past T are filled with neutral ones (neutral_tail).  A
+// chunk is replayed from its checkpoint, keeping each token's belief and step
+// intermediates in registers, and then reversed.
 // Gradients overwrite their inputs in the tile (gk over k, gq over q, gd over
 // d, gv over v, gp over p, gr over r) and leave with the next tile's loads.
 //

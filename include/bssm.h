@@ -505,17 +505,17 @@ int bssm_rotation_checkpoint(int key_dim);
  * waves of the latter do not fill the GPU and each wave's time is its own
  * instruction stream, which the row layout shortens; at large N the row
  * layout's extra lane work costs more than it saves (the backward first).
- * The backward also needs the preferred checkpoint chunk.  Direction 2 (3): the largest N, within direction 0's (1's), for
- * which the row forward (backward) runs as two (three) waves per 4
- * sequences, the covariance and mean halves (the covariance replay, the
- * covariance reverse and the mean) on separate SIMDs, bitwise the one-wave
- * results.  bf16 and float8 keys, values and queries (the _bf16 / _fp8 entry
+ * The backward also needs the preferred checkpoint chunk.  Direction 2 (3):
+ * the largest N, within direction 0's (1's), for which the row forward
+ * (backward) runs as two (three) waves per 4 sequences, the covariance and
+ * mean halves (the covariance replay, the covariance reverse and the mean) on
+ * separate SIMDs, bitwise the one-wave results.  bf16 and float8 keys, values and queries (the _bf16 / _fp8 entry
  * points) take the row kernels only within the two-wave (three-wave) limits
  * (widened on chip, bitwise the float32 split kernels on the widened values).
  * Direction 4: the largest N for which the D = 4 rotation forward
  * (bssm_forward_chunked_rotation) uses its row-per-sequence kernel (16-byte
- * aligned streams).  Defaults: 24576, 8192, 2048, 2048,
- * 32768, the measured crossovers.
+ * aligned streams).  Defaults: 24576, 8192, 2048, 2048, 32768, the measured
+ * crossovers.
  * Sets the limit when limit >= 0 and returns the previous one; limit < 0
  * only reads it; -1 for any other direction.  Results of the row and
  * rotated layouts agree within float32 rounding, not bitwise.  With the

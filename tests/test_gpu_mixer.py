@@ -189,13 +189,13 @@ def test_mixer_autograd_boundary(cuda_device, monkeypatch, leaves):
 
 
 def test_mixer_unsupported_shapes_take_the_op_chain(cuda_device):
-    """Heads not a multiple of 16 or T not a multiple of 4: the reference op chain + bayesian_layer."""
+    """Heads not a multiple of 4: the reference op chain + bayesian_layer.  Multiples of 4, and any T: the kernels."""
     from bayes_ssm import mixer
 
-    for b, t, h in ((1, 24, 8), (2, 30, 16)):
+    for b, t, h in ((1, 24, 8), (2, 30, 16), (1, 24, 6), (2, 7, 10)):
         views, _ = O.make_mixer_inputs(b, t, h, seed=5)
         dv = _device_views(views, cuda_device)
-        assert mixer._fused_eligible(tuple(dv), h) is None
+        assert (mixer._fused_eligible(tuple(dv), h) is None) == (h % 4 != 0)
         read, mT, cT = mixer.bayes_mixer_core(*dv, heads=h)
         e_read, e_mT, e_cT = O.mixer_core(*views, h)
         close(read, e_read, f"read b={b} t={t} h={h}")

@@ -476,6 +476,20 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
   if (a.gc0) st32(make_rsrc(a.gc0 + n0, valid * 4u), T > 0 ? gc0 : Gs, col == 0 ? 4u * seq : kOob, 0);
 }
 
+// Whether the backward above is faster than the generic one at a T that is not
+// whole chunks.  Its LDS holds 768 workgroups (6144 sequences) on the chip at a
+// time, the generic kernel's registers 2048 (16384 sequences): the time of a
+// round of the latter is 2.25 times that of the former's, 1.55 times where much
+// of the last block of 32 tokens is filled up or rows start off a 16-byte
+// boundary (fits at 17 T and 16 n).  T = 100: 34 against 55 us at n = 6144, 62
+// against 63 at 12288, 82 against 71 at 16384; T = 44: 21, 27; 37, 32; 52, 35.
+// Up to 5 tokens are filled up to 32 at any n (T = 4: 6.8 against 5.8 us at 4096).
+bool ragged_faster(int64_t n, int64_t t) {
+  if (t < 6) return false;
+  const bool full = (t >= 24 && t < 32) || (t >= 64 && t % 4 == 0);
+  return (n + 6143) / 6144 * 20 < (n + 16383) / 16384 * (full ? 45 : 31);
+}
+
 }  // namespace d1
 
 bool d1_forward_ok(const FwdArgs& a) {
@@ -484,7 +498,8 @@ bool d1_forward_ok(const FwdArgs& a) {
 }
 
 bool d1_backward_ok(const BwdArgs& a, bool fixed) {
-  const bool tail = a.t % d1::kChunk == 0 || !(fixed && (a.gmf != nullptr || a.gcf != nullptr));
+  const bool tail = a.t % d1::kChunk == 0 || (d1::ragged_faster(a.n, a.t) &&
+                                              !(fixed && (a.gmf != nullptr || a.gcf != nullptr)));
   return a.base16 && a.t > 0 && tail && a.chunk == d1::kChunk && a.t * 256 < (int64_t(1) << 31) &&
          (a.nb + 1) * 256 < (int64_t(1) << 31);
 }

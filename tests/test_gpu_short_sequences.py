@@ -1,0 +1,22 @@
+"""Either side of the rules that choose between kernels by the number of sequences and a last chunk or tile that is not
+whole: D = 1 backward (filled up, or generic), D = 4 backward (row or rotated layout), D = 8 forward of less than a tile.
+Against the float64 oracle at the parity tolerance; N leaves idle slots in the last wave."""
+from __future__ import annotations
+
+import pytest
+
+from tests.test_gpu_parity import ABIS, _case
+from tests.test_gpu_ragged import CHUNK, _check, _run
+
+pytestmark = pytest.mark.gpu
+
+CASES = [(1, n, t) for n, t in ((21, 5), (21, 6), (6143, 20), (6147, 20), (12290, 28), (12290, 30), (6147, 36))]
+
+
+@pytest.mark.parametrize("d,n,t", CASES)
+@pytest.mark.parametrize("final_grads", [False, True])
+def test_matches_oracle(cuda_device, d, n, t, final_grads):
+    print(f"short sequences D{d} n={n} t={t} final_grads={final_grads}", flush=True)
+    cpu, dev = _case(n, t, d, seed=600 + t, device=cuda_device)
+    outs, grads = _run(d, dev, ABIS[0], final_grads)
+    _check(cpu, outs, grads, ABIS[0], CHUNK[d], final_grads)

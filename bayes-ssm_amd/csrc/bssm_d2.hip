@@ -633,7 +633,8 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
   // Tokens len .. 7 of the last block made neutral: k = q = v = gy = 0, d = 1,
   // p = 0, r = 1.  Their step leaves the belief and their reverse the carried
   // adjoints as they are, so the chunk T ends in runs whole pieces.  (With
-  // FIXED only while the adjoints are zero; d2_backward_ok sees to it.)
+  // FIXED only while the adjoints are zero; d2_backward_ok sees to it.)  Whole
+  // pieces of 4 need none (4096 x 4: 4.9 us with it, 4.4 without).
   auto neutral_tail = [&](float* sl, float* kq, int len) {
     for (int t = len; t < BT; ++t) {
       const int v = 128 * t + 8 * (seq ^ t) + 2 * g;
@@ -747,7 +748,7 @@ __global__ __launch_bounds__(kWave) void backward_kernel(BwdArgs a) {
       if (m + 1 < npair) store_kq(kbuf(m + 1), m + 1);
     }
     if (blk > 0) issue(other, blk - 1);
-    if (i == 0) neutral_tail(cur, kbuf(m) + 256 * (blk & 1), static_cast<int>(T - blk * BT));
+    if (i == 0 && (T & 3u) != 0) neutral_tail(cur, kbuf(m) + 256 * (blk & 1), static_cast<int>(T - blk * BT));
     run_chunk(cur, kbuf(m) + 256 * (blk & 1), (T - blk * BT) <= 4u ? 1 : 2, blk == 0);
   }
   if (nblk > 0) {
@@ -773,7 +774,7 @@ bool d2_forward_ok(const FwdArgs& a) {
 }
 
 bool d2_backward_ok(const BwdArgs& a, bool fixed) {
-  const bool tail = a.t % d2::kChunk == 0 || !(fixed && (a.gmf != nullptr || a.gcf != nullptr));
+  const bool tail = a.t % 4 == 0 || !(fixed && (a.gmf != nullptr || a.gcf != nullptr));
   return a.base16 && a.t > 0 && tail && a.chunk == d2::kChunk && a.t * 512 < (int64_t(1) << 31) &&
          (a.nb + 1) * 1024 < (int64_t(1) << 31);
 }

@@ -20,3 +20,14 @@ def test_matches_oracle(cuda_device, d, n, t, final_grads):
     cpu, dev = _case(n, t, d, seed=600 + t, device=cuda_device)
     outs, grads = _run(d, dev, ABIS[0], final_grads)
     _check(cpu, outs, grads, ABIS[0], CHUNK[d], final_grads)
+
+
+@pytest.mark.parametrize("t", [4, 8, 12, 20])
+@pytest.mark.parametrize("final_grads", [False, True])
+@pytest.mark.parametrize("abi", ABIS, ids=[a[0] for a in ABIS])
+def test_d2_whole_pieces(cuda_device, abi, final_grads, t):
+    """T a multiple of 4 runs the D = 2 backward's pieces as they are, fixed dynamics with final-state gradients too."""
+    print(f"short sequences D2 {abi[0]} t={t} final_grads={final_grads}", flush=True)
+    cpu, dev = _case(21, t, 2, seed=650 + t, device=cuda_device)
+    outs, grads = _run(2, dev, abi, final_grads)
+    _check(cpu, outs, grads, abi, CHUNK[2], final_grads)

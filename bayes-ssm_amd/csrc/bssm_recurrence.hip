@@ -509,7 +509,15 @@ hipError_t launch_backward(int key_dim, bool fixed, bool dyn, const BwdArgs& a, 
   // start off a 16-byte boundary, and widened copies); 64 sequences, T = 437,
   // float32 forward: 50 against 562 us.
   const bool row_tail = a.t % 16 == 0 || !(fixed && (a.gmf != nullptr || a.gcf != nullptr));
-  if (key_dim == 4 && a.rot4 && a.n <= row_limit && row_tail && a.chunk == kRot4Chunk)
+  // The rotated kernels skip what is missing of a 16-token tile in pieces of 4,
+  // the row kernels run it: at these shares of the tiles (all of T = 4, 8, 12,
+  // 20, 24, 36; T = 4 and 8; T = 4) the former are faster.  T = 4: 7.1 against
+  // 11.9 us at n = 8192, 5.9 against 9.0 at 4096, 5.8 against 6.3 at 1024; T =
+  // 20: 17.3 against 20.6 at 8192, 14.7 against 14.8 at 4096; T = 28 (an eighth
+  // missing): 23.5 against 22.5 at 8192.
+  const int64_t tiles = (a.t + 15) / 16 * 16, quarters = a.n > 4096 ? 1 : a.n > 2048 ? 2 : 3;
+  const bool short_rows = a.t % 4 == 0 && a.t % 16 != 0 && 4 * (tiles - a.t) >= quarters * tiles;
+  if (key_dim == 4 && a.rot4 && a.n <= row_limit && row_tail && !short_rows && a.chunk == kRot4Chunk)
     return launch_backward_small(fixed, dyn, a, stream);
   if (key_dim == 4 && a.rot4) return launch_backward_r4(fixed, dyn, a, stream);
   if (key_dim == 1 && d1_backward_ok(a, fixed)) return launch_backward_d1(fixed, dyn, a, stream);

@@ -623,7 +623,7 @@ def bayesian_layer(
             if device.type == "cuda" and len(batch_shape) == 1 and t > 0:
                 from .fused_cuda import RotationProbe, fused_rotation_bayesian
 
-                probe = RotationProbe(device) if checks.pending else None
+                probe = RotationProbe(device) if checks.pending and d == RotationProbe.KEY_DIM else None
                 fused = fused_rotation_bayesian(keys, values, queries,
                                                 rotation_radii.expand(*batch_shape, t, d // 2),
                                                 rotation_angles.expand(*batch_shape, t, d // 2), process_variances,

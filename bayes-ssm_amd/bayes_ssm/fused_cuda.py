@@ -577,8 +577,10 @@ def fused_diagonal_bayesian(
 
 class RotationProbe:
     """The rotation forward's value checks: ``checked`` tells whether its kernel made them, ``faults`` (int32 [1] on the
-    device) holds their bits then (``bssm_forward_chunked_rotation_checked``)."""
+    device) holds their bits then (``bssm_forward_chunked_rotation_checked``).  Only for the key dimension whose kernel
+    makes them: clearing ``faults`` is a launch of its own (10 us of the other dimensions' calls)."""
 
+    KEY_DIM = 4
     # Argument name -> (bit of an entry that is not finite, bit of a variance of the wrong sign).
     BITS = {"keys": (1, 0), "values": (2, 0), "queries": (4, 0), "rotation_radii": (8, 0), "rotation_angles": (16, 0),
             "process_variances": (32, 128), "observation_variances": (64, 256)}

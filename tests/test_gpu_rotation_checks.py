@@ -74,7 +74,11 @@ def test_first_fault_in_order_and_other_tensors(cuda_device):
 
 
 @pytest.mark.parametrize("d", [2, 8])
-def test_other_key_dimensions_keep_the_pass(cuda_device, d):
+def test_other_key_dimensions_keep_the_pass(cuda_device, monkeypatch, d):
+    """... and have no probe: its kernel makes no checks for them."""
+    from bayes_ssm import fused_cuda
+
+    monkeypatch.setattr(fused_cuda.RotationProbe, "__init__", lambda *a: pytest.fail("a probe was made"))
     xs = _inputs(3, 9, d, cuda_device)
     _run(xs)
     xs[6][1, 4] = 0.0

@@ -505,7 +505,9 @@ int bssm_rotation_checkpoint(int key_dim);
  * waves of the latter do not fill the GPU and each wave's time is its own
  * instruction stream, which the row layout shortens; at large N the row
  * layout's extra lane work costs more than it saves (the backward first).
- * The backward also needs the preferred checkpoint chunk.  Direction 2 (3):
+ * The backward also needs the preferred checkpoint chunk, and leaves short
+ * rows off whole 16-token tiles to the rotated kernels where these are faster
+ * (T = 4 at every N, 8 above 2048, 12, 20, 24 and 36 above 4096).  Direction 2 (3):
  * the largest N, within direction 0's (1's), for which the row forward
  * (backward) runs as two (three) waves per 4 sequences, the covariance and
  * mean halves (the covariance replay, the covariance reverse and the mean) on
@@ -521,8 +523,8 @@ int bssm_rotation_checkpoint(int key_dim);
  * rotated layouts agree within float32 rounding, not bitwise.  With the
  * default limits the forward results of a sequence are the same bits for
  * every N up to 24576 (the row layout's one- and two-wave forwards are
- * bitwise one another); its gradients change layout above 8192 sequences
- * and then differ in the last bits: at config 3 (T = 512), the same
+ * bitwise one another); its gradients change layout above 8192 sequences (at
+ * the T named above, at theirs) and then differ in the last bits: at config 3 (T = 512), the same
  * sequences inside N = 16384 and inside N = 2048 or 32 differ by at most
  * 1.2e-4 absolute (dL/dr) and 2e-5 for the other gradients, inside the
  * 1e-5 relative + 1e-4 absolute tolerance both meet against the float64

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 CASES = [(1, n, t) for n, t in ((21, 5), (21, 6), (6143, 20), (6147, 20), (12290, 28), (12290, 30), (6147, 36))]
 CASES += [(4, n, t) for n, t in ((21, 4), (2047, 8), (2053, 8), (4095, 20), (4099, 20), (4099, 36), (4099, 28))]
-CASES += [(8, n, t) for n, t in ((4095, 12), (4099, 12), (4099, 13), (4099, 8))]
+CASES += [(8, n, t) for n, t in ((4095, 12), (4099, 12), (4099, 13), (8195, 8))]
 
 
 @pytest.mark.parametrize("d,n,t", CASES)

@@ -80,6 +80,12 @@ def _chunk_arg(b: int, heads: int, t: int, backward: bool = False) -> int:
     return interval | _hip.ANY_SHAPE | (_hip.ROW_KERNELS if rows else 0)
 
 
+def _readout_unused(grad_out: Optional[Tensor], heads: int, t: int) -> bool:
+    """Off whole tiles the gate and the norm weight have no gradient (not a zero one) when only the final state is
+    differentiated, as in the op chain."""
+    return grad_out is None and not _whole_tiles(heads, t)
+
+
 def _partials(chunk: int, b: int, heads: int, device: torch.device) -> Tensor:
     """Partial sums of the norm-weight gradient: a row, or with the small-batch kernels four, for each 16 heads of a
     batch row."""
@@ -382,6 +388,7 @@ class _MixerReadoutFunction(torch.autograd.Function):
         heads, lds = ctx.heads, ctx.lds
         need = ctx.needs_input_grad
         dev = q_proj.device
+        unused = _readout_unused(grad_out, heads, t)
         if grad_out is None:
             grad_out = torch.zeros(b, t, heads * VALUE_DIM, device=dev, dtype=torch.bfloat16)
         else:
@@ -408,10 +415,10 @@ class _MixerReadoutFunction(torch.autograd.Function):
                       P(cov0), P(bmean), P(bcov), P(read_bf16), P(grad_out), P(gm), P(gc), P(gq), P(gk), P(gv),
                       P(gdl), P(gnz), P(ggate), P(partials), P(gm0), P(gc0), b, t, heads, chunk,
                       ctx.denominator_floor, 0, _hip.stream_of(dev))
-        gw = partials.sum(0).to(ctx.weight_dtype) if need[6] else None
+        gw = partials.sum(0).to(ctx.weight_dtype) if need[6] and not unused else None
         return (gq if need[0] else None, gk if need[1] else None, gv if need[2] else None,
-                gdl if need[3] else None, gnz if need[4] else None, ggate if need[5] else None, gw, gm0, gc0,
-                None, None, None, None)
+                gdl if need[3] else None, gnz if need[4] else None, ggate if need[5] and not unused else None, gw,
+                gm0, gc0, None, None, None, None)
 
 
 def bayes_mixer_readout(
@@ -523,6 +530,7 @@ class _MixerBlockFunction(torch.autograd.Function):
         core, aux_w = 16 * heads, 6 * heads
         need = ctx.needs_input_grad
         dev = projected.device
+        unused = _readout_unused(grad_out, heads, t)
         if grad_out is None:
             grad_out = torch.zeros(b, t, heads * VALUE_DIM, device=dev, dtype=torch.bfloat16)
         else:
@@ -553,7 +561,9 @@ class _MixerBlockFunction(torch.autograd.Function):
                       chunk, ctx.denominator_floor, _hip.stream_of(dev))
         if g_conv is not None and g_conv.dtype != ctx.conv_dtype:
             g_conv = g_conv.to(ctx.conv_dtype)
-        if g_norm is not None and g_norm.dtype != ctx.norm_dtype:
+        if unused:
+            g_norm = None
+        elif g_norm is not None and g_norm.dtype != ctx.norm_dtype:
             g_norm = g_norm.to(ctx.norm_dtype)
         if g_bias is not None and g_bias.dtype != ctx.bias_dtype:
             g_bias = g_bias.to(ctx.bias_dtype)

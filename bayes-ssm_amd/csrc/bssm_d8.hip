@@ -714,10 +714,9 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void
 // bases.  A last tile that is not a multiple of 8 tokens runs token by token:
 // where there is no other tile, the generic kernel is the faster one with many
 // sequences (T = 12: 10.0 against 9.4 us at n = 4096, 12.4 against 14.0 at
-// 8192, 18.7 against 22.2 at 16384; T = 8: 9.8 against 10.1 at 8192, 15.1
-// against 17.2 at 16384).
+// 8192, 18.7 against 22.2 at 16384).
 bool d8_forward_ok(const FwdArgs& a) {
-  if (a.t < 16 && a.n > (a.t % 8 != 0 ? 4096 : 8192)) return false;
+  if (a.t < 16 && a.t % 8 != 0 && a.n > 4096) return false;
   return a.base16 && a.in_fmt == kInF32 && a.t > 0 && a.t * 256 < (int64_t(1) << 31) &&
          (a.nb + 1) * 2048 < (int64_t(1) << 31);
 }

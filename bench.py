@@ -72,11 +72,17 @@ def dispatched_kernels(d: int, m: int, n: int, t: int, interval: int) -> tuple[s
         fwd = "bssm::sn::forward_kernel<false, 0> (row layout, 16 lanes per sequence)"
     else:
         fwd = "bssm::r4::forward_kernel<false, 0> (rotated layout, 4 lanes per sequence)"
-    row_bwd = interval == _hip.preferred_checkpoint(4)
-    if row_bwd and n <= lim[3]:
-        bwd = f"bssm::sn::backward_split_kernel<false, true, 0, {groups}> (row layout, three waves per 4 sequences)"
+    # Short rows that leave much of their last 16-token tile empty run on the rotated layout.
+    tiles, quarters = -(-t // 16) * 16, 1 if n > 4096 else 2 if n > 2048 else 3
+    short_rows = t % 4 == 0 and t % 16 != 0 and 4 * (tiles - t) >= quarters * tiles
+    row_bwd = interval == _hip.preferred_checkpoint(4) and not short_rows
+    if row_bwd and n <= min(lim[1], lim[3]):
+        ragged = "true" if t % 8 or groups == 2 else "false"
+        bwd = (f"bssm::sn::backward_split_kernel<false, true, 0, {groups}, {ragged}> (row layout, three waves per "
+               "4 sequences)")
     elif row_bwd and n <= lim[1]:
-        bwd = "bssm::sn::backward_kernel<false, true> (row layout, 16 lanes per sequence)"
+        ragged = "true" if t % 16 else "false"
+        bwd = f"bssm::sn::backward_kernel<false, true, {ragged}> (row layout, 16 lanes per sequence)"
     else:
         ragged = "true" if t % 4 else "false"  # T ends inside a 4-token piece
         bwd = (f"bssm::r4::backward_tile_kernel<false, true, 0, {interval}, {ragged}> (rotated layout, "
